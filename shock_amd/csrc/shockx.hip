@@ -442,16 +442,127 @@ enum { V_F0, V_F1, V_F2, V_F3, V_F4, V_U0, V_U1, V_U2, V_U3, V_U4, V_LAM, V_U, V
 // fields of the window).  Diagonal metric: no normal components; the sign of the
 // metric entry rides on V_LAM (the spectral radius is positive) and J moves to V_NX, which keeps
 // the 8 x 32 tile's window under 40 KB (four blocks per CU).
-// DIFF (FP64 WENO5): the F and U arrays hold node-to-node differences once the node pass is
-// done, and one more array keeps rho for the interface state (below).
-template <int S, int AX, bool MIX>
-constexpr bool weno_diff() { return S == 5 && !MIX; }
 template <int S, int TA, int TDI, int AX, bool MIX>
 constexpr int weno_lds()
 {
     constexpr int NW = (TDI - 1 + (S + 1)) * TA;
     constexpr int NVK = (AX < 0) ? NV : NV - 3;
-    return NVK * NW + ((MIX || weno_diff<S, AX, MIX>()) ? NW : 0);
+    return NVK * NW + (MIX ? NW : 0);
+}
+
+// Value of the next lane (lane 63: its own).  All 64 lanes must be active.
+__device__ __forceinline__ double next_lane(const double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)b, hi = (int)(b >> 32);
+    const int nlo = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);   // wave_shl:1
+    const int nhi = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)nhi << 32) | (unsigned)nlo);
+}
+
+// FP64 WENO5 flux of the interface between nodes ob+2 and ob+3 of a window row, less F[ob+2]: the
+// central part in differences, Theta = F[2] + (D[1] + 6 D[2] - D[3]) / 12 (D[s] = F[s+1] - F[s]),
+// whose F[2] terms telescope in the divergence (node 3's divergence = D[2], returned in dcur, plus
+// the difference of the two interface values), and R Phi.
+// The six nodes pass through registers once: a pair of neighbours gives its differences of F and U,
+// the split differences dF +- lam J dU, and their five characteristic projections (char_project), so
+// the window is read 80 to 120 times per interface instead of 190 (once per non-zero entry of the
+// left eigenvectors), which had the LDS as busy as the FP64 pipe, and FP64 instructions fall from 926
+// to about 750 (256^3, diagonal metric: xi sweep 1.04 -> 0.83 ms, k_eta 1.42 -> 1.26, k_zeta 1.70 -> 1.55).
+// Bound by the FP64 pipe and its latency at four waves per SIMD, so registers decide: the projections
+// are pinned pair by pair (else the compiler keeps several pairs in flight, 148-166 VGPRs), which
+// leaves 126 VGPRs along zeta.  Along xi and eta one pass over all fields still spilled two registers
+// (k_eta 1.31 ms), so they take the shear fields, which need three of the five components, in a
+// second pass over the row.
+template <int AX, int NW, int VJ>
+__device__ __forceinline__ void weno5_flux(const double *sm, const int ob, const Consts &k, double out[5], double dcur[5])
+{
+    const int oc = ob + 2;
+    auto mean = [&](const int v) { return 0.5 * (sm[v * NW + oc] + sm[v * NW + oc + 1]); };
+    const double cs = mean(V_C);
+    const double rho = mean(V_U0);
+    CharBasis c;
+    c.u[0] = mean(V_U); c.u[1] = mean(V_V); c.u[2] = mean(V_W);
+    if constexpr (AX < 0) {
+        c.n[0] = mean(V_NX); c.n[1] = mean(V_NY); c.n[2] = mean(V_NZ);
+    } else {
+        c.s = 0.5 * (copysign(1.0, sm[V_LAM * NW + oc]) + copysign(1.0, sm[V_LAM * NW + oc + 1]));
+    }
+    char_basis<AX>(c, rho, cs, k.gamma);
+    double lam = 0.0;
+#pragma unroll
+    for (int s = 0; s < 6; s++) lam = fmax(lam, fabs(sm[V_LAM * NW + ob + s]));
+    const double lj = lam * mean(VJ);
+
+    // epsilon of the indicators as w5_pair forms them: a third of the reference's, and scaled with
+    // the square of what the projections leave out (char_project)
+    const double e3 = k.eps * (1. / 3.);
+    const double es = (AX < 0) ? e3 : e3 * (rho * rho), ea = 2.0 * e3;
+    double psi[5];
+    // one pass over the row's five pairs for the fields of MASK (bit f: field f)
+    auto pass = [&](auto mask_c) {
+        constexpr int MASK = decltype(mask_c)::value;
+        double fp[5][4], fm[5][4];               // split characteristic differences: f+ of pairs 0..3, f- of 4..1
+        double pf[5], pu[5];
+        auto need = [](const int q) { return AX < 0 || (MASK & 25) || q == 0 || q != 1 + AX && q != 4; };
+#pragma unroll
+        for (int q = 0; q < 5; q++)
+            if (need(q)) { pf[q] = sm[(V_F0 + q) * NW + ob]; pu[q] = sm[(V_U0 + q) * NW + ob]; }
+#pragma unroll
+        for (int s = 0; s < 5; s++) {
+            double dF[5] = {}, dU[5] = {};
+#pragma unroll
+            for (int q = 0; q < 5; q++) {
+                if (!need(q)) continue;
+                const double f = sm[(V_F0 + q) * NW + ob + s + 1], u = sm[(V_U0 + q) * NW + ob + s + 1];
+                dF[q] = f - pf[q]; dU[q] = u - pu[q];
+                pf[q] = f; pu[q] = u;
+            }
+            double g[5], o[5];
+            if (s < 4) {
+#pragma unroll
+                for (int q = 0; q < 5; q++) g[q] = fma(lj, dU[q], dF[q]);
+                char_project<AX>(c, g, o);
+#pragma unroll
+                for (int f = 0; f < 5; f++) if (MASK >> f & 1) fp[f][s] = o[f];
+            }
+            if (s > 0) {
+#pragma unroll
+                for (int q = 0; q < 5; q++) g[q] = fma(-lj, dU[q], dF[q]);
+                char_project<AX>(c, g, o);
+#pragma unroll
+                for (int f = 0; f < 5; f++) if (MASK >> f & 1) fm[f][4 - s] = o[f];
+            }
+            // one pair's loads and projections at a time (registers)
+#pragma unroll
+            for (int f = 0; f < 5; f++) {
+                if (!(MASK >> f & 1)) continue;
+                if (s < 4) asm volatile("" : "+v"(fp[f][s]));
+                if (s > 0) asm volatile("" : "+v"(fm[f][4 - s]));
+            }
+            asm volatile("" ::: "memory");
+        }
+        if constexpr (MASK & 1) psi[0] = w5_pair(e3, fp[0], fm[0]);
+        if constexpr (MASK & 2) psi[1] = w5_pair(es, fp[1], fm[1]);
+        if constexpr (MASK & 4) psi[2] = w5_pair(es, fp[2], fm[2]);
+        if constexpr (MASK & 8) psi[3] = w5_pair(ea, fp[3], fm[3]);
+        if constexpr (MASK & 16) psi[4] = w5_pair(ea, fp[4], fm[4]);
+    };
+    if constexpr (AX == 0 || AX == 1) {
+        pass(std::integral_constant<int, 25>{});
+        asm volatile("" : "+v"(psi[0]), "+v"(psi[3]), "+v"(psi[4]) : : "memory");
+        pass(std::integral_constant<int, 6>{});
+    } else {
+        pass(std::integral_constant<int, 31>{});
+    }
+    char_assemble<AX>(c, rho, cs * cs * k.igm1, psi, out);
+#pragma unroll
+    for (int m = 0; m < 5; m++) {
+        const double *F = &sm[(V_F0 + m) * NW + ob];
+        const double d2 = F[3] - F[2];
+        out[m] += 1. / 12. * (((F[2] - F[1]) - (F[4] - F[3])) + 6. * d2);
+        dcur[m] = d2;
+    }
 }
 
 // KEEP: leave Q alone and return this sweep's contribution of the thread's node in keep[5] (a
@@ -467,15 +578,12 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     constexpr int NT = TA * TDI;
     constexpr int NVK = (AX < 0) ? NV : NV - 3;
     constexpr int VJ = (AX < 0) ? V_J : V_NX;
-    // DIFF (FP64 WENO5, any metric): after the node pass, position o of the F and U arrays holds
-    // node o+1 minus node o.
-    // The projection then runs on the five differences the indicators use (instead of six node
-    // values, whose differences were taken after projecting), and the central part Theta is
-    // written in differences: Theta = F[oc] + (D[oc-1] + 6 D[oc] - D[oc+1]) / 12, whose F[oc]
-    // terms telescope in the divergence (node oc+1's divergence = D[oc] + the difference of the
-    // two interface values without F).  rho, for the interface state, keeps its own array VRHO.
-    constexpr bool DIFF = weno_diff<S, AX, MIX>();
-    constexpr int VRHO = NVK;
+    // FP64 WENO5 streams the stencil through registers pair by pair (weno5_flux); the others project
+    // one characteristic field at a time.
+    constexpr bool PAIRS = (S == 5 && !MIX);
+    // the plus-side interface value of a node's divergence comes from the next lane where a tile row
+    // never straddles two wavefronts
+    constexpr bool SHFL = (64 % TDI == 0);
     double *const sm = lds;                       // NVK * NW (+ NW)
     // mixed form: the FP32 differences of F (arrays 0..4) and U (5..9).  Once formed, the node
     // values of rho u, rho v, rho w and rho e are not read again, so arrays 0..7 take their place
@@ -553,7 +661,6 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
             sm[V_LAM * NW + o] = (md > 0.0) ? lam : -lam;
         }
         sm[V_U0 * NW + o] = rho;
-        if constexpr (DIFF) sm[VRHO * NW + o] = rho;
         sm[V_U1 * NW + o] = rho * u;
         sm[V_U2 * NW + o] = rho * v;
         sm[V_U3 * NW + o] = rho * w;
@@ -595,43 +702,21 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
         }
         __syncthreads();
     }
-    if constexpr (DIFF) {
-        // node-to-node differences of F and U, all read before any is written over the node values
-        constexpr int PER = (NW + NT - 1) / NT;
-        double dv[PER][10];
-#pragma unroll
-        for (int r = 0; r < PER; r++) {
-            const int idx = t + r * NT;
-            if (idx < NW && idx % WD != WD - 1) {
-#pragma unroll
-                for (int q = 0; q < 10; q++) dv[r][q] = sm[(V_F0 + q) * NW + idx + 1] - sm[(V_F0 + q) * NW + idx];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < PER; r++) {
-            const int idx = t + r * NT;
-            if (idx < NW && idx % WD != WD - 1) {
-#pragma unroll
-                for (int q = 0; q < 10; q++) sm[(V_F0 + q) * NW + idx] = dv[r][q];
-            }
-        }
-        __syncthreads();
-    }
 
     // phase 2: interface flux between nodes (d0-1+di) and (d0+di)
     const int ta = t / TDI, di = t - ta * TDI;
     const int ob = ta * WD + di;                 // window position of the stencil's first node
     const int oc = ob + R;                       // left node of the interface
     double out[5];
-    double dcur[5];                              // DIFF: D[oc] of every field, for the divergence
-    {
+    double dcur[5];                              // PAIRS: F[oc+1] - F[oc], for the divergence
+    if constexpr (PAIRS) {
+        weno5_flux<AX, NW, VJ>(sm, ob, k, out, dcur);
+    } else {
         const double Jh = (sm[VJ * NW + oc] + sm[VJ * NW + oc + 1]) / 2.0;
         const double u = 0.5 * (sm[V_U * NW + oc] + sm[V_U * NW + oc + 1]);
         const double v = 0.5 * (sm[V_V * NW + oc] + sm[V_V * NW + oc + 1]);
         const double w = 0.5 * (sm[V_W * NW + oc] + sm[V_W * NW + oc + 1]);
-        constexpr int VR = DIFF ? VRHO : V_U0;
-        const double rho = 0.5 * (sm[VR * NW + oc] + sm[VR * NW + oc + 1]);
+        const double rho = 0.5 * (sm[V_U0 * NW + oc] + sm[V_U0 * NW + oc + 1]);
         const double cs = 0.5 * (sm[V_C * NW + oc] + sm[V_C * NW + oc + 1]);
         double nx, ny, nz;
         if constexpr (AX < 0) {
@@ -701,29 +786,6 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
             double Lc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
             if constexpr (AX < 0) left_row<c>(e, Lc);
             else left_row_ax<c, (AX < 0 ? 0 : AX)>(e, nsig, Lc);
-            if constexpr (DIFF) {
-                // projected differences da_s = L_c . (F_{s+1} - F_s), db_s likewise for U, on the
-                // five node pairs of the stencil; f+ differences on pairs 0..3, f- on 4..1
-                double da[5], db[5];
-#pragma unroll
-                for (int s = 0; s < 5; s++) {
-                    double aa = 0.0, bb = 0.0;
-#pragma unroll
-                    for (int q = 0; q < 5; q++) {
-                        if (AX < 0 || lnz(c, AX, q)) {
-                            aa += Lc[q] * sm[(V_F0 + q) * NW + ob + s];
-                            bb += Lc[q] * sm[(V_U0 + q) * NW + ob + s];
-                        }
-                    }
-                    da[s] = aa;
-                    db[s] = bb;
-                }
-                phis[c] = 0.5 * (-phi_w5_fast(k.eps, da[0] + lj * db[0], da[1] + lj * db[1], da[2] + lj * db[2],
-                                              da[3] + lj * db[3])
-                                 + phi_w5_fast(k.eps, da[4] - lj * db[4], da[3] - lj * db[3], da[2] - lj * db[2],
-                                               da[1] - lj * db[1]));
-                return;
-            }
             double av[2 * G], bv[2 * G];
 #pragma unroll
             for (int s = 0; s < 2 * G; s++) {
@@ -748,7 +810,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
                 fp[s] = av[s] + lj * bv[s];
                 fm[s] = av[2 * G - 1 - s] - lj * bv[2 * G - 1 - s];
             }
-            // WENO9 (WENO5 takes the difference form above): the indicators need the node values
+            // WENO9 (FP64 WENO5 goes through weno5_flux): the indicators need the node values
             if constexpr (S == 9) {
                 double dp_[8], dm_[8];
 #pragma unroll
@@ -767,11 +829,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
             constexpr int m = decltype(mm)::value;
             const double *F = &sm[(V_F0 + m) * NW];
             double th;
-            if constexpr (DIFF) {
-                // Theta without F[oc] (added back in the divergence as D[oc], the F difference)
-                th = 1. / 12. * ((F[oc - 1] - F[oc + 1]) + 6. * F[oc]);
-                dcur[m] = F[oc];
-            } else if constexpr (S == 5) {
+            if constexpr (S == 5) {
                 th = 1. / 12. * (-1. * (F[oc - 1] + F[oc + 2]) + 7. * (F[oc] + F[oc + 1]));
             } else {
                 th = 1. / 840. * (533. * (F[oc + 1] + F[oc]) - 139. * (F[oc + 2] + F[oc - 1])
@@ -804,10 +862,18 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
         assemble(std::integral_constant<int, 3>{});
         assemble(std::integral_constant<int, 4>{});
     }
-    __syncthreads();
+    double nxt[5];
+    if constexpr (SHFL) {
 #pragma unroll
-    for (int m = 0; m < 5; m++) sm[m * NT + t] = out[m];
-    __syncthreads();
+        for (int m = 0; m < 5; m++) nxt[m] = next_lane(out[m]);
+    } else {
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 5; m++) sm[m * NT + t] = out[m];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 5; m++) nxt[m] = (di < TDI - 1) ? sm[m * NT + t + 1] : 0.0;
+    }
 
     // phase 3: divergence into Q for the tile's TDI-1 nodes
     if (di < TDI - 1) {
@@ -817,20 +883,19 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
             const long n = bbase + (long)pa * a.sA + (long)(dn + a.oD) * a.sD;
 #pragma unroll
             for (int m = 0; m < 5; m++) {
-                double dv = sm[m * NT + t + 1] - sm[m * NT + t];
-                if constexpr (DIFF) dv = dcur[m] + dv;
+                double dv = nxt[m] - out[m];
+                if constexpr (PAIRS) dv = dcur[m] + dv;
                 if constexpr (KEEP) keep[m] = -dv;
                 else a.q.f[m][n] = (a.first ? 0.0 : a.q.f[m][n]) - dv;
             }
         }
     }
 }
-// Waves per SIMD asked of the compiler: the diagonal W5 xi and eta sweeps otherwise take 134
-// VGPRs (three waves per SIMD); at 128 (126 for xi, no spills) they run four and are measured 7-9 %
-// faster.  The other variants are left to the compiler (the zeta sweep measured slower under the
-// same bound).
+// Waves per SIMD asked of the compiler: the diagonal FP64 W5 sweeps run four (122-128 VGPRs, at most two
+// spilled), which the LDS of an 8 x 32 or 4 x 64 tile allows too; at three waves (132-134 VGPRs) the xi
+// sweep took 0.87 ms at 256^3 against 0.83.  The other variants are left to the compiler.
 template <int S, int AX, bool MIX>
-constexpr int weno_min_waves() { return (S == 5 && (AX == 0 || AX == 1) && !MIX) ? 4 : 1; }
+constexpr int weno_min_waves() { return (S == 5 && AX >= 0 && !MIX) ? 4 : 1; }
 
 template <int S, int TA, int TDI, int AX, bool MIX>
 __global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, AX, MIX>())) void k_weno(WenoArgs a)
@@ -1323,7 +1388,7 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
     double nxt[4];
     if constexpr (SHFL) {
 #pragma unroll
-        for (int m = 0; m < 4; m++) nxt[m] = __shfl_down(out[4 + m], 1);
+        for (int m = 0; m < 4; m++) nxt[m] = next_lane(out[4 + m]);
     } else {
 #pragma unroll
         for (int m = 0; m < 4; m++) fo[m * NT + t] = out[4 + m];
@@ -1447,8 +1512,8 @@ __device__ __forceinline__ void zeta_body(const ZetaArgs &z, const int bx, const
     // kernel, which stores Q instead of updating the stage, made it slower)
     visc_body<S, 2, 4, 64, true, true, true>(z.v, bx, by, bz, lds, inv);
 }
-// FP64 W5: held to 128 VGPRs (four waves per SIMD, as the LDS allows); measured 11 % faster than
-// the compiler's own 136
+// FP64 W5: held to 128 VGPRs (four waves per SIMD, as the LDS allows): 1.55 ms at 256^3 against
+// 1.67 at three waves
 template <int S, bool MIX>
 __global__ __launch_bounds__(256, ((S == 5 && !MIX) ? 4 : 1)) void k_zeta(ZetaArgs z)
 {
@@ -1478,10 +1543,8 @@ __device__ __forceinline__ void eta_body(const EtaArgs &z, const int bx, const i
     __syncthreads();
     visc_body<5, 1, 8, 32, true, true>(z.v, bx, by, bz, lds, inv);
 }
-// FP64: asked for three waves per SIMD.  With the WENO phase in difference form it takes 124
-// VGPRs, so four fit (1.44 ms at 256^3; 1.53-1.57 ms at 140 VGPRs and three waves); forcing four
-// when it needed 140 spilled and measured 1.82 ms.
-constexpr int ETA_WAVES = 3;
+// FP64: four waves per SIMD (126 VGPRs; weno5_flux)
+constexpr int ETA_WAVES = 4;
 template <bool MIX>
 __global__ __launch_bounds__(256, (MIX ? 1 : ETA_WAVES)) void k_eta(EtaArgs z)
 {
@@ -2560,6 +2623,7 @@ extern "C" int shx_create(const shx_desc *desc, shx_case **out)
     k.suth = 100.4 / d.T0;
     k.eps = d.eps_override > 0.0 ? d.eps_override : 10. * pow(DBL_MIN, 0.5);
     k.gm1_ups = (d.gamma - 1.0) / k.upsilon;
+    k.igm1 = 1.0 / (d.gamma - 1.0);
     k.mms = d.manufactured ? 1 : 0;
     if (S == 9) {
         const double in9[10] = {1. / 1260., -23. / 2520., 127. / 2520., -473. / 2520., 1627. / 2520.,

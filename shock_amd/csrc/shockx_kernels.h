@@ -12,6 +12,7 @@ namespace shx {
 struct Consts {
     double gamma, upsilon, psi, gam_heat, suth, eps;
     double gm1_ups;   // (gamma - 1) / Upsilon
+    double igm1;      // 1 / (gamma - 1)
     double mach;      // reference Mach number (post-processing)
     double zd_mid[10], zd_int[10], zd_der[11];
     int mms;
@@ -300,24 +301,142 @@ __device__ __forceinline__ void scaled_sq(double s[N], const int lo)
     }
 }
 
-// Jiang-Shu WENO5 deviation from the central flux (Phi_Function_W5, src/WENO.c:118-204) with one
-// reciprocal for the weights: for q_k = s_k^2, w0 = q1 q2 / D and w2 = 3 q0 q1 / D with
-// D = q1 q2 + 6 q0 q2 + 3 q0 q1.
-__device__ __forceinline__ double phi_w5_fast(const double eps, const double d0, const double d1,
-                                              const double d2, const double d3)
+// ---- characteristic projection without the eigenvector entries ------------------------------------
+// The left and right eigenvectors above applied to a vector g = (g0, gm, g4) of differences through
+// S = gm - g0 u (momentum less the mean velocity's share) and t = g4 - u.S - |u|^2/2 g0 (the pressure
+// difference over gamma - 1):
+//   L_0..2 . g = n_c E + (n x S)-component / rho,  E = g0 - (gamma-1)/c^2 t
+//   L_3,4 . g  = ((gamma-1)/c t +- n.S) / sqrt(2)
+// which is 23 operations for the five projections (11 with a diagonal metric) instead of 25 (19), and
+// needs no entry of L in registers.  char_project leaves out constant factors of a field, which the
+// assembly puts back: the deviation Phi is homogeneous of degree one in its inputs, so only epsilon
+// has to follow (times the factor's inverse squared).  Left out: 1/sqrt(2) of the acoustic fields;
+// with a diagonal metric also the normal's sign and the shear fields' 1/rho, against which the right
+// eigenvectors' rho cancels.
+struct CharBasis {
+    double u[3];          // mean velocity
+    double n[3], rn[3];   // mean unit normal, over rho (general metric)
+    double s;             // diagonal metric: the normal's component along the axis (+-1; 0 between
+                          // nodes of opposite sign)
+    double q2h, ic, gic, gic2;   // |u|^2 / 2, 1/c, (gamma-1)/c, (gamma-1)/c^2
+};
+template <int AX>
+__device__ __forceinline__ void char_basis(CharBasis &c, const double rho, const double cs, const double gamma)
 {
-    const double t0 = d0 - d1, t1 = d0 - 3. * d1;
-    const double t2 = d1 - d2, t3 = d1 + d2;
-    const double t4 = d2 - d3, t5 = 3. * d2 - d3;
-    double q[3] = {13. * t0 * t0 + 3. * t1 * t1 + eps, 13. * t2 * t2 + 3. * t3 * t3 + eps,
-                   13. * t4 * t4 + 3. * t5 * t5 + eps};
-    scaled_sq<3>(q, -250);
-    const double P0 = q[1] * q[2], P2 = 3. * (q[0] * q[1]);
-    const double r = frcp(P0 + 6. * (q[0] * q[2]) + P2);
-    const double w0 = P0 * r, w2 = P2 * r;
-    const double q1 = d0 - 2. * d1 + d2;
-    const double qq2 = d1 - 2. * d2 + d3;
-    return 1. / 3. * w0 * q1 + 1. / 6. * (w2 - 0.5) * qq2;
+    c.q2h = 0.5 * (c.u[0] * c.u[0] + c.u[1] * c.u[1] + c.u[2] * c.u[2]);
+    c.ic = frcp(cs);
+    c.gic = (gamma - 1.0) * c.ic;
+    c.gic2 = c.gic * c.ic;
+    if constexpr (AX < 0) {
+        const double ir = frcp(rho);
+#pragma unroll
+        for (int q = 0; q < 3; q++) c.rn[q] = c.n[q] * ir;
+    }
+}
+// o: fields 0, 1, 2 (diagonal metric: entropy, then the shear fields of the axes after AX), acoustic +, -
+template <int AX>
+__device__ __forceinline__ void char_project(const CharBasis &c, const double g[5], double o[5])
+{
+    double S[3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) S[q] = fma(-c.u[q], g[0], g[1 + q]);
+    const double t = fma(-c.u[2], S[2], fma(-c.u[1], S[1], fma(-c.u[0], S[0], fma(-c.q2h, g[0], g[4]))));
+    const double E = fma(-c.gic2, t, g[0]);
+    const double Xc = c.gic * t;
+    if constexpr (AX < 0) {
+        o[0] = fma(c.n[0], E, fma(c.rn[2], S[1], -(c.rn[1] * S[2])));
+        o[1] = fma(c.n[1], E, fma(c.rn[0], S[2], -(c.rn[2] * S[0])));
+        o[2] = fma(c.n[2], E, fma(c.rn[1], S[0], -(c.rn[0] * S[1])));
+        const double sn = fma(c.n[2], S[2], fma(c.n[1], S[1], c.n[0] * S[0]));
+        o[3] = Xc + sn;
+        o[4] = Xc - sn;
+    } else {
+        o[0] = E;
+        o[1] = S[(AX + 1) % 3];
+        o[2] = S[(AX + 2) % 3];
+        o[3] = fma(c.s, S[AX], Xc);
+        o[4] = fma(-c.s, S[AX], Xc);
+    }
+}
+// R . Phi from the fields' deviations psi (six times Phi, as w5_pair returns them); c2g = c^2/(gamma-1)
+template <int AX>
+__device__ __forceinline__ void char_assemble(const CharBasis &c, const double rho, const double c2g,
+                                              const double psi[5], double out[5])
+{
+    const double P = (c.ic * (1. / 12.)) * (psi[3] + psi[4]);
+    if constexpr (AX < 0) {
+        const double D = (1. / 12.) * (psi[3] - psi[4]);
+        const double r6 = rho * (1. / 6.);
+        const double M0 = fma(1. / 6., fma(c.n[2], psi[2], fma(c.n[1], psi[1], c.n[0] * psi[0])), P);
+        double W[3];
+        W[0] = r6 * fma(c.n[1], psi[2], -(c.n[2] * psi[1]));
+        W[1] = r6 * fma(c.n[2], psi[0], -(c.n[0] * psi[2]));
+        W[2] = r6 * fma(c.n[0], psi[1], -(c.n[1] * psi[0]));
+#pragma unroll
+        for (int q = 0; q < 3; q++) W[q] = fma(c.n[q], D, W[q]);
+        out[0] = M0;
+#pragma unroll
+        for (int q = 0; q < 3; q++) out[1 + q] = fma(c.u[q], M0, W[q]);
+        out[4] = fma(c.q2h, M0, fma(c2g, P, fma(c.u[2], W[2], fma(c.u[1], W[1], c.u[0] * W[0]))));
+    } else {
+        constexpr int T1 = (AX + 1) % 3, T2 = (AX + 2) % 3;
+        const double s6 = (c.s * c.s) * (1. / 6.);
+        const double D = (c.s * (1. / 12.)) * (psi[3] - psi[4]);
+        const double W1 = s6 * psi[1], W2 = s6 * psi[2];
+        const double M0 = fma(s6, psi[0], P);
+        out[0] = M0;
+        out[1 + AX] = fma(c.u[AX], M0, D);
+        out[1 + T1] = fma(c.u[T1], M0, W1);
+        out[1 + T2] = fma(c.u[T2], M0, W2);
+        out[4] = fma(c.q2h, M0, fma(c2g, P, fma(c.u[AX], D, fma(c.u[T1], W1, c.u[T2] * W2))));
+    }
+}
+
+// Six times the Jiang-Shu WENO5 deviation of a field (Phi_Function_W5, src/WENO.c:118-204, of the minus
+// side less the plus side), from the four split differences of each side.  With IS_k the indicators
+// over three, q_k = IS_k + eps and a = q1 q2, b = q0 q1, c = q0 q2:
+//   3 Phi = N / D - (second difference) / 4,  D = a^2 + 3 b^2 + 6 c^2,  N = a^2 (d0-2d1+d2) + 3/2 b^2 (d1-2d2+d3)
+// and the two sides share one reciprocal.  The indicators of both sides are scaled by the power of two
+// that brings the largest to [1, 2) (exact; the weights are ratios), and the scaled epsilon is held at
+// f = 2^-150: the smallest product, of a side without differences (D = 10 f^4) and a side with one
+// indicator (9 f^2), is then 2^-894, still normal.  The other side's largest differences bound what
+// that floor can change: where it replaces all indicators of a side, that side's differences are below
+// 2^-75 of the other's, less than the rounding of their sum.
+__device__ __forceinline__ double w5_pair(const double eps, const double p[4], const double m[4])
+{
+    double I[2][3], g1[2], g2[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const double *d = h ? m : p;
+        const double t0 = d[0] - d[1], t1 = fma(-3., d[1], d[0]);
+        const double t2 = d[1] - d[2], t3 = d[1] + d[2];
+        const double t4 = d[2] - d[3], t5 = fma(3., d[2], -d[3]);
+        I[h][0] = fma(13. / 3. * t0, t0, t1 * t1);
+        I[h][1] = fma(13. / 3. * t2, t2, t3 * t3);
+        I[h][2] = fma(13. / 3. * t4, t4, t5 * t5);
+        g1[h] = t0 - t2;
+        g2[h] = t2 - t4;
+    }
+    const double mx = fmax(fmax(fmax(I[0][0], I[0][1]), fmax(I[0][2], I[1][0])), fmax(fmax(I[1][1], I[1][2]), eps));
+    const int hi = (int)(__double_as_longlong(mx) >> 32);
+    const double sc = __longlong_as_double((long long)(0x7FE00000 - (hi & 0x7FF00000)) << 32);   // 2^-exponent(mx)
+    const double fl = fmax(eps * sc, 0x1p-150);
+    double N[2], D[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const double q0 = fma(I[h][0], sc, fl), q1 = fma(I[h][1], sc, fl), q2 = fma(I[h][2], sc, fl);
+        const double a = q1 * q2, b = q0 * q1, c = q0 * q2;
+        const double A = a * a, B = 1.5 * b * b;
+        D[h] = fma(6. * c, c, fma(2., B, A));
+        N[h] = fma(B, g2[h], A * g1[h]);
+    }
+    const double num = fma(N[1], D[0], -(N[0] * D[1]));
+    // num / (D[0] D[1]): the hardware reciprocal (24 bits) with one third-order step
+    const double dd = D[0] * D[1];
+    const double r = __builtin_amdgcn_rcp(dd);
+    const double e = fma(-dd, r, 1.0);
+    const double y = num * r;
+    return fma(0.25, g2[0] - g2[1], fma(y, fma(e, e, e), y));
 }
 
 // ---- FP32 forms for the mixed-precision sweeps ------------------------------------------------
