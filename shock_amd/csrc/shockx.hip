@@ -2680,6 +2680,14 @@ extern "C" int shx_create(const shx_desc *desc, shx_case **out)
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) { shx_destroy(c); return set_err(SHX_ERR_HIP, "setup: %s", hipGetErrorString(e)); }
     c->cur = 0;
+    // WENO tiles until shx_tune times them: 4 x 64 along the contiguous axis and 16 x 16 across it, but
+    // 8 x 32 across it for the diagonal metric where the sweep is not the FP64 WENO9 one: that window
+    // holds 1.19 nodes per interface node against 1.40, and its LDS lets a fourth block on a CU (256^3:
+    // xi sweep 0.89 -> 0.82 ms FP64, 0.93 -> 0.81 mixed; 144 x 112 x 128 mixed WENO9: 224 -> 172 and
+    // 247 -> 188 us).  FP64 WENO9 (two blocks by registers) loses 5 % on eta, the general metric
+    // (three blocks either way) 8 %.
+    const bool wide = gm.dims == 3 && (d.quirks & SHX_QUIRK_METRIC_DIAG3D) && (S == 5 || d.precision == SHX_MIXED);
+    for (int dir = 0; dir < 3; dir++) c->wtile[dir] = (wide && gm.st[dir] != 1) ? 1 : 0;
     *out = c;
     return SHX_OK;
 }
