@@ -2475,6 +2475,7 @@ struct shx_case {
     int nan_seen;          // the count last read
     struct HostIo { unsigned long long red[RED_SLOTS]; int nan; int pad; double mms[4]; } *h_io;   // pinned landing slots
     int dev;               // the device current at shx_create (the stream's)
+    int ncu;               // its compute units
     int st_in, st_out, st_bx, st_by;   // buffers of the step in progress (step_begin .. step_end)
     int iface;             // faces of kind SHX_BC_INTERFACE
     shx_blocks *blocks = nullptr;      // the multi-block case that holds this block
@@ -2652,6 +2653,7 @@ extern "C" int shx_create(const shx_desc *desc, shx_case **out)
     }
 
     hipError_t e = hipGetDevice(&c->dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, c->dev);
     if (e == hipSuccess) e = hipStreamCreate(&c->stream);
     if (e != hipSuccess) { delete c; return set_err(SHX_ERR_HIP, "hipStreamCreate: %s", hipGetErrorString(e)); }
     const size_t bytes = sizeof(double) * (size_t)gm.nalloc;
@@ -3206,14 +3208,37 @@ static bool fuse_xi(const shx_case *c)
 static bool fuse_eta(const shx_case *c) { return fuse_xi(c) && fuse_zeta(c); }
 
 static double iso_factor(const shx_case *c);
+// (j, k) columns of a case's march, and the i planes a block of it walks.  A block (one fits on a CU)
+// passes ci + 2g planes one after the other, each bound by its latency, so ci minimises rounds of
+// blocks x planes per block: fewer planes where the columns alone leave CUs idle, longer chunks (fewer
+// halo planes) where they fill them.  cols: the columns of all cases in the launch.  Against 32 planes
+// for every size: 48^3 96 -> 22 us, 97 x 85 x 106 WENO9 136 -> 48, 119 x 96 x 104 full metric 114 -> 49,
+// 176 x 128 x 136 WENO9 167 -> 130, 256^3 940 -> 866 (44 planes).
+static int march_columns(const Geom &gm, const bool xi)
+{
+    return (int)(nblk(gm.ng[2], xi ? GKX : GK) * nblk(gm.ng[1], xi ? GJX : GJ));
+}
+static int march_planes(const shx_case *c, const long cols)
+{
+    const int n = c->gm.ng[0];
+    long best = -1;
+    int planes = n;
+    for (int chunks = 1; chunks <= n; chunks++) {
+        const int ci = (n + chunks - 1) / chunks;
+        const long blocks = cols * nblk(n, ci), rounds = (blocks + c->ncu - 1) / c->ncu;
+        const long cost = rounds * (ci + 2 * c->gm.g);
+        if (best < 0 || cost < best) { best = cost; planes = ci; }
+    }
+    return planes;
+}
 // argument record of the 3D derivative march on stage input pr; xi: with the viscous xi terms
-static GradArgs grad_args(const shx_case *c, double *const *pr, const bool xi)
+static GradArgs grad_args(const shx_case *c, double *const *pr, const bool xi, const int planes)
 {
     GradArgs ga;
     memset(&ga, 0, sizeof ga);
     for (int m = 0; m < 5; m++) ga.pr.f[m] = pr[m];
     for (int m = 0; m < 12; m++) ga.gr.f[m] = c->grad[m];
-    ga.T = c->T; ga.gm = c->gm; ga.k = c->k; ga.ci = 32; ga.tgrad = c->diag ? 0 : 1;
+    ga.T = c->T; ga.gm = c->gm; ga.k = c->k; ga.ci = planes; ga.tgrad = c->diag ? 0 : 1;
     if (xi) {
         for (int m = 0; m < 5; m++) ga.q.f[m] = c->q[m];
         ga.mu = c->mu; ga.m0 = c->met[0]; ga.m4 = c->met[4]; ga.m8 = c->met[8]; ga.J = c->met[9];
@@ -3222,9 +3247,9 @@ static GradArgs grad_args(const shx_case *c, double *const *pr, const bool xi)
     }
     return ga;
 }
-static dim3 march_grid(const Geom &gm, const bool xi)
+static dim3 march_grid(const Geom &gm, const bool xi, const int planes)
 {
-    return dim3(nblk(gm.ng[2], xi ? GKX : GK), nblk(gm.ng[1], xi ? GJX : GJ), nblk(gm.ng[0], 32));
+    return dim3(nblk(gm.ng[2], xi ? GKX : GK), nblk(gm.ng[1], xi ? GJX : GJ), nblk(gm.ng[0], planes));
 }
 // Nodal derivatives of the viscous terms (3D: the march; 2D: pointwise).  xi: the march also adds
 // the viscous xi terms to Q (fuse_xi cases, after the WENO xi sweep).
@@ -3234,9 +3259,10 @@ static int grad_march(shx_case *c, double *const *pr, const bool xi)
     int rc = tbeg(c, xi ? KT_GRADXI : KT_GRAD);
     if (rc) return rc;
     if (gm.dims == 3) {
-        GradArgs ga = grad_args(c, pr, xi);
+        const int planes = march_planes(c, march_columns(gm, xi));
+        GradArgs ga = grad_args(c, pr, xi, planes);
         const void *fn = xi ? (const void *)&k_visc_grad_march_xi<5> : march_kernel(c->d.space_order, ga.tgrad, false);
-        const dim3 grid = flat_grid(march_grid(gm, xi), ga.tg, 0);
+        const dim3 grid = flat_grid(march_grid(gm, xi, planes), ga.tg, 0);
         void *args[] = {&ga};
         HIPCHK(hipLaunchKernel(fn, grid, dim3(xi ? GKX * GJX : GK * GJ), args, 0, c->stream));
     } else {
@@ -4070,6 +4096,8 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
             // periodic ghost fill of the stage input with CalcValues
             std::vector<char> recs, grecs;
             std::vector<dim3> grids, ggrids;
+            long cols = 0;
+            for (int i = 0; i < nc; i++) cols += march_columns(g[i]->gm, false);
             for (int i = 0; i < nc; i++) {
                 shx_case *c = g[i];
                 GhostValuesArgs a;
@@ -4078,14 +4106,9 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                 a.T = c->T; a.mu = c->mu; a.P = c->P; a.C = c->C; a.gm = c->gm; a.k = c->k;
                 put(recs, a);
                 grids.push_back(dim3(nblk(c->gm.ntot, 256)));
-                GradArgs ga;
-                memset(&ga, 0, sizeof ga);
-                for (int m = 0; m < 5; m++) ga.pr.f[m] = in[i][m];
-                ga.T = c->T;
-                for (int m = 0; m < 12; m++) ga.gr.f[m] = c->grad[m];
-                ga.gm = c->gm; ga.k = c->k; ga.ci = 32; ga.tgrad = c->diag ? 0 : 1;
-                put(grecs, ga);
-                if (dims == 3) ggrids.push_back(dim3(nblk(c->gm.ng[2], GK), nblk(c->gm.ng[1], GJ), nblk(c->gm.ng[0], 32)));
+                const int planes = (dims == 3) ? march_planes(c, cols) : 0;
+                put(grecs, grad_args(c, in[i], false, planes));
+                if (dims == 3) ggrids.push_back(march_grid(c->gm, false, planes));
                 else ggrids.push_back(dim3(nblk(c->gm.ntot, 256)));
             }
             batch_add(b, (const void *)&k_ghost_values_batch<false>, (const void *)&k_ghost_values_batch<true>, 256, BK_VALUES, recs, sizeof(GhostValuesArgs), grids);
@@ -4117,9 +4140,12 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
         if (fx) {
             std::vector<char> recs;
             std::vector<dim3> grids;
+            long cols = 0;
+            for (int i = 0; i < nc; i++) cols += march_columns(g[i]->gm, true);
             for (int i = 0; i < nc; i++) {
-                put(recs, grad_args(g[i], in[i], true));
-                grids.push_back(march_grid(g[i]->gm, true));
+                const int planes = march_planes(g[i], cols);
+                put(recs, grad_args(g[i], in[i], true, planes));
+                grids.push_back(march_grid(g[i]->gm, true, planes));
             }
             batch_add(b, (const void *)&k_march_xi_batch<false>, (const void *)&k_march_xi_batch<true>, GKX * GJX,
                       BK_GRAD, recs, sizeof(GradArgs), grids, ORDER_NODES);
