@@ -460,24 +460,29 @@ __device__ __forceinline__ double next_lane(const double v)
     return __longlong_as_double(((long long)nhi << 32) | (unsigned)nlo);
 }
 
-// FP64 WENO5 flux of the interface between nodes ob+2 and ob+3 of a window row, less F[ob+2]: the
-// central part in differences, Theta = F[2] + (D[1] + 6 D[2] - D[3]) / 12 (D[s] = F[s+1] - F[s]),
-// whose F[2] terms telescope in the divergence (node 3's divergence = D[2], returned in dcur, plus
-// the difference of the two interface values), and R Phi.
-// The six nodes pass through registers once: a pair of neighbours gives its differences of F and U,
-// the split differences dF +- lam J dU, and their five characteristic projections (char_project), so
-// the window is read 80 to 120 times per interface instead of 190 (once per non-zero entry of the
+// FP64 WENO flux of the interface between nodes ob+R and ob+R+1 of a window row (R = G-1), less
+// F[ob+R]: the central part in differences D[j] = F[ob+R+j+1] - F[ob+R+j],
+//   Theta - F = (D[-1] + 6 D[0] - D[1]) / 12                                              (WENO5)
+//             = (420 D[0] + 113 (D[-1]-D[1]) - 26 (D[-2]-D[2]) + 3 (D[-3]-D[3])) / 840     (WENO9),
+// whose F terms telescope in the divergence (the upper node's divergence = D[0], returned in dcur,
+// plus the difference of the two interface values), and R Phi.
+// The nodes pass through registers once: a pair of neighbours gives its differences of F and U, the
+// split differences dF +- lam J dU, and their five characteristic projections (char_project), so the
+// window is read 80 to 120 times per WENO5 interface instead of 190 (once per non-zero entry of the
 // left eigenvectors), which had the LDS as busy as the FP64 pipe, and FP64 instructions fall from 926
-// to about 750 (256^3, diagonal metric: xi sweep 1.04 -> 0.83 ms, k_eta 1.42 -> 1.26, k_zeta 1.70 -> 1.55).
-// Bound by the FP64 pipe and its latency at four waves per SIMD, so registers decide: the projections
-// are pinned pair by pair (else the compiler keeps several pairs in flight, 148-166 VGPRs), which
-// leaves 126 VGPRs along zeta.  Along xi and eta one pass over all fields still spilled two registers
-// (k_eta 1.31 ms), so they take the shear fields, which need three of the five components, in a
-// second pass over the row.
-template <int AX, int NW, int VJ>
-__device__ __forceinline__ void weno5_flux(const double *sm, const int ob, const Consts &k, double out[5], double dcur[5])
+// to about 750 (256^3, diagonal metric: xi sweep 1.04 -> 0.82 ms, k_eta 1.42 -> 1.26, k_zeta 1.70 -> 1.57).
+// WENO9, 176 x 128 x 136: xi and eta sweeps 425 and 457 -> 308 and 326 us, k_zeta 684 -> 489 (indicators as
+// sums of squares of the differences, w9_is, and three waves per SIMD instead of two).
+// Bound by the FP64 pipe and its latency, so registers decide: the projections are pinned pair by pair
+// (else the compiler keeps several pairs in flight, 148-166 VGPRs for WENO5), which leaves WENO5 along
+// zeta 128 VGPRs, four waves per SIMD.  Along xi and eta one pass over all fields still spilled two
+// registers (k_eta 1.31 ms), so they take the shear fields, which need three of the five components,
+// in a second pass over the row; so does WENO9 everywhere, for three waves.
+template <int S, int AX, int NW, int VJ>
+__device__ __forceinline__ void weno_flux(const double *sm, const int ob, const Consts &k, double out[5], double dcur[5])
 {
-    const int oc = ob + 2;
+    constexpr int R = (S - 1) / 2;
+    const int oc = ob + R;
     auto mean = [&](const int v) { return 0.5 * (sm[v * NW + oc] + sm[v * NW + oc + 1]); };
     const double cs = mean(V_C);
     const double rho = mean(V_U0);
@@ -491,25 +496,26 @@ __device__ __forceinline__ void weno5_flux(const double *sm, const int ob, const
     char_basis<AX>(c, rho, cs, k.gamma);
     double lam = 0.0;
 #pragma unroll
-    for (int s = 0; s < 6; s++) lam = fmax(lam, fabs(sm[V_LAM * NW + ob + s]));
+    for (int s = 0; s < S + 1; s++) lam = fmax(lam, fabs(sm[V_LAM * NW + ob + s]));
     const double lj = lam * mean(VJ);
 
-    // epsilon of the indicators as w5_pair forms them: a third of the reference's, and scaled with
-    // the square of what the projections leave out (char_project)
-    const double e3 = k.eps * (1. / 3.);
-    const double es = (AX < 0) ? e3 : e3 * (rho * rho), ea = 2.0 * e3;
+    // epsilon of the indicators as w5_pair and w9_pair form them, scaled with the square of what the
+    // projections leave out (char_project)
+    const double e0 = (S == 5) ? k.eps * (1. / 3.) : k.eps;
+    const double es = (AX < 0) ? e0 : e0 * (rho * rho), ea = 2.0 * e0;
     double psi[5];
-    // one pass over the row's five pairs for the fields of MASK (bit f: field f)
+    // one pass over the row's pairs for the fields of MASK (bit f: field f)
     auto pass = [&](auto mask_c) {
         constexpr int MASK = decltype(mask_c)::value;
-        double fp[5][4], fm[5][4];               // split characteristic differences: f+ of pairs 0..3, f- of 4..1
+        double fp[5][S - 1], fm[5][S - 1];       // split characteristic differences: f+ of pairs 0..S-2, f- of S-1..1
         double pf[5], pu[5];
-        auto need = [](const int q) { return AX < 0 || (MASK & 25) || q == 0 || q != 1 + AX && q != 4; };
+        // components the fields need: all, or mass and the transverse momenta for the shear fields
+        auto need = [](const int q) { return AX < 0 || (MASK & 25) || (q != 1 + AX && q != 4); };
 #pragma unroll
         for (int q = 0; q < 5; q++)
             if (need(q)) { pf[q] = sm[(V_F0 + q) * NW + ob]; pu[q] = sm[(V_U0 + q) * NW + ob]; }
 #pragma unroll
-        for (int s = 0; s < 5; s++) {
+        for (int s = 0; s < S; s++) {
             double dF[5] = {}, dU[5] = {};
 #pragma unroll
             for (int q = 0; q < 5; q++) {
@@ -519,7 +525,7 @@ __device__ __forceinline__ void weno5_flux(const double *sm, const int ob, const
                 pf[q] = f; pu[q] = u;
             }
             double g[5], o[5];
-            if (s < 4) {
+            if (s < S - 1) {
 #pragma unroll
                 for (int q = 0; q < 5; q++) g[q] = fma(lj, dU[q], dF[q]);
                 char_project<AX>(c, g, o);
@@ -531,24 +537,30 @@ __device__ __forceinline__ void weno5_flux(const double *sm, const int ob, const
                 for (int q = 0; q < 5; q++) g[q] = fma(-lj, dU[q], dF[q]);
                 char_project<AX>(c, g, o);
 #pragma unroll
-                for (int f = 0; f < 5; f++) if (MASK >> f & 1) fm[f][4 - s] = o[f];
+                for (int f = 0; f < 5; f++) if (MASK >> f & 1) fm[f][S - 1 - s] = o[f];
             }
             // one pair's loads and projections at a time (registers)
 #pragma unroll
             for (int f = 0; f < 5; f++) {
                 if (!(MASK >> f & 1)) continue;
-                if (s < 4) asm volatile("" : "+v"(fp[f][s]));
-                if (s > 0) asm volatile("" : "+v"(fm[f][4 - s]));
+                if (s < S - 1) asm volatile("" : "+v"(fp[f][s]));
+                if (s > 0) asm volatile("" : "+v"(fm[f][S - 1 - s]));
             }
             asm volatile("" ::: "memory");
         }
-        if constexpr (MASK & 1) psi[0] = w5_pair(e3, fp[0], fm[0]);
-        if constexpr (MASK & 2) psi[1] = w5_pair(es, fp[1], fm[1]);
-        if constexpr (MASK & 4) psi[2] = w5_pair(es, fp[2], fm[2]);
-        if constexpr (MASK & 8) psi[3] = w5_pair(ea, fp[3], fm[3]);
-        if constexpr (MASK & 16) psi[4] = w5_pair(ea, fp[4], fm[4]);
+#pragma unroll
+        for (int f = 0; f < 5; f++) {
+            if (!(MASK >> f & 1)) continue;
+            const double e = (f >= 3) ? ea : (f ? es : e0);
+            if constexpr (S == 5) psi[f] = w5_pair(e, fp[f], fm[f]);
+            else psi[f] = w9_pair(e, fp[f], fm[f]);
+        }
     };
-    if constexpr (AX == 0 || AX == 1) {
+    if constexpr (S == 9 && AX < 0) {
+        pass(std::integral_constant<int, 24>{});
+        asm volatile("" : "+v"(psi[3]), "+v"(psi[4]) : : "memory");
+        pass(std::integral_constant<int, 7>{});
+    } else if constexpr (S == 9 || AX == 0 || AX == 1) {
         pass(std::integral_constant<int, 25>{});
         asm volatile("" : "+v"(psi[0]), "+v"(psi[3]), "+v"(psi[4]) : : "memory");
         pass(std::integral_constant<int, 6>{});
@@ -558,10 +570,16 @@ __device__ __forceinline__ void weno5_flux(const double *sm, const int ob, const
     char_assemble<AX>(c, rho, cs * cs * k.igm1, psi, out);
 #pragma unroll
     for (int m = 0; m < 5; m++) {
-        const double *F = &sm[(V_F0 + m) * NW + ob];
-        const double d2 = F[3] - F[2];
-        out[m] += 1. / 12. * (((F[2] - F[1]) - (F[4] - F[3])) + 6. * d2);
-        dcur[m] = d2;
+        const double *F = &sm[(V_F0 + m) * NW + oc];
+        const double d0 = F[1] - F[0];
+        const double a1 = (F[0] - F[-1]) - (F[2] - F[1]);
+        if constexpr (S == 5) {
+            out[m] += 1. / 12. * (a1 + 6. * d0);
+        } else {
+            const double a2 = (F[-1] - F[-2]) - (F[3] - F[2]), a3 = (F[-2] - F[-3]) - (F[4] - F[3]);
+            out[m] += 1. / 840. * (420. * d0 + 113. * a1 - 26. * a2 + 3. * a3);
+        }
+        dcur[m] = d0;
     }
 }
 
@@ -578,9 +596,9 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     constexpr int NT = TA * TDI;
     constexpr int NVK = (AX < 0) ? NV : NV - 3;
     constexpr int VJ = (AX < 0) ? V_J : V_NX;
-    // FP64 WENO5 streams the stencil through registers pair by pair (weno5_flux); the others project
-    // one characteristic field at a time.
-    constexpr bool PAIRS = (S == 5 && !MIX);
+    // the FP64 form streams the stencil through registers pair by pair (weno_flux); the mixed form
+    // projects one characteristic field at a time
+    constexpr bool PAIRS = !MIX;
     // the plus-side interface value of a node's divergence comes from the next lane where a tile row
     // never straddles two wavefronts
     constexpr bool SHFL = (64 % TDI == 0);
@@ -710,7 +728,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     double out[5];
     double dcur[5];                              // PAIRS: F[oc+1] - F[oc], for the divergence
     if constexpr (PAIRS) {
-        weno5_flux<AX, NW, VJ>(sm, ob, k, out, dcur);
+        weno_flux<S, AX, NW, VJ>(sm, ob, k, out, dcur);
     } else {
         const double Jh = (sm[VJ * NW + oc] + sm[VJ * NW + oc + 1]) / 2.0;
         const double u = 0.5 * (sm[V_U * NW + oc] + sm[V_U * NW + oc + 1]);
@@ -739,84 +757,42 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
         // Characteristic projection per field c: a_s = L_c . F_s and b_s = L_c . U_s on the 2G
         // stencil nodes, f+_s = (a_s + lam J b_s)/2 on nodes m-r..m+r and f-_s = (a - lam J b)/2
         // on the mirrored nodes m+r+1..m-r+1 (src/WENO.c:334-385).
-        double phis[5];
         float phif[5];
         auto project = [&](auto cc) {
             constexpr int c = decltype(cc)::value;
-            if constexpr (MIX) {
-                double Ld[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-                if constexpr (AX < 0) left_row<c>(e, Ld);
-                else left_row_ax<c, (AX < 0 ? 0 : AX)>(e, nsig, Ld);
-                float Lf[5];
+            double Ld[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+            if constexpr (AX < 0) left_row<c>(e, Ld);
+            else left_row_ax<c, (AX < 0 ? 0 : AX)>(e, nsig, Ld);
+            float Lf[5];
 #pragma unroll
-                for (int q = 0; q < 5; q++) Lf[q] = (float)Ld[q];
-                const float ljf = (float)lj;
-                // projected differences da_s = L_c . (F_{s+1} - F_s), db_s likewise for U
-                float dp[S - 1], dm[S - 1];
-                float da[2 * G - 1], db[2 * G - 1];
+            for (int q = 0; q < 5; q++) Lf[q] = (float)Ld[q];
+            const float ljf = (float)lj;
+            // projected differences da_s = L_c . (F_{s+1} - F_s), db_s likewise for U
+            float dp[S - 1], dm[S - 1];
+            float da[2 * G - 1], db[2 * G - 1];
 #pragma unroll
-                for (int s = 0; s < 2 * G - 1; s++) {
-                    float x = 0.f, y = 0.f;
-#pragma unroll
-                    for (int q = 0; q < 5; q++) {
-                        if (AX < 0 || lnz(c, AX, q)) {
-                            x += Lf[q] * dfa(q)[ob + s];
-                            y += Lf[q] * dfa(5 + q)[ob + s];
-                        }
-                    }
-                    da[s] = x;
-                    db[s] = y;
-                }
-                // differences of the split fluxes (times 2, see below): f+ on nodes 0..S-1, f- mirrored
-#pragma unroll
-                for (int s = 0; s < S - 1; s++) {
-                    dp[s] = da[s] + ljf * db[s];
-                    dm[s] = da[S - 1 - s] - ljf * db[S - 1 - s];
-                }
-                if constexpr (S == 5) {
-                    phif[c] = 0.5f * (-phi_w5_f(dp[0], dp[1], dp[2], dp[3]) + phi_w5_f(dm[0], dm[1], dm[2], dm[3]));
-                } else {
-                    phif[c] = 0.5f * (-phi_w9_f(dp) + phi_w9_f(dm));
-                }
-                return;
-            } else {
-            // re-read the stencil from LDS for every field instead of keeping 60 values live
-            // across the five fields: 164 instead of 228 VGPRs, three waves per SIMD
-            asm volatile("" ::: "memory");
-            double Lc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            if constexpr (AX < 0) left_row<c>(e, Lc);
-            else left_row_ax<c, (AX < 0 ? 0 : AX)>(e, nsig, Lc);
-            double av[2 * G], bv[2 * G];
-#pragma unroll
-            for (int s = 0; s < 2 * G; s++) {
-                double aa = 0.0, bb = 0.0;
+            for (int s = 0; s < 2 * G - 1; s++) {
+                float x = 0.f, y = 0.f;
 #pragma unroll
                 for (int q = 0; q < 5; q++) {
                     if (AX < 0 || lnz(c, AX, q)) {
-                        aa += Lc[q] * sm[(V_F0 + q) * NW + ob + s];
-                        bb += Lc[q] * sm[(V_U0 + q) * NW + ob + s];
+                        x += Lf[q] * dfa(q)[ob + s];
+                        y += Lf[q] * dfa(5 + q)[ob + s];
                     }
                 }
-                av[s] = aa;
-                bv[s] = bb;
+                da[s] = x;
+                db[s] = y;
             }
-            // The split fluxes are formed without their factor 1/2, which is applied to Phi
-            // instead: Phi is homogeneous of degree one in its inputs (the weights depend on
-            // ratios of the indicators, rescaled by exact powers of two), so halving the inputs
-            // or the output gives the same bits wherever epsilon is far below the indicators.
-            double fp[S], fm[S];
+            // differences of the split fluxes (times 2, see below): f+ on nodes 0..S-1, f- mirrored
 #pragma unroll
-            for (int s = 0; s < S; s++) {
-                fp[s] = av[s] + lj * bv[s];
-                fm[s] = av[2 * G - 1 - s] - lj * bv[2 * G - 1 - s];
+            for (int s = 0; s < S - 1; s++) {
+                dp[s] = da[s] + ljf * db[s];
+                dm[s] = da[S - 1 - s] - ljf * db[S - 1 - s];
             }
-            // WENO9 (FP64 WENO5 goes through weno5_flux): the indicators need the node values
-            if constexpr (S == 9) {
-                double dp_[8], dm_[8];
-#pragma unroll
-                for (int s = 0; s < 8; s++) { dp_[s] = fp[s + 1] - fp[s]; dm_[s] = fm[s] - fm[s + 1]; }
-                phis[c] = 0.5 * (-phi_w9(k.eps, fp, dp_) + phi_w9(k.eps, fm, dm_));
-            }
+            if constexpr (S == 5) {
+                phif[c] = 0.5f * (-phi_w5_f(dp[0], dp[1], dp[2], dp[3]) + phi_w5_f(dm[0], dm[1], dm[2], dm[3]));
+            } else {
+                phif[c] = 0.5f * (-phi_w9_f(dp) + phi_w9_f(dm));
             }
         };
         project(std::integral_constant<int, 0>{});
@@ -836,25 +812,13 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
                                   + 29. * (F[oc + 3] + F[oc - 2]) - 3. * (F[oc + 4] + F[oc - 3]));
             }
             double Rr[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            if constexpr (MIX) {
-                if constexpr (AX < 0) right_row<m>(e, Rr);
-                else right_row_ax<m, (AX < 0 ? 0 : AX)>(e, nsig, Rr);
-                float acc = 0.f;
+            if constexpr (AX < 0) right_row<m>(e, Rr);
+            else right_row_ax<m, (AX < 0 ? 0 : AX)>(e, nsig, Rr);
+            float acc = 0.f;
 #pragma unroll
-                for (int cc = 0; cc < 5; cc++)
-                    if (AX < 0 || rnz(m, AX, cc)) acc += (float)Rr[cc] * phif[cc];
-                out[m] = (double)acc + th;
-            } else if constexpr (AX < 0) {
-                right_row<m>(e, Rr);
-                out[m] = phis[0] * Rr[0] + phis[1] * Rr[1] + phis[2] * Rr[2] + phis[3] * Rr[3] + phis[4] * Rr[4] + th;
-            } else {
-                right_row_ax<m, (AX < 0 ? 0 : AX)>(e, nsig, Rr);
-                double acc = 0.0;
-#pragma unroll
-                for (int cc = 0; cc < 5; cc++)
-                    if (rnz(m, AX, cc)) acc = acc + phis[cc] * Rr[cc];
-                out[m] = acc + th;
-            }
+            for (int cc = 0; cc < 5; cc++)
+                if (AX < 0 || rnz(m, AX, cc)) acc += (float)Rr[cc] * phif[cc];
+            out[m] = (double)acc + th;
         };
         assemble(std::integral_constant<int, 0>{});
         assemble(std::integral_constant<int, 1>{});
@@ -895,7 +859,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
 // spilled), which the LDS of an 8 x 32 or 4 x 64 tile allows too; at three waves (132-134 VGPRs) the xi
 // sweep took 0.87 ms at 256^3 against 0.83.  The other variants are left to the compiler.
 template <int S, int AX, bool MIX>
-constexpr int weno_min_waves() { return (S == 5 && AX >= 0 && !MIX) ? 4 : 1; }
+constexpr int weno_min_waves() { return (AX >= 0 && !MIX) ? (S == 5 ? 4 : 3) : 1; }
 
 template <int S, int TA, int TDI, int AX, bool MIX>
 __global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, AX, MIX>())) void k_weno(WenoArgs a)
@@ -1515,7 +1479,7 @@ __device__ __forceinline__ void zeta_body(const ZetaArgs &z, const int bx, const
 // FP64 W5: held to 128 VGPRs (four waves per SIMD, as the LDS allows): 1.55 ms at 256^3 against
 // 1.67 at three waves
 template <int S, bool MIX>
-__global__ __launch_bounds__(256, ((S == 5 && !MIX) ? 4 : 1)) void k_zeta(ZetaArgs z)
+__global__ __launch_bounds__(256, (weno_min_waves<S, 2, MIX>())) void k_zeta(ZetaArgs z)
 {
     __shared__ double lds[zeta_lds<S, MIX>()];
     int bx, by, bz;
@@ -2043,7 +2007,7 @@ __global__ __launch_bounds__(TA * TDI) void k_visc_batch(BATCH_PARAMS(ViscArgs))
     });
 }
 template <int S, bool MIX, bool P>
-__global__ __launch_bounds__(256, ((S == 5 && !MIX) ? 4 : 1)) void k_zeta_batch(BATCH_PARAMS(ZetaArgs))
+__global__ __launch_bounds__(256, (weno_min_waves<S, 2, MIX>())) void k_zeta_batch(BATCH_PARAMS(ZetaArgs))
 {
     __shared__ double lds[zeta_lds<S, MIX>()];
     batch_walk<P>(total, [&](const int b) {
@@ -2686,8 +2650,8 @@ extern "C" int shx_create(const shx_desc *desc, shx_case **out)
     // 8 x 32 across it for the diagonal metric where the sweep is not the FP64 WENO9 one: that window
     // holds 1.19 nodes per interface node against 1.40, and its LDS lets a fourth block on a CU (256^3:
     // xi sweep 0.89 -> 0.82 ms FP64, 0.93 -> 0.81 mixed; 144 x 112 x 128 mixed WENO9: 224 -> 172 and
-    // 247 -> 188 us).  FP64 WENO9 (two blocks by registers) loses 5 % on eta, the general metric
-    // (three blocks either way) 8 %.
+    // 247 -> 188 us).  FP64 WENO9 and the general metric run three blocks either way and lose on eta
+    // (176 x 128 x 136 WENO9 326 -> 352 us, 119 x 96 x 104 general 79 -> 87).
     const bool wide = gm.dims == 3 && (d.quirks & SHX_QUIRK_METRIC_DIAG3D) && (S == 5 || d.precision == SHX_MIXED);
     for (int dir = 0; dir < 3; dir++) c->wtile[dir] = (wide && gm.st[dir] != 1) ? 1 : 0;
     *out = c;

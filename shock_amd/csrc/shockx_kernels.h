@@ -68,64 +68,6 @@ __device__ __forceinline__ long padded_node(const Geom &gm, const long t, int ij
 }
 
 // ---------------------------------------------------------------------------------------
-// Characteristic eigenvectors of the Euler flux Jacobian in direction nh at the arithmetic
-// interface average (CalcEigenVectorsIn*Direction, src/WENO.c:1085-1548).
-__device__ __forceinline__ void eigvec(const double nx, const double ny, const double nz,
-                                       const double u, const double v, const double w,
-                                       const double rho, const double cs, const double gamma,
-                                       double L[5][5], double R[5][5])
-{
-    const double s2 = 1.4142135623730951;  // sqrt(2.), correctly rounded
-    const double q2 = (u * u + v * v + w * w);
-    const double M = sqrt(q2) / cs;
-    const double gc = ((gamma - 1.0) / (cs * cs));
-    const double ics = (1. / (cs * s2));
-    const double un = (u * nx + v * ny + w * nz);
-    const double irho = 1. / rho;
-    const double hm = 1.0 - 0.5 * (gamma - 1.0) * (M * M);
-    const double h0 = q2 / 2. + cs * cs / (gamma - 1.);
-
-    R[0][0] = nx; R[0][1] = ny; R[0][2] = nz; R[0][3] = ics; R[0][4] = ics;
-    R[1][0] = u * nx; R[1][1] = u * ny - rho * nz; R[1][2] = u * nz + rho * ny;
-    R[1][3] = ics * (u + nx * cs); R[1][4] = ics * (u - nx * cs);
-    R[2][0] = v * nx + rho * nz; R[2][1] = v * ny; R[2][2] = v * nz - rho * nx;
-    R[2][3] = ics * (v + ny * cs); R[2][4] = ics * (v - ny * cs);
-    R[3][0] = w * nx - rho * ny; R[3][1] = w * ny + rho * nx; R[3][2] = w * nz;
-    R[3][3] = ics * (w + nz * cs); R[3][4] = ics * (w - nz * cs);
-    R[4][0] = q2 / 2. * nx + rho * (v * nz - w * ny);
-    R[4][1] = q2 / 2. * ny + rho * (w * nx - u * nz);
-    R[4][2] = q2 / 2. * nz + rho * (u * ny - v * nx);
-    R[4][3] = ics * (h0 + cs * un);
-    R[4][4] = ics * (h0 - cs * un);
-
-    L[0][0] = nx * hm - irho * (v * nz - w * ny);
-    L[0][1] = gc * u * nx;
-    L[0][2] = gc * v * nx + nz * irho;
-    L[0][3] = gc * w * nx - ny * irho;
-    L[0][4] = -gc * nx;
-    L[1][0] = ny * hm - irho * (w * nx - u * nz);
-    L[1][1] = gc * u * ny - nz * irho;
-    L[1][2] = gc * v * ny;
-    L[1][3] = gc * w * ny + nx * irho;
-    L[1][4] = -gc * ny;
-    L[2][0] = nz * hm - irho * (u * ny - v * nx);
-    L[2][1] = gc * u * nz + ny * irho;
-    L[2][2] = gc * v * nz - nx * irho;
-    L[2][3] = gc * w * nz;
-    L[2][4] = -gc * nz;
-    const double gs = (gamma - 1.0) / cs;
-    L[3][0] = ics * ((gamma - 1.0) * q2 / 2. - cs * un);
-    L[3][1] = (-gs * u + nx) / s2;
-    L[3][2] = (-gs * v + ny) / s2;
-    L[3][3] = (-gs * w + nz) / s2;
-    L[3][4] = (gamma - 1.) * ics;
-    L[4][0] = ics * ((gamma - 1.0) * q2 / 2. + cs * un);
-    L[4][1] = (-gs * u - nx) / s2;
-    L[4][2] = (-gs * v - ny) / s2;
-    L[4][3] = (-gs * w - nz) / s2;
-    L[4][4] = (gamma - 1.) * ics;
-}
-
 // Reciprocal from the hardware estimate (v_rcp_f64) refined by two Newton steps: within an ulp
 // of 1/x for the normal, finite arguments the flux kernels pass, at a fraction of the cost of
 // the IEEE-exact division sequence.
@@ -282,25 +224,6 @@ __device__ __forceinline__ void right_row_ax(const Eig &e, const double s, doubl
     }
 }
 
-// Smoothness indicators s_k = IS_k + eps scaled by a common power of two so the largest lies in
-// [1/2, 1), each clamped from below at 2^lo.  The nonlinear weights d_k / s_k^2 normalised to sum
-// one are unchanged by the common scale; the clamp only touches stencils whose weight is below
-// 2^(2 lo) of the largest one's.
-template <int N>
-__device__ __forceinline__ void scaled_sq(double s[N], const int lo)
-{
-    double mx = s[0];
-#pragma unroll
-    for (int i = 1; i < N; i++) mx = fmax(mx, s[i]);
-    const int ex = __builtin_amdgcn_frexp_exp(mx);
-    const double floor_ = __builtin_amdgcn_ldexp(1.0, lo);
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-        const double t = fmax(__builtin_amdgcn_ldexp(s[i], -ex), floor_);
-        s[i] = t * t;
-    }
-}
-
 // ---- characteristic projection without the eigenvector entries ------------------------------------
 // The left and right eigenvectors above applied to a vector g = (g0, gm, g4) of differences through
 // S = gm - g0 u (momentum less the mean velocity's share) and t = g4 - u.S - |u|^2/2 g0 (the pressure
@@ -392,6 +315,23 @@ __device__ __forceinline__ void char_assemble(const CharBasis &c, const double r
     }
 }
 
+// 2^-floor(log2 x) of a positive normal x
+__device__ __forceinline__ double inv_pow2(const double x)
+{
+    const int hi = (int)(__double_as_longlong(x) >> 32);
+    return __longlong_as_double((long long)(0x7FE00000 - (hi & 0x7FF00000)) << 32);
+}
+// N[1] / D[1] - N[0] / D[0] with one reciprocal: the hardware's (24 bits) and one third-order step
+__device__ __forceinline__ double pair_quotient(const double N[2], const double D[2])
+{
+    const double num = fma(N[1], D[0], -(N[0] * D[1]));
+    const double dd = D[0] * D[1];
+    const double r = __builtin_amdgcn_rcp(dd);
+    const double e = fma(-dd, r, 1.0);
+    const double y = num * r;
+    return fma(y, fma(e, e, e), y);
+}
+
 // Six times the Jiang-Shu WENO5 deviation of a field (Phi_Function_W5, src/WENO.c:118-204, of the minus
 // side less the plus side), from the four split differences of each side.  With IS_k the indicators
 // over three, q_k = IS_k + eps and a = q1 q2, b = q0 q1, c = q0 q2:
@@ -418,8 +358,7 @@ __device__ __forceinline__ double w5_pair(const double eps, const double p[4], c
         g2[h] = t2 - t4;
     }
     const double mx = fmax(fmax(fmax(I[0][0], I[0][1]), fmax(I[0][2], I[1][0])), fmax(fmax(I[1][1], I[1][2]), eps));
-    const int hi = (int)(__double_as_longlong(mx) >> 32);
-    const double sc = __longlong_as_double((long long)(0x7FE00000 - (hi & 0x7FF00000)) << 32);   // 2^-exponent(mx)
+    const double sc = inv_pow2(mx);
     const double fl = fmax(eps * sc, 0x1p-150);
     double N[2], D[2];
 #pragma unroll
@@ -430,19 +369,15 @@ __device__ __forceinline__ double w5_pair(const double eps, const double p[4], c
         D[h] = fma(6. * c, c, fma(2., B, A));
         N[h] = fma(B, g2[h], A * g1[h]);
     }
-    const double num = fma(N[1], D[0], -(N[0] * D[1]));
-    // num / (D[0] D[1]): the hardware reciprocal (24 bits) with one third-order step
-    const double dd = D[0] * D[1];
-    const double r = __builtin_amdgcn_rcp(dd);
-    const double e = fma(-dd, r, 1.0);
-    const double y = num * r;
-    return fma(0.25, g2[0] - g2[1], fma(y, fma(e, e, e), y));
+    return fma(0.25, g2[0] - g2[1], pair_quotient(N, D));
 }
 
 // ---- FP32 forms for the mixed-precision sweeps ------------------------------------------------
-// Same formulas as phi_w5_fast / phi_w9 on locally offset FP32 inputs (node-to-node differences).  epsilon is dropped: FP32 cannot hold the
-// reference's 10 sqrt(DBL_MIN), and the clamp in scaled_sq_f gives the ideal weights where all
-// indicators vanish, which is what an epsilon far below every indicator does.
+// Smoothness indicators scaled by a common power of two so that the largest lies in [1/2, 1), each
+// clamped from below at 2^lo and squared; the weights are ratios, so the scale drops out.  Inputs are
+// FP32 node-to-node differences.  epsilon is dropped: FP32 cannot hold the reference's
+// 10 sqrt(DBL_MIN), and the clamp gives the ideal weights where all indicators vanish, which is what an
+// epsilon far below every indicator does.
 template <int N>
 __device__ __forceinline__ void scaled_sq_f(float s[N], const int lo)
 {
@@ -522,72 +457,68 @@ __device__ __forceinline__ float phi_w9_f(const float *d)
          + (1.f / 60.f) * w4 * (3.f * q2 - 2.f * q3 + 3.f * q4) - (1.f / 840.f) * (39.f * q2 - 14.f * q3 + 3.f * q4);
 }
 
-// Balsara-Shu WENO9 (Phi_Function_W9, src/WENO.c:11-116); f: 9 point values, d: 8 differences.
-// The smoothness indicators keep the reference's quadratic forms in the point values.
-__device__ __forceinline__ double phi_w9(const double eps, const double *f, const double *d)
+// Balsara-Shu indicator of one five-point sub-stencil from its four differences, as the sum of squares
+// of the LDL^T factorisation of its quadratic form (exact rationals, as in phi_w9_f): the same number
+// as the reference's form in point values (src/WENO.c:11-116), without its cancellation between terms
+// of the size of the squared values, in 14 operations instead of 20.  K: sub-stencil 0, 1 or 2; 3 and 4
+// are 1 and 0 mirrored.
+template <int K>
+__device__ __forceinline__ double w9_is(const double a, const double b, const double c, const double d)
 {
-    const double is0 = f[0] * (22658. * f[0] - 208501. * f[1] + 364863. * f[2] - 288007. * f[3] + 86329. * f[4])
-        + f[1] * (482963. * f[1] - 1704396. * f[2] + 1358458. * f[3] - 411487. * f[4])
-        + f[2] * (1521393. * f[2] - 2462076. * f[3] + 758823. * f[4])
-        + f[3] * (1020563. * f[3] - 649501. * f[4])
-        + f[4] * (107918. * f[4]);
-    const double is1 = f[1] * (6908. * f[1] - 60871. * f[2] + 99213. * f[3] - 70237. * f[4] + 18079. * f[5])
-        + f[2] * (138563. * f[2] - 464976. * f[3] + 337018. * f[4] - 88297. * f[5])
-        + f[3] * (406293. * f[3] - 611976. * f[4] + 165153. * f[5])
-        + f[4] * (242723. * f[4] - 140251. * f[5])
-        + f[5] * (22658. * f[5]);
-    const double is2 = f[2] * (6908. * f[2] - 51001. * f[3] + 67923. * f[4] - 38947. * f[5] + 8209. * f[6])
-        + f[3] * (104963. * f[3] - 299076. * f[4] + 179098. * f[5] - 38947. * f[6])
-        + f[4] * (231153. * f[4] - 299076. * f[5] + 67923. * f[6])
-        + f[5] * (104963. * f[5] - 51001. * f[6])
-        + f[6] * (6908. * f[6]);
-    const double is3 = f[3] * (22658. * f[3] - 140251. * f[4] + 165153. * f[5] - 88297. * f[6] + 18079. * f[7])
-        + f[4] * (242723. * f[4] - 611976. * f[5] + 337018. * f[6] - 70237. * f[7])
-        + f[5] * (406293. * f[5] - 464976. * f[6] + 99213. * f[7])
-        + f[6] * (138563. * f[6] - 60871. * f[7])
-        + f[7] * (6908. * f[7]);
-    const double is4 = f[4] * (107918. * f[4] - 649501. * f[5] + 758823. * f[6] - 411487. * f[7] + 86329. * f[8])
-        + f[5] * (1020563. * f[5] - 2462076. * f[6] + 1358458. * f[7] - 288007. * f[8])
-        + f[6] * (1521393. * f[6] - 1704396. * f[7] + 364863. * f[8])
-        + f[7] * (482963. * f[7] - 208501. * f[8])
-        + f[8] * (22658. * f[8]);
-    // weights d_k / q_k normalised with one reciprocal: w_k = d_k prod_{j != k} q_j / D
-    double q[5] = {is0 + eps, is1 + eps, is2 + eps, is3 + eps, is4 + eps};
-    scaled_sq<5>(q, -120);
-    const double p01 = q[0] * q[1], p012 = p01 * q[2], s34 = q[3] * q[4], s234 = q[2] * s34;
-    const double P0 = q[1] * s234, P1 = q[0] * s234, P2 = p01 * s34, P3 = p012 * q[4], P4 = p012 * q[3];
-    const double A0 = (1. / 126.) * P0, A2 = (10. / 21.) * P2, A3 = (20. / 63.) * P3, A4 = (5. / 126.) * P4;
-    const double ia = frcp(A0 + (10. / 63.) * P1 + A2 + A3 + A4);
-    const double w0 = A0 * ia, w2 = A2 * ia, w3 = A3 * ia, w4 = A4 * ia;
-    const double q1 = d[0] - 4. * d[1] + 6. * d[2] - 4. * d[3] + d[4];
-    const double q2 = d[1] - 4. * d[2] + 6. * d[3] - 4. * d[4] + d[5];
-    const double q3 = d[2] - 4. * d[3] + 6. * d[4] - 4. * d[5] + d[6];
-    const double q4 = d[3] - 4. * d[4] + 6. * d[5] - 4. * d[6] + d[7];
-    return 1. / 5. * w0 * q1 + 1. / 20. * w2 * q2 + 1. / 60. * w3 * (3. * q2 - 2. * q3)
-         + 1. / 60. * w4 * (3. * q2 - 2. * q3 + 3. * q4) - 1. / 840. * (39. * q2 - 14. * q3 + 3. * q4);
+    if constexpr (K == 0) {
+        const double y0 = fma(-86329. / 45316., d, fma(100839. / 22658., c, fma(-163185. / 45316., b, a)));
+        const double y1 = fma(1813059. / 838195., d, fma(-41089198. / 14249315., c, b));
+        const double y2 = fma(-350813921. / 232768856., d, c);
+        return fma(22658. * y0, y0, fma(299235615. / 90632. * y1, y1,
+               fma(39105167808. / 14249315. * y2, y2, (116566909305. / 29096107. * d) * d)));
+    } else if constexpr (K == 1) {
+        const double y0 = fma(-18079. / 13816., d, fma(26079. / 6908., c, fma(-47055. / 13816., b, a)));
+        const double y1 = fma(5686883. / 5880675., d, fma(-12448558. / 5880675., c, b));
+        const double y2 = fma(-146761231. / 232768856., d, c);
+        return fma(6908. * y0, y0, fma(123494175. / 27632. * y1, y1,
+               fma(13035055936. / 1960225. * y2, y2, (116566909305. / 29096107. * d) * d)));
+    } else {
+        const double y0 = fma(-8209. / 13816., d, fma(15369. / 6908., c, fma(-37185. / 13816., b, a)));
+        const double y1 = fma(5686883. / 14249315., d, fma(-1032654. / 838195., c, b));
+        const double y2 = fma(-20636113. / 51089708., d, c);
+        return fma(6908. * y0, y0, fma(299235615. / 27632. * y1, y1,
+               fma(8583070944. / 838195. * y2, y2, (233133818610. / 217131259. * d) * d)));
+    }
 }
 
-// 30 viscous metric factors of one node for direction `dir` (CreateViscidMetric,
-// src/Functions.c:6245-6386): the Newtonian stress contracted with metric rows a (= dir) and
-// r_b (b = xi, eta, zeta), times J.
-__device__ __forceinline__ void visc_fac(const int dir, const double m[10], double fac[30])
+// Six times the WENO9 deviation of a field (Phi_Function_W9, src/WENO.c:11-116, of the minus side less
+// the plus side, as w5_pair) from the eight split differences of each side.  Each side's indicators are
+// scaled by the power of two that brings the largest to [1, 2) and epsilon is held at f = 2^-80 there:
+// with s_k = (IS_k + eps)^2 the sums D = sum_k 126 d_k prod_{j != k} s_j are at least f^6, so the product
+// of both sides' stays normal for the one reciprocal, and a capped weight is below 2^-160.
+__device__ __forceinline__ double w9_pair(const double eps, const double p[8], const double m[8])
 {
-    const double J = m[9];
-    const double a0 = m[3 * dir], a1 = m[3 * dir + 1], a2 = m[3 * dir + 2];
+    double N[2], D[2], T[2];
 #pragma unroll
-    for (int b = 0; b < 3; b++) {
-        const double r0 = m[3 * b], r1 = m[3 * b + 1], r2 = m[3 * b + 2];
-        fac[0 + b] = J * (4.0 / 3.0 * r0 * a0 + r1 * a1 + r2 * a2);
-        fac[3 + b] = J * (-2.0 / 3.0 * r1 * a0 + r0 * a1);
-        fac[6 + b] = J * (-2.0 / 3.0 * r2 * a0 + r0 * a2);
-        fac[9 + b] = J * (r1 * a0 - 2.0 / 3.0 * r0 * a1);
-        fac[12 + b] = J * (r0 * a0 + 4.0 / 3.0 * r1 * a1 + r2 * a2);
-        fac[15 + b] = J * (-2.0 / 3.0 * r2 * a1 + r1 * a2);
-        fac[18 + b] = J * (r2 * a0 - 2.0 / 3.0 * r0 * a2);
-        fac[21 + b] = J * (r2 * a1 - 2.0 / 3.0 * r1 * a2);
-        fac[24 + b] = J * (r0 * a0 + r1 * a1 + 4.0 / 3.0 * r2 * a2);
-        fac[27 + b] = J * (r0 * a0 + r1 * a1 + r2 * a2);
+    for (int h = 0; h < 2; h++) {
+        const double *d = h ? m : p;
+        double s[5] = {w9_is<0>(d[0], d[1], d[2], d[3]), w9_is<1>(d[1], d[2], d[3], d[4]),
+                       w9_is<2>(d[2], d[3], d[4], d[5]), w9_is<1>(d[6], d[5], d[4], d[3]),
+                       w9_is<0>(d[7], d[6], d[5], d[4])};
+        const double mx = fmax(fmax(fmax(s[0], s[1]), fmax(s[2], s[3])), fmax(s[4], eps));
+        const double sc = inv_pow2(mx);
+        const double fl = fmax(eps * sc, 0x1p-80);
+#pragma unroll
+        for (int k = 0; k < 5; k++) {
+            const double q = fma(s[k], sc, fl);
+            s[k] = q * q;
+        }
+        const double p01 = s[0] * s[1], p012 = p01 * s[2], s34 = s[3] * s[4], s234 = s[2] * s34;
+        const double P0 = s[1] * s234, P1 = s[0] * s234, P2 = p01 * s34, P3 = p012 * s[4], P4 = p012 * s[3];
+        D[h] = fma(5., P4, fma(40., P3, fma(60., P2, fma(20., P1, P0))));
+        double v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = fma(6., d[k + 2], fma(-4., d[k + 1] + d[k + 3], d[k] + d[k + 4]));
+        const double r = fma(3., v[1], -2. * v[2]);
+        N[h] = fma(0.25 * P4, fma(3., v[3], r), fma(2. * P3, r, fma(9. * P2, v[1], (0.6 * P0) * v[0])));
+        T[h] = fma(39., v[1], fma(-14., v[2], 3. * v[3]));
     }
+    return fma(1. / 280., T[0] - T[1], pair_quotient(N, D));
 }
 
 __device__ __forceinline__ double pressure(const Consts &k, double rho, double u, double v, double w, double e)
