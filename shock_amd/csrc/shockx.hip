@@ -6,7 +6,7 @@
 //   k_calc_values      T and mu on every padded node (CalcValues, src/Functions.c:2392-2481;
 //                      p, c and theta are recomputed inside the flux kernels instead of stored)
 //   k_face_bc          boundary writers of non-periodic faces, in face order (src/BC.c:13-74)
-//   k_visc_grad_march  nodal derivatives of u,v,w,T (src/ZD.c:697-810); k_visc_grad in 2D
+//   k_visc_grad_march  nodal derivatives of u,v,w,T (src/ZD.c:697-810)
 //   k_weno             one launch per direction: LDS-staged pencil, characteristic WENO
 //                      interface fluxes and their divergence fused, interface fluxes never
 //                      reach HBM (CalcFluxesIn*Direction, src/WENO.c:206-1083)
@@ -16,6 +16,7 @@
 //                      into another buffer (the reference updates in place after all fluxes of
 //                      the stage are assembled, which the separate buffer reproduces exactly)
 //   k_rk_update        source + RK update for inviscid runs
+//   k_plane            2D: all of the above after the ghost fill in one kernel per stage
 // Every hot kernel body is also reachable through a k_*_batch twin that runs many cases from
 // one launch over a tile work list (shx_batch_*).
 #include "shockx_kernels.h"
@@ -306,8 +307,9 @@ __global__ void k_carry_ghosts(CFields5 from, Fields5 to, Geom gm)
 {
     carry_body(from, to, gm, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
-// every ghost node (periodic directions included) copied from one buffer to another
-__global__ void k_copy_ghosts(CFields5 from, Fields5 to, Geom gm)
+// every ghost node (periodic directions included) copied from one buffer to another; image: from its
+// periodic image there (all directions periodic: what a ghost fill of that buffer holds)
+__global__ void k_copy_ghosts(CFields5 from, Fields5 to, Geom gm, int image)
 {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= gm.ntot) return;
@@ -318,8 +320,10 @@ __global__ void k_copy_ghosts(CFields5 from, Fields5 to, Geom gm)
     for (int d = 0; d < 3; d++)
         if (gm.ng[d] > 1 && (idx[d] < gm.lo[d] || idx[d] >= gm.lo[d] + gm.n[d])) ghost = true;
     if (!ghost) return;
+    long src = n;
+    if (image) src = periodic_image(gm, idx, ghost);
 #pragma unroll
-    for (int m = 0; m < 5; m++) to.f[m][n] = from.f[m][n];
+    for (int m = 0; m < 5; m++) to.f[m][n] = from.f[m][src];
 }
 
 // T = |p/rho| and mu (Sutherland, or 1 under the manufactured solution) of one node, CalcValues
@@ -429,6 +433,7 @@ struct WenoArgs {
     int first;            // 1: Q = -div (first direction of the stage), 0: Q -= div
     int coalesce_d;       // load mapping: 1 when the sweep axis is contiguous in memory
     int alignA;           // tiles start at padded A index 0 (A axis contiguous, pitch padded)
+    int wrap;             // the stage input's ghosts are read at their periodic image (2D tiles)
     Consts k;
 };
 
@@ -592,7 +597,9 @@ __device__ __forceinline__ void weno_flux(const double *sm, const int ob, const 
 
 // KEEP: leave Q alone and return this sweep's contribution of the thread's node in keep[5] (a
 // fused kernel adds it later); otherwise Q = -div (first sweep of the stage) or Q -= div.
-template <int S, int TA, int TDI, int AX, bool MIX, bool KEEP = false>
+// NT: threads that sweep the tile together, a multiple of the wavefront not below TA * TDI (those past it
+// repeat the last row); a group of NT threads within a larger block.
+template <int S, int TA, int TDI, int AX, bool MIX, bool KEEP = false, int NT = TA * TDI>
 __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const int by, const int bz,
                                           double *lds, double *keep = nullptr)
 {
@@ -600,7 +607,6 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     constexpr int R = G - 1;
     constexpr int WD = TDI - 1 + 2 * G;   // window nodes along the sweep
     constexpr int NW = WD * TA;
-    constexpr int NT = TA * TDI;
     constexpr int NVK = (AX < 0) ? NV : NV - 3;
     constexpr int VJ = (AX < 0) ? V_J : V_NX;
     // the FP64 form streams the stencil through registers pair by pair (weno_flux); the mixed form
@@ -618,7 +624,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
         return (j < 8) ? (float *)(lds + V_U1 * NW) + j * NW : (float *)(lds + NVK * NW) + (j - 8) * NW;
     };
 
-    const int t = threadIdx.x;
+    const int t = (NT == TA * TDI) ? threadIdx.x : threadIdx.x % NT;
     // first padded A index of the tile (aligned to TA when the A axis is contiguous in memory)
     const int pa0 = a.alignA ? bx * TA : bx * TA + a.oA;
     const int b = by;
@@ -639,8 +645,11 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
         int dp = d0 - G + dd + a.oD;
         dp = max(0, min(dp, a.ngD - 1));
         const long n = bbase + (long)pa * a.sA + (long)dp * a.sD;
-        const double rho = a.pr.f[0][n], u = a.pr.f[1][n], v = a.pr.f[2][n], w = a.pr.f[3][n],
-                     e = a.pr.f[4][n];
+        // wrap: a ghost node of the stage input is read at its periodic image
+        long ns = n;
+        if (NT != TA * TDI && a.wrap) ns += (long)(dp < a.oD ? a.nD : (dp >= a.oD + a.nD ? -a.nD : 0)) * a.sD;
+        const double rho = a.pr.f[0][ns], u = a.pr.f[1][ns], v = a.pr.f[2][ns], w = a.pr.f[3][ns],
+                     e = a.pr.f[4][ns];
         const double J = a.J[n];
         double p = pressure_fast(k, rho, u, v, w, e);
         const double ir = frcp(rho);
@@ -729,7 +738,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     }
 
     // phase 2: interface flux between nodes (d0-1+di) and (d0+di)
-    const int ta = t / TDI, di = t - ta * TDI;
+    const int ta = (NT == TA * TDI) ? t / TDI : min(t / TDI, TA - 1), di = t % TDI;
     const int ob = ta * WD + di;                 // window position of the stencil's first node
     const int oc = ob + R;                       // left node of the interface
     double out[5];
@@ -847,7 +856,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     }
 
     // phase 3: divergence into Q for the tile's TDI-1 nodes
-    if (di < TDI - 1) {
+    if (di < TDI - 1 && t < TA * TDI) {
         const int dn = d0 + di;
         const int pa = pa0 + ta;
         if (dn < a.nD && pa >= a.oA && pa < a.oA + a.nA) {
@@ -1035,7 +1044,6 @@ struct ViscArgs {
     int ngA;                      // padded extent of the A axis
     int coalesce_d;
     int alignA;
-    int three;
     int bug;                      // zeta stencil k offset taken from j (DIR = 2 only)
     int fuse_rk;                  // last sweep of the stage: apply the stage update (rk)
     int iso_hi;                   // the upper face of the sweep direction is an isothermal wall:
@@ -1388,7 +1396,7 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
                     dv += k.zd_der[l] * sm[VS_V * NW + ob + l];
                     dw += k.zd_der[l] * sm[VS_W * NW + ob + l];
                 }
-                g[0 * 3 + DIR] = du; g[1 * 3 + DIR] = dv; g[2 * 3 + DIR] = a.three ? dw : 0.0;
+                g[0 * 3 + DIR] = du; g[1 * 3 + DIR] = dv; g[2 * 3 + DIR] = dw;
             }
             const double mu = sm[VS_MU * NW + p];
             double prod;
@@ -1418,7 +1426,7 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
                 qv[0] = q0[0];
                 qv[1] = q0[1] + k.psi * dF[0];
                 qv[2] = q0[2] + k.psi * dF[1];
-                qv[3] = a.three ? q0[3] + k.psi * dF[2] : q0[3];
+                qv[3] = q0[3] + k.psi * dF[2];
                 const double gh = (a.iso_hi && dn == a.nD - 1) ? a.gam_iso : k.gam_heat;
                 qv[4] = q0[4] + (gh * dF[3] + k.psi * (work + prod));
                 const double J = DIAG ? sm[(VS_M + 3) * NW + p] : sm[(VS_M + 9) * NW + p];
@@ -1441,8 +1449,7 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
                 if (ADD) a.q.f[0][n] = q0[0];
                 a.q.f[1][n] = q0[1] + k.psi * dF[0];
                 a.q.f[2][n] = q0[2] + k.psi * dF[1];
-                if (a.three) a.q.f[3][n] = q0[3] + k.psi * dF[2];
-                else if (ADD) a.q.f[3][n] = q0[3];
+                a.q.f[3][n] = q0[3] + k.psi * dF[2];
                 const double gh = (a.iso_hi && dn == a.nD - 1) ? a.gam_iso : k.gam_heat;
                 a.q.f[4][n] = q0[4] + (gh * dF[3] + k.psi * (work + prod));
             }
@@ -1563,43 +1570,10 @@ __global__ __launch_bounds__(256) void k_rk_update(UpdArgs A)
 // ---- viscous derivatives ------------------------------------------------------------------
 // grad order: u_xi,u_eta,u_zeta, v_xi,v_eta,v_zeta, w_xi,w_eta,w_zeta, T_xi,T_eta,T_zeta.
 // Direction d is evaluated where the node's d index is interior (all transverse nodes).
-__device__ __forceinline__ void grad_body(const CFields5 &pr, const gcdp T, const Fields12 &gr,
-                                          const Geom &gm, const Consts &k, const long t)
-{
-    if (t >= gm.ntot) return;
-    int idx[3];
-    const long n = padded_node(gm, t, idx);
-    const int half = gm.g;
-    const int nl = 2 * gm.g + 1;   // S + 2 points
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        if (d >= gm.dims) continue;
-        if (idx[d] < gm.lo[d] || idx[d] >= gm.lo[d] + gm.n[d]) continue;
-        const long st = gm.st[d];
-        double du = 0.0, dv = 0.0, dw = 0.0, dT = 0.0;
-        for (int l = 0; l < nl; l++) {
-            const long m = n + (long)(l - half) * st;
-            const double c = k.zd_der[l];
-            du += c * pr.f[1][m];
-            dv += c * pr.f[2][m];
-            dT += c * T[m];
-            if (gm.dims == 3) dw += c * pr.f[3][m];
-        }
-        gr.f[0 + d][n] = du;
-        gr.f[3 + d][n] = dv;
-        if (gm.dims == 3) gr.f[6 + d][n] = dw;
-        gr.f[9 + d][n] = dT;
-    }
-}
-__global__ void k_visc_grad(CFields5 pr, const double *T, Fields12 gr, Geom gm, Consts k)
-{
-    grad_body(pr, T, gr, gm, k, (long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
 // 3D nodal derivatives, marching along i.  A block owns a GK x GJ column of (j, k) nodes over the
 // full padded extent and walks a chunk of i planes: every plane is read from HBM once per chunk
 // into LDS with a g-wide halo; the j and k derivatives come from there, the i derivative from a
-// register window of 2g+1 plane centres per thread.  Outputs as k_visc_grad; the T
+// register window of 2g+1 plane centres per thread.  The T
 // derivatives only when `tgrad` (the diagonal-metric viscous sweeps never read them).
 //
 // VX (3D diagonal metric): the viscous xi direction rides along (CalcViscidFluxesInXiDirection-
@@ -1862,6 +1836,227 @@ __global__ __launch_bounds__(GKX * GJX) void k_visc_grad_march_xi(GradArgs a)
     march_body<S, false, true, GJX, GKX>(a, bx, by, bz);
 }
 
+// ---- 2D stage in one kernel -------------------------------------------------------------------------
+// A block owns 15 x 15 nodes and does the whole stage for them: both WENO sweeps, both viscous sweeps with
+// their nodal derivatives, the source and the stage update.  Threads 0-255 sweep xi, 256-511 eta, at the
+// same time and through the same code (a half's argument record is uniform per wave); 15 rows of 16
+// interfaces fill 240 of 256 threads.  Periodic cases read ghosts at their image and form T and mu from
+// what they read, so their stages need no ghost fill.
+// A plane of 64^2 to 200^2 nodes leaves most of the chip idle and its time is the chain of its launches:
+// six dependent kernels of 7-12 us per stage, one of 20 us here (64^2 WENO5 58 -> 20 us, 211 x 157 WENO9
+// 74 -> 28).  Large planes are bound by the FP64 pipe and its latency (one block per CU by LDS) and gain
+// from the passes over memory between the kernels: 1000 x 768 283 -> 224 us.
+constexpr int PT = 15;
+struct PlaneArgs {
+    WenoArgs w[2];                // the sweep records of xi and eta (Q in w[0].q)
+    CFields10 met;
+    gcdp T, mu;                   // stored T and mu (not wrap)
+    int ng[2], lo[2], nt[2];      // padded extents, first interior node, tiles (i, j)
+    long st;                      // stride along i
+    int wrap, visc, update;       // update: apply the stage update, else store Q
+    int flat;                     // the z entries of the xi and eta metric rows are zero
+    int iso_hi[2];                // upper face of the direction is an isothermal wall (ViscArgs)
+    double gam_iso;
+    RkArgs rk;
+};
+template <int S>
+constexpr int plane_visc_lds()
+{
+    constexpr int WD = PT + S + 1, RING = PT + 2;
+    return 2 * 5 * PT * PT + 4 * WD * WD + 6 * PT * WD + 9 * RING * RING + 2 * 3 * PT * PT;
+}
+template <int S, bool MIX>
+constexpr int plane_lds()
+{
+    return 2 * weno_lds<S, PT, PT + 1, -1, MIX>() > plane_visc_lds<S>() ? 2 * weno_lds<S, PT, PT + 1, -1, MIX>()
+                                                                       : plane_visc_lds<S>();
+}
+// Viscous terms of a half's direction (CalcViscidFluxesIn{Xi,Eta}DirectionDirectly, src/ZD.c:47-480) at one
+// interface and the node above it.  mb: the ring position of the lower node of the face, ms its step along the
+// direction; own4: midpoint derivatives of u, v, w, T; cr: interpolated cross derivatives of u, v, T.
+template <int DIR, bool FLAT>
+__device__ __forceinline__ void plane_face(const double *MM, const int mb, const int ms, const double own4[4],
+                                           const double cr[3], double F[4])
+{
+    constexpr int NR = (PT + 2) * (PT + 2), B = 1 - DIR;
+    double m[2][10], mu[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int o = mb + h * ms;
+#pragma unroll
+        for (int c = 0; c < 10; c++) m[h][c] = 0.0;
+        m[h][0] = MM[o]; m[h][1] = MM[NR + o]; m[h][3] = MM[2 * NR + o]; m[h][4] = MM[3 * NR + o];
+        m[h][9] = MM[4 * NR + o];
+        mu[h] = MM[5 * NR + o];
+        if constexpr (!FLAT) { m[h][2] = MM[7 * NR + o]; m[h][5] = MM[8 * NR + o]; }
+    }
+    double d[12];
+#pragma unroll
+    for (int q = 0; q < 12; q++) d[q] = 0.0;
+    d[0 * 3 + DIR] = own4[0]; d[1 * 3 + DIR] = own4[1]; d[2 * 3 + DIR] = own4[2]; d[9 + DIR] = own4[3];
+    d[0 * 3 + B] = cr[0]; d[1 * 3 + B] = cr[1]; d[9 + B] = cr[2];
+    face_flux_generic<DIR>(d, m[0], m[1], mu[0], mu[1], F);
+}
+template <int S, int DIR>
+__device__ __forceinline__ void plane_visc(const PlaneArgs &z, const int t, const int d0, const double *UV,
+                                           const double *DER, const double *MM, double *QV)
+{
+    constexpr int G = (S + 1) / 2, WD = PT + 2 * G, RN = WD * WD, ND = PT * WD, NR = (PT + 2) * (PT + 2);
+    const WenoArgs &a = z.w[DIR];
+    const Consts &k = a.k;
+    const int ta = min(t / (PT + 1), PT - 1), di = t % (PT + 1);
+    // region position of the first stencil node and its step; derivative arrays of this direction (own) and
+    // the other (cross): [u, v, T][...]
+    const int rb = (DIR == 0) ? di * WD + ta + G : (ta + G) * WD + di, rs = (DIR == 0) ? WD : 1;
+    const double *own = DER + DIR * 3 * ND, *crs = DER + (1 - DIR) * 3 * ND;
+    const int cb = (DIR == 0) ? di * PT + ta : ta * WD + di, cs = (DIR == 0) ? PT : 1;
+    double own4[4] = {0.0, 0.0, 0.0, 0.0}, cr[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int l = 0; l <= S; l++) {
+        const double cm = k.zd_mid[l], ci = k.zd_int[l];
+#pragma unroll
+        for (int f = 0; f < 4; f++) own4[f] += cm * UV[f * RN + rb + l * rs];
+#pragma unroll
+        for (int f = 0; f < 3; f++) cr[f] += ci * crs[f * ND + cb + l * cs];
+    }
+    const int mb = (DIR == 0) ? di * (PT + 2) + ta + 1 : (ta + 1) * (PT + 2) + di, ms = (DIR == 0) ? PT + 2 : 1;
+    double F[4], nxt[4];
+    if (z.flat) plane_face<DIR, true>(MM, mb, ms, own4, cr, F);
+    else plane_face<DIR, false>(MM, mb, ms, own4, cr, F);
+#pragma unroll
+    for (int m = 0; m < 4; m++) nxt[m] = next_lane(F[m]);
+    if (di < PT && t < PT * (PT + 1)) {
+        const int p = rb + G * rs;
+        double dF[4], g[9], m[10];
+#pragma unroll
+        for (int q = 0; q < 4; q++) dF[q] = nxt[q] - F[q];
+#pragma unroll
+        for (int q = 0; q < 9; q++) g[q] = 0.0;
+        const int po = (DIR == 0) ? di * WD + ta + G : (ta + G) * PT + di;   // the node in the own-direction arrays
+        const int pc = cb + G * cs;                                          // and in the cross-direction ones
+        g[0 * 3 + DIR] = own[po]; g[1 * 3 + DIR] = own[ND + po];
+        g[0 * 3 + 1 - DIR] = crs[pc]; g[1 * 3 + 1 - DIR] = crs[ND + pc];
+        const int o = mb + ms;
+#pragma unroll
+        for (int q = 0; q < 10; q++) m[q] = 0.0;
+        m[0] = MM[o]; m[1] = MM[NR + o]; m[3] = MM[2 * NR + o]; m[4] = MM[3 * NR + o]; m[9] = MM[4 * NR + o];
+        if (!z.flat) { m[2] = MM[7 * NR + o]; m[5] = MM[8 * NR + o]; }
+        const double prod = node_prod_generic<DIR>(g, m, MM[5 * NR + o]);
+        const double work = UV[p] * dF[0] + UV[RN + p] * dF[1] + UV[2 * RN + p] * dF[2];
+        const double gh = (z.iso_hi[DIR] && d0 + di == a.nD - 1) ? z.gam_iso : k.gam_heat;
+        const int node = (DIR == 0) ? di * PT + ta : ta * PT + di;
+        QV[node] = dF[0];
+        QV[PT * PT + node] = dF[1];
+        QV[2 * PT * PT + node] = (gh * dF[3] + k.psi * (work + prod));
+    }
+}
+template <int S, bool MIX>
+__device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, double *lds)
+{
+    constexpr int G = (S + 1) / 2, WD = PT + 2 * G, RN = WD * WD, ND = PT * WD, RING = PT + 2, NR = RING * RING;
+    constexpr int NN = PT * PT, WL = weno_lds<S, PT, PT + 1, -1, MIX>();
+    const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), t = threadIdx.x & 255;
+    const int ti = tile / z.nt[1], tj = tile - ti * z.nt[1];
+    const int ta = min(t / (PT + 1), PT - 1), di = t % (PT + 1);
+    double keep[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    weno_body<S, PT, PT + 1, -1, MIX, true, 256>(z.w[half], half ? ti : tj, 0, half ? tj : ti, lds + half * WL, keep);
+    __syncthreads();
+    double *const QW = lds, *const UV = QW + 2 * 5 * NN, *const DER = UV + 4 * RN, *const MM = DER + 6 * ND;
+    double *const QV = MM + 9 * NR;
+    if (di < PT && t < PT * (PT + 1)) {
+        const int node = half ? ta * PT + di : di * PT + ta;
+#pragma unroll
+        for (int m = 0; m < 5; m++) QW[(half * 5 + m) * NN + node] = keep[m];
+    }
+    const Consts &k = z.w[0].k;
+    const int i0 = z.lo[0] + ti * PT, j0 = z.lo[1] + tj * PT;    // padded index of the tile's first node
+    if (z.visc) {
+        const WenoArgs &wx = z.w[0], &wy = z.w[1];
+        for (int idx = threadIdx.x; idx < RN; idx += 512) {
+            const int li = idx / WD, lj = idx - li * WD;
+            const int i = min(i0 - G + li, z.ng[0] - 1), j = min(j0 - G + lj, z.ng[1] - 1);
+            const long n = (long)i * z.st + j;
+            const bool ring = li >= G - 1 && li <= G + PT && lj >= G - 1 && lj <= G + PT;
+            long ns = n;
+            if (z.wrap) {
+                ns += (long)(i < wx.oD ? wx.nD : (i >= wx.oD + wx.nD ? -wx.nD : 0)) * z.st;
+                ns += (j < wy.oD ? wy.nD : (j >= wy.oD + wy.nD ? -wy.nD : 0));
+            }
+            const double u = wx.pr.f[1][ns], v = wx.pr.f[2][ns], w = wx.pr.f[3][ns];
+            double T, mu = 0.0;
+            if (z.wrap) {
+                const double rho = wx.pr.f[0][ns];
+                node_tmu(k, pressure(k, rho, u, v, w, wx.pr.f[4][ns]), rho, T, mu);
+            } else {
+                T = z.T[n];
+                if (ring) mu = z.mu[n];
+            }
+            UV[idx] = u; UV[RN + idx] = v; UV[2 * RN + idx] = w; UV[3 * RN + idx] = T;
+            if (ring) {
+                double *const M = MM + (li - G + 1) * RING + lj - G + 1;
+                M[0] = z.met.f[0][n]; M[NR] = z.met.f[1][n]; M[2 * NR] = z.met.f[3][n]; M[3 * NR] = z.met.f[4][n];
+                M[4 * NR] = z.met.f[9][n];
+                M[5 * NR] = mu;
+                if (!z.flat) { M[7 * NR] = z.met.f[2][n]; M[8 * NR] = z.met.f[5][n]; }
+            }
+        }
+        __syncthreads();
+        // nodal derivatives of u, v, T: the half's direction at the nodes interior to it along that
+        // direction, over the whole region across it
+        for (int idx = t; idx < ND; idx += 256) {
+            const int rb = half ? (idx / PT) * WD + idx % PT : idx, rs = half ? 1 : WD;
+            double d[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+            for (int l = 0; l <= S + 1; l++) {
+                const double c = k.zd_der[l];
+                d[0] += c * UV[rb + l * rs];
+                d[1] += c * UV[RN + rb + l * rs];
+                d[2] += c * UV[3 * RN + rb + l * rs];
+            }
+#pragma unroll
+            for (int f = 0; f < 3; f++) DER[(half * 3 + f) * ND + idx] = d[f];
+        }
+        __syncthreads();
+        if (half == 0) plane_visc<S, 0>(z, t, ti * PT, UV, DER, MM, QV);
+        else plane_visc<S, 1>(z, t, tj * PT, UV, DER, MM, QV + 3 * NN);
+    }
+    __syncthreads();
+    double cflv = 0.0;
+    if (threadIdx.x < NN) {
+        const int node = threadIdx.x, i = i0 + node / PT, j = j0 + node % PT;
+        if (i < z.w[0].oD + z.w[0].nD && j < z.w[1].oD + z.w[1].nD) {
+            const long n = (long)i * z.st + j;
+            double q[5];
+#pragma unroll
+            for (int m = 0; m < 5; m++) q[m] = QW[m * NN + node] + QW[(5 + m) * NN + node];
+            if (z.visc) {
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    q[1] = q[1] + k.psi * QV[(h * 3 + 0) * NN + node];
+                    q[2] = q[2] + k.psi * QV[(h * 3 + 1) * NN + node];
+                    q[4] = q[4] + QV[(h * 3 + 2) * NN + node];
+                }
+            }
+            if (z.update) {
+                double m9[9];
+#pragma unroll
+                for (int c = 0; c < 9; c++) m9[c] = z.rk.cfl_red ? z.met.f[c][n] : 0.0;
+                rk_point(z.rk, n, z.met.f[9][n], q, m9, &cflv);
+            } else {
+#pragma unroll
+                for (int m = 0; m < 5; m++) z.w[0].q.f[m][n] = q[m];
+            }
+        }
+    }
+    if (z.update && z.rk.cfl_red) wave_max_to(z.rk.cfl_red, cflv);
+}
+template <int S, bool MIX>
+__global__ __launch_bounds__(512) void k_plane(PlaneArgs z)
+{
+    __shared__ double lds[plane_lds<S, MIX>()];
+    plane_body<S, MIX>(z, blockIdx.x, lds);
+}
+
 // ---- batched launches ----------------------------------------------------------------------------
 // One launch runs a kernel class over many independent cases.  The launch's work list holds one
 // descriptor per block of every case: (case, tile x, tile y, tile z), or (case, block, 0, 0) for
@@ -1959,16 +2154,6 @@ __global__ __launch_bounds__(256) void k_carry_batch(BATCH_PARAMS(CarryArgs))
         carry_body(a.from, a.to, a.gm, (long)w.y * 256 + threadIdx.x);
     });
 }
-template <bool P>
-__global__ __launch_bounds__(256) void k_grad2d_batch(BATCH_PARAMS(GradArgs))
-{
-    batch_walk<P>(total, [&](const int b) {
-        const int4 w = rec(work, b);
-        const GradArgs &a = rec(A, w.x);
-        grad_body(a.pr, a.T, a.gr, a.gm, a.k, (long)w.y * 256 + threadIdx.x);
-    });
-}
-
 template <int S, bool P, bool TG>
 __global__ __launch_bounds__(GK * GJ) void k_march_batch(BATCH_PARAMS(GradArgs))
 {
@@ -2030,6 +2215,15 @@ __global__ __launch_bounds__(256, (MIX ? 1 : ETA_WAVES)) void k_eta_batch(BATCH_
     batch_walk<P>(total, [&](const int b) {
         const int4 w = rec(work, b);
         eta_body<MIX>(rec(A, w.x), w.y, w.z, w.w, lds);
+    });
+}
+template <int S, bool MIX, bool P>
+__global__ __launch_bounds__(512) void k_plane_batch(BATCH_PARAMS(PlaneArgs))
+{
+    __shared__ double lds[plane_lds<S, MIX>()];
+    batch_walk<P>(total, [&](const int b) {
+        const int4 w = rec(work, b);
+        plane_body<S, MIX>(rec(A, w.x), w.y, lds);
     });
 }
 template <bool P>
@@ -2383,6 +2577,7 @@ static int set_err(int code, const char *fmt, ...)
                            __FILE__, __LINE__);                                               \
     } while (0)
 
+// KT_ZETA also times k_plane, the whole 2D stage
 enum { KT_GHOST, KT_VALUES, KT_WENO0, KT_WENO1, KT_WENO2, KT_GRAD, KT_VISC0, KT_VISC1, KT_VISC2, KT_RK, KT_REDUCE, KT_METRIC, KT_FACES, KT_ZETA, KT_GRADXI, KT_ETA };
 static const char *g_knames[SHX_NUM_KERNELS] = {
     "ghost_periodic", "ghost_values", "weno_xi", "weno_eta", "weno_zeta",
@@ -2439,6 +2634,7 @@ struct shx_case {
     int faces;             // number of non-periodic faces
     int needs_bs;          // some face is SHX_BC_MANUFACTURED
     int diag;              // 3D metric is diagonal (only xi_x, eta_y, zeta_z and J non-zero)
+    int flat;              // 2D: xi_z and eta_z are zero
     int wtile[3];          // WENO tile variant per direction (set by shx_tune)
     unsigned long long *d_red;
     int *d_cnt;
@@ -2934,6 +3130,7 @@ extern "C" int shx_build_metric(shx_case *c, const double *xe, const double *ye,
     hipFree(dx); hipFree(dy); hipFree(dz);
     c->has_metric = 1;
     c->diag = (gm.dims == 3 && (c->d.quirks & SHX_QUIRK_METRIC_DIAG3D)) ? 1 : 0;
+    c->flat = (gm.dims == 2) ? 1 : 0;
     return SHX_OK;
 }
 
@@ -2950,6 +3147,11 @@ extern "C" int shx_upload_metric(shx_case *c, const double *const met[10])
         for (long n = 0; n < c->gm.ntot; n++)
             if (met[offd[s]][n] != 0.0) { diag = 0; break; }
     c->diag = diag;
+    int flat = (c->gm.dims == 2);
+    for (int s = 2; s < 6 && flat; s += 3)
+        for (long n = 0; n < c->gm.ntot; n++)
+            if (met[s][n] != 0.0) { flat = 0; break; }
+    c->flat = flat;
     return SHX_OK;
 }
 
@@ -3222,36 +3424,76 @@ static dim3 march_grid(const Geom &gm, const bool xi, const int planes)
 {
     return dim3(nblk(gm.ng[2], xi ? GKX : GK), nblk(gm.ng[1], xi ? GJX : GJ), nblk(gm.ng[0], planes));
 }
-// Nodal derivatives of the viscous terms (3D: the march; 2D: pointwise).  xi: the march also adds
-// the viscous xi terms to Q (fuse_xi cases, after the WENO xi sweep).
+// Nodal derivatives of the viscous terms.  xi: the march also adds the viscous xi terms to Q (fuse_xi
+// cases, after the WENO xi sweep).
 static int grad_march(shx_case *c, double *const *pr, const bool xi)
 {
     const Geom &gm = c->gm;
     int rc = tbeg(c, xi ? KT_GRADXI : KT_GRAD);
     if (rc) return rc;
-    if (gm.dims == 3) {
-        const int planes = march_planes(c, march_columns(gm, xi));
-        GradArgs ga = grad_args(c, pr, xi, planes);
-        const void *fn = xi ? (const void *)&k_visc_grad_march_xi<5> : march_kernel(c->d.space_order, ga.tgrad, false);
-        const dim3 grid = flat_grid(march_grid(gm, xi, planes), ga.tg, 0);
-        void *args[] = {&ga};
-        HIPCHK(hipLaunchKernel(fn, grid, dim3(xi ? GKX * GJX : GK * GJ), args, 0, c->stream));
-    } else {
-        CFields5 cp;
-        Fields12 gf;
-        for (int m = 0; m < 5; m++) cp.f[m] = pr[m];
-        for (int m = 0; m < 12; m++) gf.f[m] = c->grad[m];
-        k_visc_grad<<<nblk(gm.ntot, 256), 256, 0, c->stream>>>(cp, c->T, gf, gm, c->k);
-    }
+    const int planes = march_planes(c, march_columns(gm, xi));
+    GradArgs ga = grad_args(c, pr, xi, planes);
+    const void *fn = xi ? (const void *)&k_visc_grad_march_xi<5> : march_kernel(c->d.space_order, ga.tgrad, false);
+    const dim3 grid = flat_grid(march_grid(gm, xi, planes), ga.tg, 0);
+    void *args[] = {&ga};
+    HIPCHK(hipLaunchKernel(fn, grid, dim3(xi ? GKX * GJX : GK * GJ), args, 0, c->stream));
     LAUNCH_CHECK();
     return tend(c);
 }
 static int eta_sweep(shx_case *c, double *const *pr);
+
+// ---- 2D stages: one k_plane launch (after the ghost fill and the face writers, where the case has them)
+// the stages of an all-periodic case read ghosts at their image; stored p and c need the fill's pass
+static bool plane_wraps(const shx_case *c) { return c->gm.dims == 2 && !c->faces && !c->pc; }
+static Pick plane_pick(const shx_case *c)
+{
+    const bool mix = (c->d.precision == SHX_MIXED);
+#define SHX_PLANE_PICK(S, M) \
+    Pick{(const void *)&k_plane<S, M>, (const void *)&k_plane_batch<S, M, false>, (const void *)&k_plane_batch<S, M, true>, PT, PT}
+    if (c->d.space_order == 5) return mix ? SHX_PLANE_PICK(5, true) : SHX_PLANE_PICK(5, false);
+    return mix ? SHX_PLANE_PICK(9, true) : SHX_PLANE_PICK(9, false);
+#undef SHX_PLANE_PICK
+}
+// wrap: the stage input's ghosts are not filled; rk: the stage update (null: Q is stored)
+static PlaneArgs plane_args(const shx_case *c, double *const *pr, const RkArgs *rk, const bool wrap)
+{
+    const Geom &gm = c->gm;
+    PlaneArgs z;
+    memset(&z, 0, sizeof z);
+    for (int d = 0; d < 2; d++) {
+        z.w[d] = weno_args(c, pr, d, 1);
+        z.w[d].alignA = 0;
+        z.w[d].wrap = wrap ? 1 : 0;
+        z.ng[d] = gm.ng[d]; z.lo[d] = gm.lo[d];
+        z.nt[d] = (int)nblk(gm.n[d], PT);
+        z.iso_hi[d] = (c->d.bc[2 * d + 1] == SHX_BC_WALL_ISOTHERMAL) ? 1 : 0;
+    }
+    for (int m = 0; m < 10; m++) z.met.f[m] = c->met[m];
+    z.T = c->T; z.mu = c->mu;
+    z.st = gm.st[0];
+    z.wrap = wrap ? 1 : 0;
+    z.visc = c->d.inviscid ? 0 : 1;
+    z.update = rk ? 1 : 0;
+    z.flat = c->flat;
+    z.gam_iso = iso_factor(c);
+    if (rk) z.rk = *rk;
+    return z;
+}
+static int plane_stage(shx_case *c, double *const *pr, const RkArgs *rk, const bool wrap)
+{
+    PlaneArgs z = plane_args(c, pr, rk, wrap);
+    int rc = tbeg(c, KT_ZETA);
+    if (rc) return rc;
+    if ((rc = launch_pick(plane_pick(c).single, dim3(z.nt[0] * z.nt[1]), 512, &z, c->stream))) return rc;
+    return tend(c);
+}
 // rk: when given, the last viscous sweep applies this stage update instead of storing Q
 static int stage_fluxes(shx_case *c, double *const *pr, const RkArgs *rk, double tau)
 {
     const Geom &gm = c->gm;
     int rc;
+    // a caller of the residual alone finds the ghosts of its state filled, as always
+    if (rk && plane_wraps(c)) return plane_stage(c, pr, rk, true);
     if (c->d.inviscid && !c->pc) {
         if ((rc = ghost_fill(c, pr, 5))) return rc;
     } else {
@@ -3266,12 +3508,9 @@ static int stage_fluxes(shx_case *c, double *const *pr, const RkArgs *rk, double
         if ((rc = tend(c))) return rc;
     }
     const bool fx = fuse_xi(c);
-    if (!c->d.inviscid) {
-        if ((rc = face_fill(c, pr, tau))) return rc;
-        if (!fx && (rc = grad_march(c, pr, false))) return rc;
-    } else if ((rc = face_fill(c, pr, tau))) {
-        return rc;
-    }
+    if ((rc = face_fill(c, pr, tau))) return rc;
+    if (gm.dims == 2) return plane_stage(c, pr, rk, false);
+    if (!c->d.inviscid && !fx && (rc = grad_march(c, pr, false))) return rc;
     // Q accumulates the WENO divergences, then the viscous terms; with the fused zeta direction
     // the order is WENO xi, eta, viscous xi, eta, then WENO zeta and viscous zeta together.  With
     // the viscous xi direction in the derivative march, the march runs after the WENO xi and eta
@@ -3312,7 +3551,6 @@ static Pick visc_pick_s(int dir, bool coalesce, bool diag)
     constexpr int TDN = (S == 5) ? 16 : 32;
     constexpr int TDG = (S == 5) ? 12 : 8;
     if (coalesce) {
-        if (dir == 1) return visc_pick_t<S, 1, 4, 48, false>();       // 2D eta sweep
         if (diag) return visc_pick_t<S, 2, 4, 64, true>();
         return visc_pick_t<S, 2, 4, 48, false>();
     }
@@ -3362,7 +3600,6 @@ static ViscArgs visc_args(const shx_case *c, double *const *pr, int dir, const R
     a.ngA = gm.ng[A];
     a.coalesce_d = (a.sD == 1);
     a.alignA = (a.sA == 1);
-    a.three = (gm.dims == 3);
     a.bug = (dir == 2 && (c->d.quirks & SHX_QUIRK_ZETA_VISC_J)) ? 1 : 0;
     a.k = c->k;
     a.iso_hi = (c->d.bc[2 * dir + 1] == SHX_BC_WALL_ISOTHERMAL) ? 1 : 0;
@@ -3513,10 +3750,11 @@ static int step_stage(shx_case *c, int s, double tau, int flags)
         if (flags & STEP_NAN) { rk.nan_cnt = c->d_nan; rk.nanP = c->P; }
         if (flags & STEP_CFL) rk.cfl_red = c->d_red;
     }
-    // viscous stages apply the update in their last sweep; inviscid ones in k_rk_update
-    if ((rc = stage_fluxes(c, c->prim[c->st_in], c->d.inviscid ? nullptr : &rk, tau))) return rc;
+    // viscous and 2D stages apply the update in their last kernel; 3D inviscid ones in k_rk_update
+    const bool sep = c->d.inviscid && c->gm.dims == 3;
+    if ((rc = stage_fluxes(c, c->prim[c->st_in], sep ? nullptr : &rk, tau))) return rc;
     if ((rc = carry_ghosts(c, c->prim[c->st_in], c->prim[c->st_out]))) return rc;
-    if (c->d.inviscid && (rc = rk_update(c, rk))) return rc;
+    if (sep && (rc = rk_update(c, rk))) return rc;
     c->st_in = c->st_out;
     c->st_out = (c->st_out == c->st_bx) ? c->st_by : c->st_bx;
     return SHX_OK;
@@ -4014,18 +4252,24 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                 if (any) batch_add(b, (const void *)&k_face_save_batch<false>, (const void *)&k_face_save_batch<true>, 256, BK_GHOST, recs, sizeof(BcArgs), grids);
             }
         }
+        // 2D cases that read ghosts at their image need none filled, but the state keeps those of the
+        // step's start, as it always has in a batch
+        auto fills = [&](const shx_case *c) { return s == 0 || !plane_wraps(c); };
         if (c0->d.inviscid) {   // periodic ghost fill of the stage input
             std::vector<char> recs;
             std::vector<dim3> grids;
+            long any = 0;
             for (int i = 0; i < nc; i++) {
                 GhostArgs a;
                 memset(&a, 0, sizeof a);
                 for (int m = 0; m < 5; m++) a.f.f[m] = in[i][m];
                 a.nf = 5; a.gm = g[i]->gm;
                 put(recs, a);
-                grids.push_back(dim3(nblk(g[i]->gm.ntot, 256)));
+                const long nodes = fills(g[i]) ? g[i]->gm.ntot : 0;
+                grids.push_back(dim3(nblk(nodes, 256)));
+                any += nodes;
             }
-            batch_add(b, (const void *)&k_ghost_batch<false>, (const void *)&k_ghost_batch<true>, 256, BK_GHOST, recs, sizeof(GhostArgs), grids);
+            if (any) batch_add(b, (const void *)&k_ghost_batch<false>, (const void *)&k_ghost_batch<true>, 256, BK_GHOST, recs, sizeof(GhostArgs), grids);
         }
         // face writers, one launch per face in the reference's order (after CalcValues when viscous);
         // a case contributes no blocks to the launch of a periodic face
@@ -4067,7 +4311,7 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
             // periodic ghost fill of the stage input with CalcValues
             std::vector<char> recs, grecs;
             std::vector<dim3> grids, ggrids;
-            long cols = 0;
+            long cols = 0, any = 0;
             for (int i = 0; i < nc; i++) cols += march_columns(g[i]->gm, false);
             for (int i = 0; i < nc; i++) {
                 shx_case *c = g[i];
@@ -4076,26 +4320,35 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                 for (int m = 0; m < 5; m++) a.pr.f[m] = in[i][m];
                 a.T = c->T; a.mu = c->mu; a.P = c->P; a.C = c->C; a.gm = c->gm; a.k = c->k;
                 put(recs, a);
-                grids.push_back(dim3(nblk(c->gm.ntot, 256)));
-                const int planes = (dims == 3) ? march_planes(c, cols) : 0;
+                const long nodes = fills(c) ? c->gm.ntot : 0;
+                grids.push_back(dim3(nblk(nodes, 256)));
+                any += nodes;
+                if (dims == 2) continue;
+                const int planes = march_planes(c, cols);
                 put(grecs, grad_args(c, in[i], false, planes));
-                if (dims == 3) ggrids.push_back(march_grid(c->gm, false, planes));
-                else ggrids.push_back(dim3(nblk(c->gm.ntot, 256)));
+                ggrids.push_back(march_grid(c->gm, false, planes));
             }
-            batch_add(b, (const void *)&k_ghost_values_batch<false>, (const void *)&k_ghost_values_batch<true>, 256, BK_VALUES, recs, sizeof(GhostValuesArgs), grids);
+            if (any) batch_add(b, (const void *)&k_ghost_values_batch<false>, (const void *)&k_ghost_values_batch<true>, 256, BK_VALUES, recs, sizeof(GhostValuesArgs), grids);
             add_faces();
-            if (dims == 3) {
-                // the march with the viscous xi terms follows the WENO xi sweep (below)
-                if (!fuse_xi(c0))
-                    batch_add(b, march_kernel(S, !c0->diag, true, false), march_kernel(S, !c0->diag, true, true), GK * GJ,
-                              BK_GRAD, grecs, sizeof(GradArgs), ggrids, ORDER_NODES);
-            } else {
-                batch_add(b, (const void *)&k_grad2d_batch<false>, (const void *)&k_grad2d_batch<true>, 256, BK_GRAD, grecs, sizeof(GradArgs), ggrids);
+            // the march with the viscous xi terms follows the WENO xi sweep (below)
+            if (dims == 3 && !fuse_xi(c0))
+                batch_add(b, march_kernel(S, !c0->diag, true, false), march_kernel(S, !c0->diag, true, true), GK * GJ,
+                          BK_GRAD, grecs, sizeof(GradArgs), ggrids, ORDER_NODES);
+        }
+        if (dims == 2) {
+            const Pick p = plane_pick(c0);
+            std::vector<char> recs;
+            std::vector<dim3> grids;
+            for (int i = 0; i < nc; i++) {
+                const PlaneArgs z = plane_args(g[i], in[i], &rk[i], plane_wraps(g[i]));
+                put(recs, z);
+                grids.push_back(dim3(z.nt[0] * z.nt[1]));
             }
+            batch_add(b, p.batch, p.batchp, 512, BK_WENO, recs, sizeof(PlaneArgs), grids, ORDER_NODES);
         }
         // the same sweep sequence as stage_fluxes (fused eta and zeta directions where they apply)
         const bool fz = fuse_zeta(c0), fx = fuse_xi(c0), fe = fuse_eta(c0);
-        const int nsep = fz ? dims - 1 : dims;
+        const int nsep = dims == 2 ? 0 : (fz ? dims - 1 : dims);
         for (int dir = 0; dir < nsep; dir++) {
             if (fe && dir == 1) continue;
             const Pick p = weno_pick(c0, dir);
@@ -4157,6 +4410,8 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                 grids.push_back(sweep_grid(z.w.nA, z.w.oA, z.w.alignA, z.w.nB, z.w.nD, p));
             }
             batch_add(b, p.batch, p.batchp, p.TA * p.TDI, BK_VISC, zrecs, sizeof(ZetaArgs), grids, ORDER_SWEEP);
+        } else if (dims == 2) {
+            // done
         } else if (!c0->d.inviscid) {
             for (int dir = 0; dir < dims; dir++) {
                 const Pick p = visc_pick(c0, dir);
@@ -4536,6 +4791,11 @@ extern "C" int shx_tune(shx_case *c, int reps, int choice[3])
     if (rc) return rc;
     if (reps <= 0) reps = 3;
     double *const *pr = c->prim[c->cur];
+    if (c->gm.dims == 2) {            // 2D stages run on k_plane's tile
+        if (choice)
+            for (int d = 0; d < 3; d++) choice[d] = c->wtile[d];
+        return SHX_OK;
+    }
     if ((rc = ghost_fill(c, pr, 5))) return rc;
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
@@ -4673,7 +4933,7 @@ static int sync_ghosts(shx_case *c)
     CFields5 a;
     Fields5 b;
     for (int m = 0; m < 5; m++) { a.f[m] = c->prim[c->last_in][m]; b.f[m] = c->prim[c->cur][m]; }
-    k_copy_ghosts<<<nblk(c->gm.ntot, 256), 256, 0, c->stream>>>(a, b, c->gm);
+    k_copy_ghosts<<<nblk(c->gm.ntot, 256), 256, 0, c->stream>>>(a, b, c->gm, (c->gm.dims == 2 && !c->faces) ? 1 : 0);
     LAUNCH_CHECK();
     c->last_in = -1;
     return SHX_OK;
