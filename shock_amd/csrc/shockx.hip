@@ -1054,58 +1054,47 @@ struct ViscArgs {
     Consts k;
 };
 
-// fac_{i,k,b} (CreateViscidMetric, src/Functions.c:6245-6386) from row r (= b) and row a (= D).
-template <int I, int K>
-__device__ __forceinline__ double fac_ikb(const double J, const double r0, const double r1, const double r2,
-                                          const double a0, const double a1, const double a2)
-{
-    if constexpr (I == 0 && K == 0) return J * (4.0 / 3.0 * r0 * a0 + r1 * a1 + r2 * a2);
-    if constexpr (I == 0 && K == 1) return J * (-2.0 / 3.0 * r1 * a0 + r0 * a1);
-    if constexpr (I == 0 && K == 2) return J * (-2.0 / 3.0 * r2 * a0 + r0 * a2);
-    if constexpr (I == 1 && K == 0) return J * (r1 * a0 - 2.0 / 3.0 * r0 * a1);
-    if constexpr (I == 1 && K == 1) return J * (r0 * a0 + 4.0 / 3.0 * r1 * a1 + r2 * a2);
-    if constexpr (I == 1 && K == 2) return J * (-2.0 / 3.0 * r2 * a1 + r1 * a2);
-    if constexpr (I == 2 && K == 0) return J * (r2 * a0 - 2.0 / 3.0 * r0 * a2);
-    if constexpr (I == 2 && K == 1) return J * (r2 * a1 - 2.0 / 3.0 * r1 * a2);
-    if constexpr (I == 2 && K == 2) return J * (r0 * a0 + r1 * a1 + 4.0 / 3.0 * r2 * a2);
-    return J * (r0 * a0 + r1 * a1 + r2 * a2);   // heat flux (I == 3)
-}
-
 template <int DIR> struct Others { static constexpr int b1 = (DIR == 0) ? 1 : 0; static constexpr int b2 = (DIR == 2) ? 1 : 2; };
 
-// face flux (momentum x,y,z and heat) from slot values d[12] (slot k*3+b, T slots 9+b) and the
-// metric/mu of the face's two nodes (generic metric)
+// Viscous flux of one node's metric along row a = DIR, without J and mu: the reference's factors
+// fac_{i,k,b} (CreateViscidMetric, src/Functions.c:6245-6386) contracted with the slot values d (velocity
+// derivative d[3k+b], T at 9+b).  fac is the Newtonian stress in metric rows, so the sum over k and b is the
+// stress of the Cartesian velocity gradient g_kj = sum_b d_kb r_bj along a:
+//   t_i = sum_j (g_ij + g_ji) a_j - 2/3 a_i div g,   t_3 = grad T . a.
+// 57 operations where evaluating the 30 factors takes 180.
+template <int DIR>
+__device__ __forceinline__ void stress_along(const double d[12], const double m[10], double t[4])
+{
+    double g[3][3];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) g[k][j] = d[3 * k] * m[j] + d[3 * k + 1] * m[3 + j] + d[3 * k + 2] * m[6 + j];
+    const double *a = m + 3 * DIR;
+    const double div = g[0][0] + g[1][1] + g[2][2];
+    const double p = (2. / 3.) * div;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        double acc = -(p * a[i]);
+#pragma unroll
+        for (int j = 0; j < 3; j++) acc += (g[i][j] + g[j][i]) * a[j];
+        t[i] = acc;
+    }
+    t[3] = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) t[3] += (d[9] * m[j] + d[10] * m[3 + j] + d[11] * m[6 + j]) * a[j];
+}
+// face flux (momentum x,y,z and heat): the reference's mean of mu fac over the face's two nodes
 template <int DIR>
 __device__ __forceinline__ void face_flux_generic(const double d[12], const double m0[10], const double m1[10],
                                                   const double mu0, const double mu1, double F[4])
 {
-    const double J0 = m0[9], J1 = m1[9];
-    const double a00 = m0[3 * DIR], a01 = m0[3 * DIR + 1], a02 = m0[3 * DIR + 2];
-    const double a10 = m1[3 * DIR], a11 = m1[3 * DIR + 1], a12 = m1[3 * DIR + 2];
+    double t0[4], t1[4];
+    stress_along<DIR>(d, m0, t0);
+    stress_along<DIR>(d, m1, t1);
+    const double w0 = 0.5 * (mu0 * m0[9]), w1 = 0.5 * (mu1 * m1[9]);
 #pragma unroll
-    for (int i = 0; i < 3; i++) F[i] = 0.0;
-    F[3] = 0.0;
-#define SHX_FACE_TERM(I, K, B)                                                                    \
-    {                                                                                             \
-        const double f0 = fac_ikb<I, K>(J0, m0[3 * B], m0[3 * B + 1], m0[3 * B + 2], a00, a01, a02); \
-        const double f1 = fac_ikb<I, K>(J1, m1[3 * B], m1[3 * B + 1], m1[3 * B + 2], a10, a11, a12); \
-        F[I] += d[K * 3 + B] * (0.5 * (mu0 * f0 + mu1 * f1));                                     \
-    }
-#define SHX_FACE_ROW(I) \
-    SHX_FACE_TERM(I, 0, 0) SHX_FACE_TERM(I, 0, 1) SHX_FACE_TERM(I, 0, 2) \
-    SHX_FACE_TERM(I, 1, 0) SHX_FACE_TERM(I, 1, 1) SHX_FACE_TERM(I, 1, 2) \
-    SHX_FACE_TERM(I, 2, 0) SHX_FACE_TERM(I, 2, 1) SHX_FACE_TERM(I, 2, 2)
-    SHX_FACE_ROW(0)
-    SHX_FACE_ROW(1)
-    SHX_FACE_ROW(2)
-#undef SHX_FACE_ROW
-#undef SHX_FACE_TERM
-#pragma unroll
-    for (int b = 0; b < 3; b++) {
-        const double f0 = fac_ikb<3, 0>(J0, m0[3 * b], m0[3 * b + 1], m0[3 * b + 2], a00, a01, a02);
-        const double f1 = fac_ikb<3, 0>(J1, m1[3 * b], m1[3 * b + 1], m1[3 * b + 2], a10, a11, a12);
-        F[3] += d[9 + b] * (0.5 * (mu0 * f0 + mu1 * f1));
-    }
+    for (int i = 0; i < 4; i++) F[i] = w0 * t0[i] + w1 * t1[i];
 }
 
 // diagonal metric (the reference's 3D metric): node values mD (row D, component D), mb[3]
@@ -1134,24 +1123,14 @@ __device__ __forceinline__ void face_flux_diag(const double d[12], const double 
     F[3] = d[9 + DIR] * KA;
 }
 
-// nodal product term sum_blk g_{blk,D} sum_s g_s mu fac_{blk,s} (src/ZD.c:230-266)
+// nodal product term sum_blk g_{blk,D} sum_s g_s mu fac_{blk,s} (src/ZD.c:230-266); g: nodal velocity
+// derivatives (slots as above)
 template <int DIR>
-__device__ __forceinline__ double node_prod_generic(const double g[9], const double m[10], const double mu)
+__device__ __forceinline__ double node_prod_generic(const double g[12], const double m[10], const double mu)
 {
-    const double J = m[9], a0 = m[3 * DIR], a1 = m[3 * DIR + 1], a2 = m[3 * DIR + 2];
-    double prod = 0.0;
-#define SHX_PROD_TERM(I, K, B) \
-    prod += g[I * 3 + DIR] * g[K * 3 + B] * mu * fac_ikb<I, K>(J, m[3 * B], m[3 * B + 1], m[3 * B + 2], a0, a1, a2);
-#define SHX_PROD_ROW(I) \
-    SHX_PROD_TERM(I, 0, 0) SHX_PROD_TERM(I, 0, 1) SHX_PROD_TERM(I, 0, 2) \
-    SHX_PROD_TERM(I, 1, 0) SHX_PROD_TERM(I, 1, 1) SHX_PROD_TERM(I, 1, 2) \
-    SHX_PROD_TERM(I, 2, 0) SHX_PROD_TERM(I, 2, 1) SHX_PROD_TERM(I, 2, 2)
-    SHX_PROD_ROW(0)
-    SHX_PROD_ROW(1)
-    SHX_PROD_ROW(2)
-#undef SHX_PROD_ROW
-#undef SHX_PROD_TERM
-    return prod;
+    double t[4];
+    stress_along<DIR>(g, m, t);
+    return (mu * m[9]) * (g[DIR] * t[0] + g[3 + DIR] * t[1] + g[6 + DIR] * t[2]);
 }
 
 template <int DIR>
@@ -1179,42 +1158,40 @@ __device__ __forceinline__ double node_prod_diag(const double g[9], const double
 // LDS slots
 enum { VS_U, VS_V, VS_W, VS_T, VS_MU, VS_CR };
 
-// LDS of one viscous sweep block, in doubles: the node window (NVS fields), the face hand-over
-// buffer where a tile row straddles wavefronts, and the zeta-index quirk's line values.  Plus-side
-// face values go from each thread to the previous one (the minus side stays in registers); where a
-// tile row never straddles two wavefronts (TDI divides or is a multiple of the 64-lane wavefront)
-// the hand-over is a lane shuffle.
+// LDS of one viscous sweep block, in doubles: the node window (diagonal metric: 13 fields; general: 12
+// fields, and in their place, once the face's and node's derivatives are in registers, mu and the metric
+// of the tile's nodes and the one below them), and the zeta-index quirk's line values.  Plus-side face
+// values go from each thread to the previous one by a lane move (the minus side stays in registers): a
+// tile row never straddles two wavefronts.
 template <int S, int DIR, int TA, int TDI, bool DIAG>
 constexpr int visc_lds()
 {
-    constexpr int G = (S + 1) / 2, NW = (TDI - 1 + 2 * G) * TA, NT = TA * TDI;
-    constexpr int NC = DIAG ? 4 : 8, NM = DIAG ? 4 : 10;
-    constexpr int NLV = 4 + NC, NP = 2 * G + 1;
-    constexpr bool SHFL = (64 % TDI == 0) || (TDI % 64 == 0);
-    return (VS_CR + NC + NM) * NW + (SHFL ? 0 : 4 * NT) + ((DIR == 2) ? TA * NP * NLV + TA * 2 * NLV : 0);
+    constexpr int G = (S + 1) / 2, NW = (TDI - 1 + 2 * G) * TA;
+    constexpr int NC = DIAG ? 4 : 8, NLV = 4 + NC, NP = 2 * G + 1;
+    constexpr int WIN = DIAG ? (VS_CR + NC + 4) * NW : std::max((4 + NC) * NW, 11 * (TDI + 1) * TA);
+    static_assert(64 % TDI == 0, "tile rows stay in one wavefront");
+    return WIN + ((DIR == 2) ? TA * NP * NLV + TA * 2 * NLV : 0);
 }
 
 // ADD: add add[5] (a fused WENO sweep's contribution of the thread's node) to Q before the
 // viscous terms.  PRE: load the node's Q (and U_n, Q_sum for the stage update) before the window.
-template <int S, int DIR, int TA, int TDI, bool DIAG, bool ADD = false, bool PRE = false>
-__device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const int by, const int bz,
+template <int S, int DIR, int TA, int TDI, bool ADD = false, bool PRE = false>
+__device__ __forceinline__ void visc_diag_body(const ViscArgs &a, const int bx, const int by, const int bz,
                                           double *lds, const double *add = nullptr)
 {
     constexpr int G = (S + 1) / 2;
     constexpr int WD = TDI - 1 + 2 * G;
     constexpr int NW = WD * TA;
     constexpr int NT = TA * TDI;
-    constexpr int NC = DIAG ? 4 : 8;                 // cross-derivative fields
-    constexpr int NM = DIAG ? 4 : 10;                // metric values per node
+    constexpr int NC = 4;                            // cross-derivative fields
+    constexpr int NM = 4;                            // metric values per node
     constexpr int VS_M = VS_CR + NC;
     constexpr int NVS = VS_M + NM;
     constexpr int b1 = Others<DIR>::b1, b2 = Others<DIR>::b2;
     constexpr int NP = 2 * G + 1;                    // line positions used by the zeta-index quirk
     constexpr int NLV = 4 + NC;                      // values per position: u,v,w,T + cross
-    constexpr bool SHFL = (64 % TDI == 0) || (TDI % 64 == 0);
     double *const sm = lds;
-    double *const fo = sm + NVS * NW;
-    double *const line = fo + (SHFL ? 0 : 4 * NT);
+    double *const line = sm + NVS * NW;
     double *const lined = line + TA * NP * NLV;
 
     const int t = threadIdx.x;
@@ -1254,15 +1231,10 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
         sm[VS_MU * NW + o] = a.mu[n];
 #pragma unroll
         for (int c = 0; c < NC; c++) sm[(VS_CR + c) * NW + o] = a.cr[c][n];
-        if constexpr (DIAG) {
-            sm[(VS_M + 0) * NW + o] = a.met.f[0][n];
-            sm[(VS_M + 1) * NW + o] = a.met.f[4][n];
-            sm[(VS_M + 2) * NW + o] = a.met.f[8][n];
-            sm[(VS_M + 3) * NW + o] = a.met.f[9][n];
-        } else {
-#pragma unroll
-            for (int c = 0; c < 10; c++) sm[(VS_M + c) * NW + o] = a.met.f[c][n];
-        }
+        sm[(VS_M + 0) * NW + o] = a.met.f[0][n];
+        sm[(VS_M + 1) * NW + o] = a.met.f[4][n];
+        sm[(VS_M + 2) * NW + o] = a.met.f[8][n];
+        sm[(VS_M + 3) * NW + o] = a.met.f[9][n];
     }
     const bool bug = (DIR == 2) && a.bug;
     if (bug) {
@@ -1322,21 +1294,12 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
 #pragma unroll
             for (int s = 0; s < 12; s++) d[s] = 0.0;
             d[0 * 3 + DIR] = own4[0]; d[1 * 3 + DIR] = own4[1]; d[2 * 3 + DIR] = own4[2]; d[9 + DIR] = own4[3];
-            if constexpr (DIAG) {
-                d[b1 * 3 + b1] = cr[0]; d[DIR * 3 + b1] = cr[1];
-                d[b2 * 3 + b2] = cr[2]; d[DIR * 3 + b2] = cr[3];
-                double g0[3], g1[3];
-                g0[0] = sm[(VS_M + 0) * NW + oc]; g0[1] = sm[(VS_M + 1) * NW + oc]; g0[2] = sm[(VS_M + 2) * NW + oc];
-                g1[0] = sm[(VS_M + 0) * NW + oc + 1]; g1[1] = sm[(VS_M + 1) * NW + oc + 1]; g1[2] = sm[(VS_M + 2) * NW + oc + 1];
-                face_flux_diag<DIR>(d, g0, sm[(VS_M + 3) * NW + oc], g1, sm[(VS_M + 3) * NW + oc + 1], mu0, mu1, F);
-            } else {
-                d[0 * 3 + b1] = cr[0]; d[1 * 3 + b1] = cr[1]; d[2 * 3 + b1] = cr[2]; d[9 + b1] = cr[3];
-                d[0 * 3 + b2] = cr[4]; d[1 * 3 + b2] = cr[5]; d[2 * 3 + b2] = cr[6]; d[9 + b2] = cr[7];
-                double m0[10], m1[10];
-#pragma unroll
-                for (int c = 0; c < 10; c++) { m0[c] = sm[(VS_M + c) * NW + oc]; m1[c] = sm[(VS_M + c) * NW + oc + 1]; }
-                face_flux_generic<DIR>(d, m0, m1, mu0, mu1, F);
-            }
+            d[b1 * 3 + b1] = cr[0]; d[DIR * 3 + b1] = cr[1];
+            d[b2 * 3 + b2] = cr[2]; d[DIR * 3 + b2] = cr[3];
+            double g0[3], g1[3];
+            g0[0] = sm[(VS_M + 0) * NW + oc]; g0[1] = sm[(VS_M + 1) * NW + oc]; g0[2] = sm[(VS_M + 2) * NW + oc];
+            g1[0] = sm[(VS_M + 0) * NW + oc + 1]; g1[1] = sm[(VS_M + 1) * NW + oc + 1]; g1[2] = sm[(VS_M + 2) * NW + oc + 1];
+            face_flux_diag<DIR>(d, g0, sm[(VS_M + 3) * NW + oc], g1, sm[(VS_M + 3) * NW + oc + 1], mu0, mu1, F);
         };
         if (!bug) {
             double own4[4] = {0.0, 0.0, 0.0, 0.0}, cr[NC];
@@ -1365,16 +1328,8 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
         }
     }
     double nxt[4];
-    if constexpr (SHFL) {
 #pragma unroll
-        for (int m = 0; m < 4; m++) nxt[m] = next_lane(out[4 + m]);
-    } else {
-#pragma unroll
-        for (int m = 0; m < 4; m++) fo[m * NT + t] = out[4 + m];
-        __syncthreads();
-#pragma unroll
-        for (int m = 0; m < 4; m++) nxt[m] = (di < TDI - 1) ? fo[m * NT + t + 1] : 0.0;
-    }
+    for (int m = 0; m < 4; m++) nxt[m] = next_lane(out[4 + m]);
 
     double cflv = 0.0;                           // CFL sum of this thread's node (end-of-step check)
     if (di < TDI - 1) {
@@ -1399,22 +1354,10 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
                 g[0 * 3 + DIR] = du; g[1 * 3 + DIR] = dv; g[2 * 3 + DIR] = dw;
             }
             const double mu = sm[VS_MU * NW + p];
-            double prod;
-            if constexpr (DIAG) {
-                g[b1 * 3 + b1] = sm[(VS_CR + 0) * NW + p]; g[DIR * 3 + b1] = sm[(VS_CR + 1) * NW + p];
-                g[b2 * 3 + b2] = sm[(VS_CR + 2) * NW + p]; g[DIR * 3 + b2] = sm[(VS_CR + 3) * NW + p];
-                const double gmv[3] = {sm[(VS_M + 0) * NW + p], sm[(VS_M + 1) * NW + p], sm[(VS_M + 2) * NW + p]};
-                prod = node_prod_diag<DIR>(g, gmv, sm[(VS_M + 3) * NW + p], mu);
-            } else {
-                g[0 * 3 + b1] = sm[(VS_CR + 0) * NW + p]; g[1 * 3 + b1] = sm[(VS_CR + 1) * NW + p];
-                g[2 * 3 + b1] = sm[(VS_CR + 2) * NW + p];
-                g[0 * 3 + b2] = sm[(VS_CR + 4) * NW + p]; g[1 * 3 + b2] = sm[(VS_CR + 5) * NW + p];
-                g[2 * 3 + b2] = sm[(VS_CR + 6) * NW + p];
-                double m[10];
-#pragma unroll
-                for (int c = 0; c < 10; c++) m[c] = sm[(VS_M + c) * NW + p];
-                prod = node_prod_generic<DIR>(g, m, mu);
-            }
+            g[b1 * 3 + b1] = sm[(VS_CR + 0) * NW + p]; g[DIR * 3 + b1] = sm[(VS_CR + 1) * NW + p];
+            g[b2 * 3 + b2] = sm[(VS_CR + 2) * NW + p]; g[DIR * 3 + b2] = sm[(VS_CR + 3) * NW + p];
+            const double gmv[3] = {sm[(VS_M + 0) * NW + p], sm[(VS_M + 1) * NW + p], sm[(VS_M + 2) * NW + p]};
+            const double prod = node_prod_diag<DIR>(g, gmv, sm[(VS_M + 3) * NW + p], mu);
             const double work = sm[VS_U * NW + p] * dF[0] + sm[VS_V * NW + p] * dF[1] + sm[VS_W * NW + p] * dF[2];
 #pragma unroll
             for (int m = 0; m < 5; m++) {
@@ -1429,19 +1372,14 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
                 qv[3] = q0[3] + k.psi * dF[2];
                 const double gh = (a.iso_hi && dn == a.nD - 1) ? a.gam_iso : k.gam_heat;
                 qv[4] = q0[4] + (gh * dF[3] + k.psi * (work + prod));
-                const double J = DIAG ? sm[(VS_M + 3) * NW + p] : sm[(VS_M + 9) * NW + p];
+                const double J = sm[(VS_M + 3) * NW + p];
                 if (a.rk.cfl_red) {
                     // end of step: the node's metric rows for its CFL sum
                     double m9[9];
-                    if constexpr (DIAG) {
 #pragma unroll
-                        for (int c = 0; c < 9; c++) m9[c] = 0.0;
-                        m9[0] = sm[(VS_M + 0) * NW + p]; m9[4] = sm[(VS_M + 1) * NW + p]; m9[8] = sm[(VS_M + 2) * NW + p];
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < 9; c++) m9[c] = sm[(VS_M + c) * NW + p];
-                    }
-                    rk_point<DIAG>(a.rk, n, J, qv, m9, &cflv, PRE ? &pre : nullptr);
+                    for (int c = 0; c < 9; c++) m9[c] = 0.0;
+                    m9[0] = sm[(VS_M + 0) * NW + p]; m9[4] = sm[(VS_M + 1) * NW + p]; m9[8] = sm[(VS_M + 2) * NW + p];
+                    rk_point<true>(a.rk, n, J, qv, m9, &cflv, PRE ? &pre : nullptr);
                 } else {
                     rk_point(a.rk, n, J, qv, nullptr, nullptr, PRE ? &pre : nullptr);
                 }
@@ -1456,6 +1394,201 @@ __device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const
         }
     }
     if (a.rk.cfl_red) wave_max_to(a.rk.cfl_red, cflv);
+}
+// General metric.  The window holds the differentiated fields only (u, v, w, T and eight cross
+// derivatives); once every thread has its face's derivatives and its node's, mu and the metric of the
+// tile's nodes take its place.  Bound by latency: with the metric in the window the 16 x 12 tile needed
+// 56 KB and 168 VGPRs, six waves per CU; with it, and the 30 factors per face in place of the stress
+// contraction, 119 x 96 x 104 took 128, 113 and 172 us along xi, eta and zeta (with the update), 78, 75 and
+// 123 now.
+template <int S, int DIR, int TA, int TDI>
+__device__ __forceinline__ void visc_gen_body(const ViscArgs &a, const int bx, const int by, const int bz, double *lds)
+{
+    constexpr int G = (S + 1) / 2;
+    constexpr int WD = TDI - 1 + 2 * G;
+    constexpr int NW = WD * TA;
+    constexpr int NT = TA * TDI;
+    constexpr int NC = 8;                            // cross-derivative fields
+    constexpr int b1 = Others<DIR>::b1, b2 = Others<DIR>::b2;
+    constexpr int NP = 2 * G + 1;                    // line positions used by the zeta-index quirk
+    constexpr int NLV = 4 + NC;                      // values per position: u,v,w,T + cross
+    constexpr int MD = TDI + 1, NM = MD * TA;        // metric window: the nodes of a row's faces
+    double *const sm = lds;
+    double *const line = sm + (NLV * NW > 11 * NM ? NLV * NW : 11 * NM);
+    double *const lined = line + TA * NP * NLV;
+
+    const int t = threadIdx.x;
+    const int pa0 = a.alignA ? bx * TA : bx * TA + a.oA;
+    const int b = by;
+    const int d0 = bz * (TDI - 1);
+    const long bbase = (long)(b + a.oB) * a.sB;
+    const Consts &k = a.k;
+    const int ta = t / TDI, di = t - ta * TDI;
+    const int dn = d0 + di, pa = pa0 + ta;
+    const bool own = di < TDI - 1 && dn < a.nD && pa >= a.oA && pa < a.oA + a.nA;
+    const long n = bbase + (long)pa * a.sA + (long)(dn + a.oD) * a.sD;
+
+    for (int idx = t; idx < NW; idx += NT) {
+        int aa, dd;
+        if (a.coalesce_d) { aa = idx / WD; dd = idx - aa * WD; }
+        else { dd = idx / TA; aa = idx - dd * TA; }
+        const int pa = max(a.oA, min(pa0 + aa, a.oA + a.nA - 1));
+        int dp = d0 - G + dd + a.oD;
+        dp = max(0, min(dp, a.ngD - 1));
+        const long n = bbase + (long)pa * a.sA + (long)dp * a.sD;
+        const int o = aa * WD + dd;
+        sm[0 * NW + o] = a.u[n];
+        sm[1 * NW + o] = a.v[n];
+        sm[2 * NW + o] = a.w[n];
+        sm[3 * NW + o] = a.T[n];
+#pragma unroll
+        for (int c = 0; c < NC; c++) sm[(4 + c) * NW + o] = a.cr[c][n];
+    }
+    const bool bug = (DIR == 2) && a.bug;
+    if (bug) {
+        // the reference's zeta stencil (src/ZD.c:547-548) reads positions k' = j + l - g on the
+        // (i, j) line for every k: the face values are constant along the line
+        for (int idx = t; idx < TA * NP * NLV; idx += NT) {
+            const int ln = idx / (NP * NLV);
+            const int rem = idx - ln * NP * NLV;
+            const int pos = rem / NLV, f = rem - pos * NLV;
+            const int jpad = max(a.oA, min(pa0 + ln, a.oA + a.nA - 1));   // A axis is j for DIR = 2
+            // the reference's index (i ng_j + j) ng_k + k' with k' = j - g + pos in its unpadded
+            // k-fastest layout: where k' passes the row end (ng_j > ng_k) it reads the next rows
+            // (or the next plane's first ones), which the padded layout finds at (j', k'') below
+            const int kq = jpad - G + pos;
+            long n;
+            if (kq < a.ngD) {
+                n = bbase + (long)jpad * a.sA + kq;
+            } else {
+                int jr = jpad + kq / a.ngD;
+                const int kr = kq % a.ngD;
+                const int ia = jr / a.ngA;
+                jr -= ia * a.ngA;
+                n = bbase + (long)ia * a.sB + (long)jr * a.sA + kr;
+            }
+            double val;
+            if (f == 0) val = a.u[n];
+            else if (f == 1) val = a.v[n];
+            else if (f == 2) val = a.w[n];
+            else if (f == 3) val = a.T[n];
+            else val = a.cr[f - 4][n];
+            line[(ln * NP + pos) * NLV + f] = val;
+        }
+    }
+    __syncthreads();
+    if (bug && di < 2) {
+        // di = 0: minus-side values (positions 0..S), di = 1: plus side (positions 1..S+1)
+        const double *Lp = &line[(ta * NP + di) * NLV];
+#pragma unroll
+        for (int f = 0; f < NLV; f++) {
+            double acc = 0.0;
+            const double *cf = (f < 4) ? k.zd_mid : k.zd_int;
+#pragma unroll
+            for (int l = 0; l <= S; l++) acc += cf[l] * Lp[l * NLV + f];
+            lined[(ta * 2 + di) * NLV + f] = acc;
+        }
+    }
+    if (bug) __syncthreads();
+
+    const int ob = ta * WD + di;
+    double fv[NLV];                                  // the face's derivatives (own u,v,w,T; cross)
+    double dv[3] = {0.0, 0.0, 0.0}, vel[3], gc[6];   // the node's: along the direction, velocity, cross
+#pragma unroll
+    for (int f = 0; f < NLV; f++) fv[f] = 0.0;
+    if (!bug) {
+#pragma unroll
+        for (int l = 0; l <= S; l++) {
+            const double cm = k.zd_mid[l], ci = k.zd_int[l];
+#pragma unroll
+            for (int f = 0; f < NLV; f++) fv[f] += (f < 4 ? cm : ci) * sm[f * NW + ob + l];
+        }
+    }
+#pragma unroll
+    for (int l = 0; l <= S + 1; l++)
+#pragma unroll
+        for (int q = 0; q < 3; q++) dv[q] += k.zd_der[l] * sm[q * NW + ob + l];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        vel[q] = sm[q * NW + ob + G];
+        gc[q] = sm[(4 + q) * NW + ob + G];
+        gc[3 + q] = sm[(8 + q) * NW + ob + G];
+    }
+    __syncthreads();
+    // mu and the metric, position dd of a row: node d0 - 1 + dd
+    for (int idx = t; idx < NM; idx += NT) {
+        int aa, dd;
+        if (a.coalesce_d) { aa = idx / MD; dd = idx - aa * MD; }
+        else { dd = idx / TA; aa = idx - dd * TA; }
+        const int pa = max(a.oA, min(pa0 + aa, a.oA + a.nA - 1));
+        const int dp = min(d0 - 1 + dd + a.oD, a.ngD - 1);
+        const long n = bbase + (long)pa * a.sA + (long)dp * a.sD;
+        const int o = aa * MD + dd;
+#pragma unroll
+        for (int c = 0; c < 10; c++) sm[c * NM + o] = a.met.f[c][n];
+        sm[10 * NM + o] = a.mu[n];
+    }
+    __syncthreads();
+    const int mo = ta * MD + di;                     // the face's lower node; the thread's node is the next
+    double m1[10];
+#pragma unroll
+    for (int c = 0; c < 10; c++) m1[c] = sm[c * NM + mo + 1];
+    const double mu1 = sm[10 * NM + mo + 1];
+    double F[4], nxt[4];
+    {
+        double m0[10];
+#pragma unroll
+        for (int c = 0; c < 10; c++) m0[c] = sm[c * NM + mo];
+        const double mu0 = sm[10 * NM + mo];
+        // slot layout d[k*3+b], T at 9+b
+        auto face = [&](const double *v, double *F) {
+            double d[12];
+#pragma unroll
+            for (int q = 0; q < 4; q++) { d[3 * q + DIR] = v[q]; d[3 * q + b1] = v[4 + q]; d[3 * q + b2] = v[8 + q]; }
+            face_flux_generic<DIR>(d, m0, m1, mu0, mu1, F);
+        };
+        if (!bug) {
+            face(fv, F);
+#pragma unroll
+            for (int q = 0; q < 4; q++) nxt[q] = F[q];
+        } else {
+            face(&lined[(ta * 2 + 0) * NLV], F);
+            face(&lined[(ta * 2 + 1) * NLV], nxt);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) nxt[q] = next_lane(nxt[q]);
+
+    double cflv = 0.0;                               // CFL sum of this thread's node (end-of-step check)
+    if (own) {
+        double dF[4], g[12];
+#pragma unroll
+        for (int q = 0; q < 4; q++) dF[q] = nxt[q] - F[q];
+#pragma unroll
+        for (int q = 0; q < 3; q++) { g[3 * q + DIR] = dv[q]; g[3 * q + b1] = gc[q]; g[3 * q + b2] = gc[3 + q]; g[9 + q] = 0.0; }
+        const double prod = node_prod_generic<DIR>(g, m1, mu1);
+        const double work = vel[0] * dF[0] + vel[1] * dF[1] + vel[2] * dF[2];
+        const double gh = (a.iso_hi && dn == a.nD - 1) ? a.gam_iso : k.gam_heat;
+        double qv[5];
+#pragma unroll
+        for (int q = 0; q < 5; q++) qv[q] = a.q.f[q][n];
+#pragma unroll
+        for (int q = 0; q < 3; q++) qv[1 + q] = qv[1 + q] + k.psi * dF[q];
+        qv[4] = qv[4] + (gh * dF[3] + k.psi * (work + prod));
+        if (a.fuse_rk) {
+            rk_point(a.rk, n, m1[9], qv, m1, &cflv);
+        } else {
+#pragma unroll
+            for (int q = 1; q < 5; q++) a.q.f[q][n] = qv[q];
+        }
+    }
+    if (a.rk.cfl_red) wave_max_to(a.rk.cfl_red, cflv);
+}
+template <int S, int DIR, int TA, int TDI, bool DIAG>
+__device__ __forceinline__ void visc_body(const ViscArgs &a, const int bx, const int by, const int bz, double *lds)
+{
+    if constexpr (DIAG) visc_diag_body<S, DIR, TA, TDI>(a, bx, by, bz, lds);
+    else visc_gen_body<S, DIR, TA, TDI>(a, bx, by, bz, lds);
 }
 template <int S, int DIR, int TA, int TDI, bool DIAG>
 __global__ __launch_bounds__(TA * TDI) void k_visc_sweep(ViscArgs a)
@@ -1488,7 +1621,7 @@ __device__ __forceinline__ void zeta_body(const ZetaArgs &z, const int bx, const
     __syncthreads();
     // Q, U_n and Q_sum loaded ahead (measured at 256^3: 1.95 -> 1.75 ms; the same in the fused eta
     // kernel, which stores Q instead of updating the stage, made it slower)
-    visc_body<S, 2, 4, 64, true, true, true>(z.v, bx, by, bz, lds, inv);
+    visc_diag_body<S, 2, 4, 64, true, true>(z.v, bx, by, bz, lds, inv);
 }
 // FP64 W5: held to 128 VGPRs (four waves per SIMD, as the LDS allows): 1.55 ms at 256^3 against
 // 1.67 at three waves
@@ -1519,7 +1652,7 @@ __device__ __forceinline__ void eta_body(const EtaArgs &z, const int bx, const i
     double inv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     weno_body<5, 8, 32, 1, MIX, true>(z.w, bx, by, bz, lds, inv);
     __syncthreads();
-    visc_body<5, 1, 8, 32, true, true>(z.v, bx, by, bz, lds, inv);
+    visc_diag_body<5, 1, 8, 32, true>(z.v, bx, by, bz, lds, inv);
 }
 // FP64: four waves per SIMD (126 VGPRs; weno5_flux)
 constexpr int ETA_WAVES = 4;
@@ -1843,9 +1976,9 @@ __global__ __launch_bounds__(GKX * GJX) void k_visc_grad_march_xi(GradArgs a)
 // interfaces fill 240 of 256 threads.  Periodic cases read ghosts at their image and form T and mu from
 // what they read, so their stages need no ghost fill.
 // A plane of 64^2 to 200^2 nodes leaves most of the chip idle and its time is the chain of its launches:
-// six dependent kernels of 7-12 us per stage, one of 20 us here (64^2 WENO5 58 -> 20 us, 211 x 157 WENO9
-// 74 -> 28).  Large planes are bound by the FP64 pipe and its latency (one block per CU by LDS) and gain
-// from the passes over memory between the kernels: 1000 x 768 283 -> 224 us.
+// six dependent kernels of 7-12 us per stage, one of 19 us here (64^2 WENO5 58 -> 19 us, 211 x 157 WENO9
+// 74 -> 27).  Large planes are bound by the FP64 pipe and its latency (one block per CU by LDS) and gain
+// from the passes over memory between the kernels: 1000 x 768 283 -> 205 us.
 constexpr int PT = 15;
 struct PlaneArgs {
     WenoArgs w[2];                // the sweep records of xi and eta (Q in w[0].q)
@@ -1863,7 +1996,7 @@ template <int S>
 constexpr int plane_visc_lds()
 {
     constexpr int WD = PT + S + 1, RING = PT + 2;
-    return 2 * 5 * PT * PT + 4 * WD * WD + 6 * PT * WD + 9 * RING * RING + 2 * 3 * PT * PT;
+    return 2 * 5 * PT * PT + 4 * WD * WD + 6 * PT * WD + 8 * RING * RING + 2 * 3 * PT * PT;
 }
 template <int S, bool MIX>
 constexpr int plane_lds()
@@ -1871,37 +2004,41 @@ constexpr int plane_lds()
     return 2 * weno_lds<S, PT, PT + 1, -1, MIX>() > plane_visc_lds<S>() ? 2 * weno_lds<S, PT, PT + 1, -1, MIX>()
                                                                        : plane_visc_lds<S>();
 }
-// Viscous terms of a half's direction (CalcViscidFluxesIn{Xi,Eta}DirectionDirectly, src/ZD.c:47-480) at one
-// interface and the node above it.  mb: the ring position of the lower node of the face, ms its step along the
-// direction; own4: midpoint derivatives of u, v, w, T; cr: interpolated cross derivatives of u, v, T.
+// stress_along in 2D: d holds the derivatives of u, v, T along both directions (d[3k+b], T at 9+b) and of w
+// along DIR only; the rows' z entries are zero (FLAT) or not
 template <int DIR, bool FLAT>
-__device__ __forceinline__ void plane_face(const double *MM, const int mb, const int ms, const double own4[4],
-                                           const double cr[3], double F[4])
+__device__ __forceinline__ void plane_stress(const double d[12], const double m[10], double t[4])
 {
-    constexpr int NR = (PT + 2) * (PT + 2), B = 1 - DIR;
-    double m[2][10], mu[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int o = mb + h * ms;
-#pragma unroll
-        for (int c = 0; c < 10; c++) m[h][c] = 0.0;
-        m[h][0] = MM[o]; m[h][1] = MM[NR + o]; m[h][3] = MM[2 * NR + o]; m[h][4] = MM[3 * NR + o];
-        m[h][9] = MM[4 * NR + o];
-        mu[h] = MM[5 * NR + o];
-        if constexpr (!FLAT) { m[h][2] = MM[7 * NR + o]; m[h][5] = MM[8 * NR + o]; }
+    if constexpr (!FLAT) {
+        stress_along<DIR>(d, m, t);
+    } else {
+        const double ax = m[3 * DIR], ay = m[3 * DIR + 1];
+        const double ux = d[0] * m[0] + d[1] * m[3], uy = d[0] * m[1] + d[1] * m[4];
+        const double vx = d[3] * m[0] + d[4] * m[3], vy = d[3] * m[1] + d[4] * m[4];
+        const double p = (2. / 3.) * (ux + vy), s = uy + vx;
+        t[0] = (2. * ux - p) * ax + s * ay;
+        t[1] = (2. * vy - p) * ay + s * ax;
+        t[2] = d[6 + DIR] * (ax * ax + ay * ay);
+        t[3] = (d[9] * m[0] + d[10] * m[3]) * ax + (d[9] * m[1] + d[10] * m[4]) * ay;
     }
-    double d[12];
-#pragma unroll
-    for (int q = 0; q < 12; q++) d[q] = 0.0;
-    d[0 * 3 + DIR] = own4[0]; d[1 * 3 + DIR] = own4[1]; d[2 * 3 + DIR] = own4[2]; d[9 + DIR] = own4[3];
-    d[0 * 3 + B] = cr[0]; d[1 * 3 + B] = cr[1]; d[9 + B] = cr[2];
-    face_flux_generic<DIR>(d, m[0], m[1], mu[0], mu[1], F);
 }
-template <int S, int DIR>
+// metric and mu at ring position o
+template <bool FLAT>
+__device__ __forceinline__ double plane_metric(const double *MM, const int o, double m[10])
+{
+    constexpr int NR = (PT + 2) * (PT + 2);
+#pragma unroll
+    for (int c = 0; c < 10; c++) m[c] = 0.0;
+    m[0] = MM[o]; m[1] = MM[NR + o]; m[3] = MM[2 * NR + o]; m[4] = MM[3 * NR + o]; m[9] = MM[4 * NR + o];
+    if constexpr (!FLAT) { m[2] = MM[6 * NR + o]; m[5] = MM[7 * NR + o]; }
+    return MM[5 * NR + o];
+}
+// Viscous terms of a half's direction (CalcViscidFluxesIn{Xi,Eta}DirectionDirectly, src/ZD.c:47-480).
+template <int S, int DIR, bool FLAT>
 __device__ __forceinline__ void plane_visc(const PlaneArgs &z, const int t, const int d0, const double *UV,
                                            const double *DER, const double *MM, double *QV)
 {
-    constexpr int G = (S + 1) / 2, WD = PT + 2 * G, RN = WD * WD, ND = PT * WD, NR = (PT + 2) * (PT + 2);
+    constexpr int G = (S + 1) / 2, WD = PT + 2 * G, RN = WD * WD, ND = PT * WD;
     const WenoArgs &a = z.w[DIR];
     const Consts &k = a.k;
     const int ta = min(t / (PT + 1), PT - 1), di = t % (PT + 1);
@@ -1920,28 +2057,34 @@ __device__ __forceinline__ void plane_visc(const PlaneArgs &z, const int t, cons
         for (int f = 0; f < 3; f++) cr[f] += ci * crs[f * ND + cb + l * cs];
     }
     const int mb = (DIR == 0) ? di * (PT + 2) + ta + 1 : (ta + 1) * (PT + 2) + di, ms = (DIR == 0) ? PT + 2 : 1;
-    double F[4], nxt[4];
-    if (z.flat) plane_face<DIR, true>(MM, mb, ms, own4, cr, F);
-    else plane_face<DIR, false>(MM, mb, ms, own4, cr, F);
+    double F[4], nxt[4], d[12], m0[10], m1[10], t0[4], t1[4];
 #pragma unroll
-    for (int m = 0; m < 4; m++) nxt[m] = next_lane(F[m]);
+    for (int q = 0; q < 12; q++) d[q] = 0.0;
+#pragma unroll
+    for (int f = 0; f < 4; f++) d[3 * f + DIR] = own4[f];
+    d[1 - DIR] = cr[0]; d[3 + 1 - DIR] = cr[1]; d[9 + 1 - DIR] = cr[2];
+    const double mu0 = plane_metric<FLAT>(MM, mb, m0), mu1 = plane_metric<FLAT>(MM, mb + ms, m1);
+    plane_stress<DIR, FLAT>(d, m0, t0);
+    plane_stress<DIR, FLAT>(d, m1, t1);
+    const double w0 = 0.5 * (mu0 * m0[9]), w1 = 0.5 * (mu1 * m1[9]);
+#pragma unroll
+    for (int q = 0; q < 4; q++) F[q] = w0 * t0[q] + w1 * t1[q];
+#pragma unroll
+    for (int q = 0; q < 4; q++) nxt[q] = next_lane(F[q]);
     if (di < PT && t < PT * (PT + 1)) {
         const int p = rb + G * rs;
-        double dF[4], g[9], m[10];
+        double dF[4];
 #pragma unroll
         for (int q = 0; q < 4; q++) dF[q] = nxt[q] - F[q];
-#pragma unroll
-        for (int q = 0; q < 9; q++) g[q] = 0.0;
         const int po = (DIR == 0) ? di * WD + ta + G : (ta + G) * PT + di;   // the node in the own-direction arrays
         const int pc = cb + G * cs;                                          // and in the cross-direction ones
-        g[0 * 3 + DIR] = own[po]; g[1 * 3 + DIR] = own[ND + po];
-        g[0 * 3 + 1 - DIR] = crs[pc]; g[1 * 3 + 1 - DIR] = crs[ND + pc];
-        const int o = mb + ms;
+        double g[12];
 #pragma unroll
-        for (int q = 0; q < 10; q++) m[q] = 0.0;
-        m[0] = MM[o]; m[1] = MM[NR + o]; m[3] = MM[2 * NR + o]; m[4] = MM[3 * NR + o]; m[9] = MM[4 * NR + o];
-        if (!z.flat) { m[2] = MM[7 * NR + o]; m[5] = MM[8 * NR + o]; }
-        const double prod = node_prod_generic<DIR>(g, m, MM[5 * NR + o]);
+        for (int q = 0; q < 12; q++) g[q] = 0.0;
+        g[DIR] = own[po]; g[3 + DIR] = own[ND + po];
+        g[1 - DIR] = crs[pc]; g[3 + 1 - DIR] = crs[ND + pc];
+        plane_stress<DIR, FLAT>(g, m1, t1);
+        const double prod = (mu1 * m1[9]) * (g[DIR] * t1[0] + g[3 + DIR] * t1[1]);
         const double work = UV[p] * dF[0] + UV[RN + p] * dF[1] + UV[2 * RN + p] * dF[2];
         const double gh = (z.iso_hi[DIR] && d0 + di == a.nD - 1) ? z.gam_iso : k.gam_heat;
         const int node = (DIR == 0) ? di * PT + ta : ta * PT + di;
@@ -1962,7 +2105,7 @@ __device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, d
     weno_body<S, PT, PT + 1, -1, MIX, true, 256>(z.w[half], half ? ti : tj, 0, half ? tj : ti, lds + half * WL, keep);
     __syncthreads();
     double *const QW = lds, *const UV = QW + 2 * 5 * NN, *const DER = UV + 4 * RN, *const MM = DER + 6 * ND;
-    double *const QV = MM + 9 * NR;
+    double *const QV = MM + 8 * NR;
     if (di < PT && t < PT * (PT + 1)) {
         const int node = half ? ta * PT + di : di * PT + ta;
 #pragma unroll
@@ -1997,7 +2140,7 @@ __device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, d
                 M[0] = z.met.f[0][n]; M[NR] = z.met.f[1][n]; M[2 * NR] = z.met.f[3][n]; M[3 * NR] = z.met.f[4][n];
                 M[4 * NR] = z.met.f[9][n];
                 M[5 * NR] = mu;
-                if (!z.flat) { M[7 * NR] = z.met.f[2][n]; M[8 * NR] = z.met.f[5][n]; }
+                if (!z.flat) { M[6 * NR] = z.met.f[2][n]; M[7 * NR] = z.met.f[5][n]; }
             }
         }
         __syncthreads();
@@ -2017,8 +2160,13 @@ __device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, d
             for (int f = 0; f < 3; f++) DER[(half * 3 + f) * ND + idx] = d[f];
         }
         __syncthreads();
-        if (half == 0) plane_visc<S, 0>(z, t, ti * PT, UV, DER, MM, QV);
-        else plane_visc<S, 1>(z, t, tj * PT, UV, DER, MM, QV + 3 * NN);
+        if (z.flat) {
+            if (half == 0) plane_visc<S, 0, true>(z, t, ti * PT, UV, DER, MM, QV);
+            else plane_visc<S, 1, true>(z, t, tj * PT, UV, DER, MM, QV + 3 * NN);
+        } else {
+            if (half == 0) plane_visc<S, 0, false>(z, t, ti * PT, UV, DER, MM, QV);
+            else plane_visc<S, 1, false>(z, t, tj * PT, UV, DER, MM, QV + 3 * NN);
+        }
     }
     __syncthreads();
     double cflv = 0.0;
@@ -3541,21 +3689,17 @@ static Pick visc_pick_t()
             (const void *)&k_visc_batch<S, DIR, TA, TDI, DIAG, true>, TA, TDI};
 }
 
-// tiles sized so that the LDS window (13 or 23 values per node) plus the face buffer fit:
-// diagonal metric 16 x 16 for WENO5 and 16 x 32 for WENO9, whose 2G = 10 halo rows make short
-// tiles re-read most of their window (16 x 32 runs the WENO9 xi / eta sweeps 21 % faster than
-// 16 x 12 at 384^3; WENO5 is fastest at 16 x 16); generic 16 x 12 / 16 x 8 (4 x 48 contiguous)
+// tiles sized so that three or four blocks share a CU: diagonal metric 16 x 16 for WENO5 and 16 x 32 for
+// WENO9, whose 2G = 10 halo rows make short tiles re-read most of their window (16 x 32 runs the WENO9
+// xi / eta sweeps 21 % faster than 16 x 12 at 384^3; WENO5 is fastest at 16 x 16); general metric 16 x 16;
+// 4 x 64 along the contiguous axis
 template <int S>
 static Pick visc_pick_s(int dir, bool coalesce, bool diag)
 {
     constexpr int TDN = (S == 5) ? 16 : 32;
-    constexpr int TDG = (S == 5) ? 12 : 8;
-    if (coalesce) {
-        if (diag) return visc_pick_t<S, 2, 4, 64, true>();
-        return visc_pick_t<S, 2, 4, 48, false>();
-    }
+    if (coalesce) return diag ? visc_pick_t<S, 2, 4, 64, true>() : visc_pick_t<S, 2, 4, 64, false>();
     if (diag) return (dir == 0) ? visc_pick_t<S, 0, 16, TDN, true>() : visc_pick_t<S, 1, 16, TDN, true>();
-    return (dir == 0) ? visc_pick_t<S, 0, 16, TDG, false>() : visc_pick_t<S, 1, 16, TDG, false>();
+    return (dir == 0) ? visc_pick_t<S, 0, 16, 16, false>() : visc_pick_t<S, 1, 16, 16, false>();
 }
 
 static Pick visc_pick(const shx_case *c, int dir)
