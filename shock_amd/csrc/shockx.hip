@@ -906,6 +906,8 @@ struct RkArgs {
     // non-finite interior densities (those nodes get rho = u = v = w (= stored p) = 1e6);
     // cfl_red: the maximum of the node CFL sum, as the bits of a positive double
     int *nan_cnt;
+    int *nan_flag;           // pinned host word set to 1 with the count, which the host reads after the
+                             // step instead of copying the count (null in batches)
     gdp nanP;
     unsigned long long *cfl_red;
     double gamma, upsilon;
@@ -1029,6 +1031,7 @@ __device__ __forceinline__ void rk_point(const RkArgs &A, const long n, const do
         A.out.f[0][n] = 1000000; A.out.f[1][n] = 1000000; A.out.f[2][n] = 1000000; A.out.f[3][n] = 1000000;
         if (A.nanP) A.nanP[n] = 1000000;
         atomicAdd(A.nan_cnt, 1);
+        if (A.nan_flag) __hip_atomic_store(A.nan_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     } else if (A.cfl_red && cfl) {
         *cfl = node_cfl_sum<DIAG>(A.gamma, A.upsilon, A.three ? 3 : 2, nv[0], nv[1], nv[2], nv[3], nv[4], m9);
     }
@@ -2476,6 +2479,21 @@ __global__ void k_cfl_max(CFields5 pr, CFields10 met, Geom gm, Consts k, unsigne
     }
 }
 
+// the maximum of the slots to a pinned host word; the slots are left clear (one block of RED_SLOTS)
+__global__ __launch_bounds__(RED_SLOTS) void k_red_report(unsigned long long *red, unsigned long long *host)
+{
+    __shared__ double sh[RED_SLOTS / 64];
+    const double v = wave_max(__longlong_as_double((long long)red[threadIdx.x]));
+    red[threadIdx.x] = 0;
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double m = sh[0];
+        for (int w = 1; w < RED_SLOTS / 64; w++) m = fmax(m, sh[w]);
+        __hip_atomic_store(host, (unsigned long long)__double_as_longlong(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // checkNAN (src/Functions.c:5419-5467): count and overwrite non-finite interior rho (and the
 // stored p, where it is kept).
 __global__ void k_check_nan(Fields5 pr, gdp P, Geom gm, int *count)
@@ -2788,7 +2806,7 @@ struct shx_case {
     int *d_cnt;
     int *d_nan;            // running count of the fused checkNAN (shx_run, shx_run_cfl, shx_simulate)
     int nan_seen;          // the count last read
-    struct HostIo { unsigned long long red[RED_SLOTS]; int nan; int pad; double mms[4]; } *h_io;   // pinned landing slots
+    struct HostIo { unsigned long long red; int nan; int nan_flag; double mms[4]; } *h_io;   // pinned landing slots
     int dev;               // the device current at shx_create (the stream's)
     int ncu;               // its compute units
     int st_in, st_out, st_bx, st_by;   // buffers of the step in progress (step_begin .. step_end)
@@ -2994,7 +3012,7 @@ extern "C" int shx_create(const shx_desc *desc, shx_case **out)
     if (e == hipSuccess) e = hipMalloc((void **)&c->d_nan, sizeof(int));
     if (e == hipSuccess) e = hipMemsetAsync(c->d_nan, 0, sizeof(int), c->stream);
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_io, sizeof(shx_case::HostIo), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) { memset(c->h_io, 0, sizeof(shx_case::HostIo)); e = hipStreamSynchronize(c->stream); }
     if (e != hipSuccess) { shx_destroy(c); return set_err(SHX_ERR_HIP, "setup: %s", hipGetErrorString(e)); }
     c->cur = 0;
     // WENO tiles until shx_tune times them: 4 x 64 along the contiguous axis and 16 x 16 across it, but
@@ -3872,7 +3890,7 @@ enum { STEP_NAN = 1, STEP_CFL = 2 };
 
 // One time step (CalcRungeKutta and the step-end copy).  flags: STEP_NAN adds checkNAN on the new
 // state to the running count c->d_nan; STEP_CFL puts the maximum node CFL sum of the new state
-// into c->d_red (which the caller clears).
+// into c->d_red (clear before it).
 // A step in three parts, so that the blocks of a multi-block case advance stage by stage together:
 // step_begin (the Rudy faces' step-start state; buffers), step_stage (one stage), step_end (the
 // step-end copy).  Stage s reads buffer st_in and writes st_out; stage s+1 reads what stage s wrote
@@ -3891,7 +3909,7 @@ static int step_stage(shx_case *c, int s, double tau, int flags)
     int rc;
     RkArgs rk = rk_args(c, c->prim[c->st_in], c->prim[c->st_out], s, tau);
     if (s == c->d.time_order - 1) {
-        if (flags & STEP_NAN) { rk.nan_cnt = c->d_nan; rk.nanP = c->P; }
+        if (flags & STEP_NAN) { rk.nan_cnt = c->d_nan; rk.nan_flag = &c->h_io->nan_flag; rk.nanP = c->P; }
         if (flags & STEP_CFL) rk.cfl_red = c->d_red;
     }
     // viscous and 2D stages apply the update in their last kernel; 3D inviscid ones in k_rk_update
@@ -3925,9 +3943,14 @@ static int step_rk(shx_case *c, double tau, int flags)
 
 extern "C" int shx_calc_runge_kutta(shx_case *c, double tau) { return step_rk(c, tau, 0); }
 
-// Non-finite densities the fused checkNAN found since the last call (synchronizes the stream).
+// Non-finite densities the fused checkNAN found since the last call (synchronizes the stream).  The
+// update raises the host's flag with the count, so a finite step costs no copy.
 static int nan_found(shx_case *c, int &fresh)
 {
+    HIPCHK(hipStreamSynchronize(c->stream));
+    fresh = 0;
+    if (!*(volatile int *)&c->h_io->nan_flag) return SHX_OK;
+    c->h_io->nan_flag = 0;
     HIPCHK(hipMemcpyAsync(&c->h_io->nan, c->d_nan, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     fresh = c->h_io->nan - c->nan_seen;
@@ -4988,12 +5011,10 @@ extern "C" int shx_run(shx_case *c, double tau, int nsteps)
     return SHX_OK;
 }
 
-// the maximum node CFL sum the last reduction into c->d_red left (its slots copied to h_io->red,
-// stream synchronized)
+// the maximum node CFL sum red_fetch left (stream synchronized)
 static double red_max(shx_case *c)
 {
-    unsigned long long mb = 0;
-    for (int s = 0; s < RED_SLOTS; s++) mb = std::max(mb, c->h_io->red[s]);
+    const unsigned long long mb = *(volatile unsigned long long *)&c->h_io->red;
     double mx;
     memcpy(&mx, &mb, sizeof mx);
     return mx;
@@ -5003,10 +5024,12 @@ static int red_clear(shx_case *c)
     HIPCHK(hipMemsetAsync(c->d_red, 0, sizeof(unsigned long long) * RED_SLOTS, c->stream));
     return SHX_OK;
 }
+// the slots' maximum into the host's word, and the slots cleared for the next reduction: one small
+// launch where a step used to end in a fill and two copies
 static int red_fetch(shx_case *c)
 {
-    HIPCHK(hipMemcpyAsync(c->h_io->red, c->d_red, sizeof(unsigned long long) * RED_SLOTS, hipMemcpyDeviceToHost,
-                          c->stream));
+    k_red_report<<<1, RED_SLOTS, 0, c->stream>>>(c->d_red, &c->h_io->red);
+    LAUNCH_CHECK();
     return SHX_OK;
 }
 
@@ -5035,7 +5058,6 @@ extern "C" int shx_run_cfl(shx_case *c, double cfl, int nsteps, double *time)
         const double mx = red_max(c);
         if (!(mx > 0.0) || !std::isfinite(mx)) return set_err(SHX_ERR_NAN, "CFL maximum %g before step %d", mx, s + 1);
         const double dt = cfl / mx;
-        if ((rc = red_clear(c))) return rc;
         if ((rc = step_rk(c, dt, STEP_NAN | STEP_CFL))) return rc;
         if ((rc = red_fetch(c))) return rc;
         int bad = 0;
