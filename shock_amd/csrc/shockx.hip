@@ -2713,6 +2713,42 @@ __global__ void k_check_metric(gcdp J, Geom gm, int *count)
     if ((threadIdx.x & 63) == 0 && bad) atomicAdd(count, bad);
 }
 
+// Rows of several device fields (pitched) to or from dense rows in pinned host memory, doubles
+// [t0, t0 + n) of the fields' dense concatenation; an upload may fill further copies of each field.
+// PCIe bounds both (53-57 GB/s, as a pitched DMA reaches), and one launch serves all fields.
+constexpr int XFER_FIELDS = 10;
+struct XferArgs {
+    gdp dev[XFER_FIELDS], more[2][XFER_FIELDS];
+    double *host;
+    long t0, n, w, pitch, hw;     // row length, device pitch, doubles of one dense field
+    int copies;                   // of `more` filled by an upload
+};
+__device__ __forceinline__ long xfer_index(const XferArgs &a, const long t, int &m)
+{
+    m = (int)(t / a.hw);
+    const long r = t - (long)m * a.hw, row = r / a.w;
+    return row * a.pitch + (r - row * a.w);
+}
+__global__ __launch_bounds__(256) void k_pack(XferArgs a)
+{
+    for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < a.n; q += (long)gridDim.x * 256) {
+        int m;
+        const long n = xfer_index(a, a.t0 + q, m);
+        a.host[q] = a.dev[m][n];
+    }
+}
+__global__ __launch_bounds__(256) void k_unpack(XferArgs a)
+{
+    for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < a.n; q += (long)gridDim.x * 256) {
+        int m;
+        const long n = xfer_index(a, a.t0 + q, m);
+        const double v = a.host[q];
+        a.dev[m][n] = v;
+        if (a.copies > 0) a.more[0][m][n] = v;
+        if (a.copies > 1) a.more[1][m][n] = v;
+    }
+}
+
 // Plain streaming copy of n doubles (calibration of hardware byte counters).
 __global__ void k_copy(const double *__restrict__ a, double *__restrict__ b, long n)
 {
@@ -2772,6 +2808,8 @@ static void wall_corrector(const int kind, const int dir, double cr[3])
     if (kind == SHX_BC_WALL_NOSLIP || kind == SHX_BC_WALL_ISOTHERMAL) cr[0] = cr[1] = cr[2] = -1.0;
 }
 
+constexpr int STAGE_SLOTS = 8;   // staging slots of host transfers, two per host thread
+
 struct shx_case {
     shx_desc d;
     Geom gm;
@@ -2822,11 +2860,11 @@ struct shx_case {
     // they were at shx_batch_create); stepping the case alone while it is set would leave the
     // batch advancing a stale buffer
     shx_batch *batch = nullptr;
-    // pinned staging of host transfers (allocated on the first upload or download): two buffers
-    // of stage_bytes, each with the event of the copy that last used it
-    double *stage_h[2] = {nullptr, nullptr};
-    hipEvent_t stage_ev[2] = {nullptr, nullptr};
-    size_t stage_bytes = 0;
+    // pinned staging of host transfers (allocated on the first upload or download): STAGE_SLOTS slots
+    // of stage_len doubles, each with the event of the launch that last used it
+    double *stage_h = nullptr;
+    hipEvent_t stage_ev[STAGE_SLOTS] = {};
+    long stage_len = 0;
 };
 
 extern "C" const char *shx_last_error(void) { return g_err; }
@@ -3040,10 +3078,9 @@ extern "C" int shx_destroy(shx_case *c)
     for (int m = 0; m < 6; m++) hipFree(c->bs[m]);
     hipFree(c->T); hipFree(c->mu); hipFree(c->d_red); hipFree(c->d_cnt); hipFree(c->d_nan);
     if (c->h_io) hipHostFree(c->h_io);
-    for (int b = 0; b < 2; b++) {
+    for (int b = 0; b < STAGE_SLOTS; b++)
         if (c->stage_ev[b]) hipEventDestroy(c->stage_ev[b]);
-        if (c->stage_h[b]) hipHostFree(c->stage_h[b]);
-    }
+    if (c->stage_h) hipHostFree(c->stage_h);
     hipFree(c->P); hipFree(c->C); hipFree(c->PL); hipFree(c->RL); hipFree(c->UL); hipFree(c->C0);
     for (int b = 0; b < 2; b++) {
         for (int m = 0; m < 5; m++) hipFree(c->bk[b][m]);
@@ -3066,104 +3103,136 @@ extern "C" int shx_padded_extent(const shx_case *c, int ng[3])
     return SHX_OK;
 }
 
-// host arrays use the reference layout (dense rows); device rows are padded to the pitch
-static void row_geometry(const shx_case *c, size_t &width, size_t &height, size_t &dpitch)
+// Host transfers.  Host arrays use the reference layout (dense rows); device rows are padded to the
+// pitch.  k_pack and k_unpack move chunks of all fields of a call between the device and slots of pinned
+// memory, and host threads copy between the slots and the caller's arrays.  A thread owns every fourth
+// chunk and two slots: the launch of its next chunk is in flight while it copies one (a thread copies
+// ~14 GB/s, PCIe moves 53), and no thread waits for another.  Field by field through two slots, with a
+// copy's threads started per slot, the pipeline drained between fields: state downloads of a 64^2 plane
+// 118 -> 21 us, 48^3 479 -> 250, 1000 x 768 1.25 -> 0.80 ms, 97 x 85 x 106 1.74 -> 1.12, 256^3 14.9 either
+// way (PCIe).  2 MB slots and four threads: 512 KB slots or eight threads measured slower.
+// A pitched copy straight to or from pageable memory ran at 0.3 GB/s.
+constexpr long STAGE_MIN = 1L << 15, STAGE_MAX = 1L << 18;   // doubles per slot: 256 KB to 2 MB
+struct Xfer {
+    shx_case *c;
+    XferArgs k;
+    bool up;
+    double *host[XFER_FIELDS];    // the caller's arrays (read only by an upload)
+    long total, chunk;
+    int threads;
+};
+static hipError_t xfer_launch(const Xfer &x, const long i, const int slot)
+{
+    XferArgs k = x.k;
+    k.t0 = i * x.chunk;
+    k.n = std::min(x.chunk, x.total - k.t0);
+    k.host = x.c->stage_h + (long)slot * x.c->stage_len;
+    const unsigned grid = (unsigned)std::min<long>((k.n + 255) / 256, 1024);
+    if (x.up) k_unpack<<<grid, 256, 0, x.c->stream>>>(k);
+    else k_pack<<<grid, 256, 0, x.c->stream>>>(k);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipEventRecord(x.c->stage_ev[slot], x.c->stream);
+    return e;
+}
+// chunk i between its slot and the caller's arrays
+static void xfer_copy(const Xfer &x, const long i, const int slot)
+{
+    const double *s = x.c->stage_h + (long)slot * x.c->stage_len;
+    for (long t = i * x.chunk, end = std::min(t + x.chunk, x.total); t < end;) {
+        const long m = t / x.k.hw, r = t - m * x.k.hw, n = std::min(x.k.hw - r, end - t);
+        if (x.up) memcpy((void *)s, x.host[m] + r, sizeof(double) * n);
+        else memcpy(x.host[m] + r, s, sizeof(double) * n);
+        s += n;
+        t += n;
+    }
+}
+// the chunks of thread id: id, id + threads, ...
+static hipError_t xfer_chunks(const Xfer &x, const int id)
+{
+    const long nc = (x.total + x.chunk - 1) / x.chunk;
+    const int s0 = 2 * id;
+    hipError_t e = id ? hipSetDevice(x.c->dev) : hipSuccess;   // a new thread starts on device 0
+    long turn = 0;
+    if (x.up) {
+        // a slot's previous launch (two turns back, or an earlier call's) has read it
+        for (long i = id; i < nc && e == hipSuccess; i += x.threads, turn++) {
+            const int slot = s0 + (int)(turn & 1);
+            if ((e = hipEventSynchronize(x.c->stage_ev[slot])) != hipSuccess) break;
+            xfer_copy(x, i, slot);
+            e = xfer_launch(x, i, slot);
+        }
+        return e;
+    }
+    for (int q = 0; q < 2 && e == hipSuccess; q++)
+        if (id + (long)q * x.threads < nc) e = xfer_launch(x, id + (long)q * x.threads, s0 + q);
+    for (long i = id; i < nc && e == hipSuccess; i += x.threads, turn++) {
+        const int slot = s0 + (int)(turn & 1);
+        if ((e = hipEventSynchronize(x.c->stage_ev[slot])) != hipSuccess) break;
+        xfer_copy(x, i, slot);
+        if (i + 2L * x.threads < nc) e = xfer_launch(x, i + 2L * x.threads, slot);
+    }
+    return e;
+}
+// nf fields between the device arrays dev and the caller's dense arrays host; an upload also fills the
+// `copies` further arrays of each field.  A download returns with the arrays written; an upload once they
+// have been read (the launches may still be in flight on the case's stream).
+static int transfer(shx_case *c, const bool up, const int nf, double *const *dev, double *const *host,
+                    double *const *const *more = nullptr, const int copies = 0)
 {
     const Geom &gm = c->gm;
-    if (gm.dims == 3) { width = sizeof(double) * gm.ng[2]; height = (size_t)gm.ng[0] * gm.ng[1]; dpitch = sizeof(double) * gm.st[1]; }
-    else { width = sizeof(double) * gm.ng[1]; height = (size_t)gm.ng[0]; dpitch = sizeof(double) * gm.st[0]; }
-}
-// Host transfers go through two pinned staging buffers: a pitched copy between the padded device
-// rows and dense rows in pinned memory (a DMA at PCIe rate), and a plain memcpy between pinned and
-// the caller's memory, chunk by chunk, the memcpy of one chunk overlapping the DMA of the next.
-// A pitched copy straight to or from pageable memory ran at 0.3 GB/s (256^3: 2.5 s to download the
-// five state fields); staged, the transfer is bound by the host memcpy.
-constexpr size_t STAGE_MAX = size_t(8) << 20;
-// memcpy of a staging chunk on up to four host threads (one host thread copies ~14 GB/s, under the
-// DMA's rate); chunks under 1 MB are copied on the calling thread
-static void stage_memcpy(void *dst, const void *src, const size_t n)
-{
-    constexpr int NTH = 4;
-    if (n < (size_t(1) << 20)) { memcpy(dst, src, n); return; }
-    const size_t part = ((n + NTH - 1) / NTH + 63) & ~size_t(63);
-    std::thread th[NTH - 1];
-    int started = 0;
-    for (int t = 1; t < NTH; t++) {
-        const size_t off = (size_t)t * part;
-        if (off >= n) break;
-        char *d = (char *)dst + off;
-        const char *sp = (const char *)src + off;
-        const size_t len = std::min(part, n - off);
-        try {
-            th[started] = std::thread([d, sp, len] { memcpy(d, sp, len); });
-            started++;
-        } catch (...) {
-            memcpy(d, sp, len);        // no thread available: copy this part here
-        }
+    Xfer x;
+    memset(&x, 0, sizeof x);
+    x.c = c;
+    x.up = up;
+    x.k.w = (gm.dims == 3) ? gm.ng[2] : gm.ng[1];
+    x.k.pitch = (gm.dims == 3) ? gm.st[1] : gm.st[0];
+    x.k.hw = gm.ntot;
+    x.k.copies = copies;
+    for (int m = 0; m < nf; m++) {
+        if (!host[m]) return set_err(SHX_ERR_ARG, "null field pointer");
+        x.k.dev[m] = dev[m];
+        x.host[m] = host[m];
+        for (int q = 0; q < copies; q++) x.k.more[q][m] = more[q][m];
     }
-    memcpy(dst, src, std::min(part, n));
-    for (int t = 0; t < started; t++) th[t].join();
-}
-static int ensure_stage(shx_case *c, const size_t w, const size_t h)
-{
-    if (c->stage_h[0]) return SHX_OK;
-    c->stage_bytes = std::max(w, std::min(STAGE_MAX, w * h));
-    for (int b = 0; b < 2; b++) {
-        HIPCHK(hipHostMalloc((void **)&c->stage_h[b], c->stage_bytes, hipHostMallocDefault));
+    x.total = (long)nf * gm.ntot;
+    if (!c->stage_h) {
+        // slots for the five fields of a state in two chunks per thread, within the limits
+        const long len = std::max(STAGE_MIN, std::min(STAGE_MAX, (5 * gm.ntot + STAGE_SLOTS - 1) / STAGE_SLOTS));
+        HIPCHK(hipHostMalloc((void **)&c->stage_h, sizeof(double) * (size_t)len * STAGE_SLOTS, hipHostMallocDefault));
+        c->stage_len = len;
+    }
+    for (int b = 0; b < STAGE_SLOTS; b++) {
+        if (c->stage_ev[b]) continue;
         HIPCHK(hipEventCreateWithFlags(&c->stage_ev[b], hipEventDisableTiming));
         HIPCHK(hipEventRecord(c->stage_ev[b], c->stream));
     }
+    x.chunk = c->stage_len;
+    const long nc = (x.total + x.chunk - 1) / x.chunk;
+    // up to four threads; a call of few small chunks stays on the calling one
+    x.threads = (x.total < 2 * STAGE_SLOTS * STAGE_MIN / 4) ? 1 : (int)std::min<long>(STAGE_SLOTS / 2, nc);
+    hipError_t err[STAGE_SLOTS / 2];
+    std::thread th[STAGE_SLOTS / 2];
+    for (int t = 1; t < x.threads; t++) {
+        err[t] = hipErrorUnknown;
+        try {
+            th[t] = std::thread([&x, &err, t] { err[t] = xfer_chunks(x, t); });
+        } catch (...) {
+        }
+    }
+    err[0] = xfer_chunks(x, 0);
+    for (int t = 1; t < x.threads; t++) {
+        if (th[t].joinable()) th[t].join();
+        else err[t] = xfer_chunks(x, t);       // no thread available: its chunks here
+    }
+    for (int t = 0; t < x.threads; t++) HIPCHK(err[t]);
     return SHX_OK;
 }
 static int copy_in(shx_case *c, double *dst, const double *src)
 {
-    if (!src) return set_err(SHX_ERR_ARG, "null field pointer");
-    size_t w, h, dp;
-    row_geometry(c, w, h, dp);
-    int rc = ensure_stage(c, w, h);
-    if (rc) return rc;
-    const size_t rows = c->stage_bytes / w;
-    int b = 0;
-    for (size_t r0 = 0; r0 < h; r0 += rows, b ^= 1) {
-        const size_t nr = std::min(rows, h - r0);
-        // the buffer's previous copy (two chunks back, or an earlier call's) has been read
-        HIPCHK(hipEventSynchronize(c->stage_ev[b]));
-        stage_memcpy(c->stage_h[b], (const char *)src + r0 * w, nr * w);
-        HIPCHK(hipMemcpy2DAsync((char *)dst + r0 * dp, dp, c->stage_h[b], w, w, nr, hipMemcpyHostToDevice,
-                                c->stream));
-        HIPCHK(hipEventRecord(c->stage_ev[b], c->stream));
-    }
-    return SHX_OK;
+    double *h = const_cast<double *>(src);
+    return transfer(c, true, 1, &dst, &h);
 }
-static int copy_out(shx_case *c, double *dst, const double *src)
-{
-    if (!dst) return set_err(SHX_ERR_ARG, "null field pointer");
-    size_t w, h, dp;
-    row_geometry(c, w, h, dp);
-    int rc = ensure_stage(c, w, h);
-    if (rc) return rc;
-    const size_t rows = c->stage_bytes / w;
-    // a staging buffer may still feed an upload's copy: the first chunk's DMA is queued behind it
-    // on the stream, and every chunk is read out only after its own event
-    size_t prev = h;     // first row of the chunk waiting to be read out (h: none)
-    int b = 0;
-    for (size_t r0 = 0;; r0 += rows, b ^= 1) {
-        if (r0 < h) {
-            const size_t nr = std::min(rows, h - r0);
-            HIPCHK(hipMemcpy2DAsync(c->stage_h[b], w, (const char *)src + r0 * dp, dp, w, nr,
-                                    hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(hipEventRecord(c->stage_ev[b], c->stream));
-        }
-        if (prev < h) {
-            const int pb = b ^ 1;
-            HIPCHK(hipEventSynchronize(c->stage_ev[pb]));
-            stage_memcpy((char *)dst + prev * w, c->stage_h[pb], std::min(rows, h - prev) * w);
-        }
-        if (r0 >= h) break;
-        prev = r0;
-    }
-    return SHX_OK;
-}
+static int copy_out(shx_case *c, double *dst, double *src) { return transfer(c, false, 1, &src, &dst); }
 
 static int ghost_fill(shx_case *c, double *const *f, int nf)
 {
@@ -3303,7 +3372,8 @@ extern "C" int shx_build_metric(shx_case *c, const double *xe, const double *ye,
 extern "C" int shx_upload_metric(shx_case *c, const double *const met[10])
 {
     if (!c || !met) return set_err(SHX_ERR_ARG, "null argument");
-    for (int m = 0; m < 10; m++) { int rc = copy_in(c, c->met[m], met[m]); if (rc) return rc; }
+    int rc = transfer(c, true, 10, c->met, const_cast<double *const *>(met));
+    if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     c->has_metric = 1;
     // the diagonal-metric kernels apply when every off-diagonal entry is exactly zero
@@ -3324,7 +3394,8 @@ extern "C" int shx_upload_metric(shx_case *c, const double *const met[10])
 extern "C" int shx_download_metric(shx_case *c, double *const met[10])
 {
     if (!c || !met) return set_err(SHX_ERR_ARG, "null argument");
-    for (int m = 0; m < 10; m++) { int rc = copy_out(c, met[m], c->met[m]); if (rc) return rc; }
+    int rc = transfer(c, false, 10, c->met, met);
+    if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     return SHX_OK;
 }
@@ -3335,13 +3406,9 @@ extern "C" int shx_upload_state(shx_case *c, const double *const prim[5])
     // every stage buffer gets the full array: ghost nodes that no fill writes keep these values,
     // as they do in the reference's single U_RK array
     const size_t bytes = sizeof(double) * (size_t)c->gm.nalloc;
-    for (int m = 0; m < 5; m++) {
-        int rc = copy_in(c, c->prim[c->cur][m], prim[m]);
-        if (rc) return rc;
-        for (int b = 0; b < 3; b++)
-            if (b != c->cur)
-                HIPCHK(hipMemcpyAsync(c->prim[b][m], c->prim[c->cur][m], bytes, hipMemcpyDeviceToDevice, c->stream));
-    }
+    double *const *more[2] = {c->prim[(c->cur + 1) % 3], c->prim[(c->cur + 2) % 3]};
+    int rc = transfer(c, true, 5, c->prim[c->cur], const_cast<double *const *>(prim), more, 2);
+    if (rc) return rc;
     if (c->pc) {
         // stored p and c of the uploaded state on every node; for Rudy faces also the step-start
         // sound speed, which stays as uploaded (the reference never recomputes U_lastStep's c)
@@ -3381,7 +3448,8 @@ extern "C" int shx_download_state(shx_case *c, double *const prim[5])
     // the ghost values the reference's U_lastStep holds after a step
     int rc0 = sync_ghosts(c);
     if (rc0) return rc0;
-    for (int m = 0; m < 5; m++) { int rc = copy_out(c, prim[m], c->prim[c->cur][m]); if (rc) return rc; }
+    int rc = transfer(c, false, 5, c->prim[c->cur], prim);
+    if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     return SHX_OK;
 }
@@ -5473,7 +5541,7 @@ extern "C" int shx_rhs(shx_case *c, double *const q[5])
         k_add_source<<<nblk(nint, 256), 256, 0, c->stream>>>(qf, sf, c->met[9], gm);
         LAUNCH_CHECK();
     }
-    for (int m = 0; m < 5; m++) { rc = copy_out(c, q[m], c->q[m]); if (rc) return rc; }
+    if ((rc = transfer(c, false, 5, c->q, q))) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     return SHX_OK;
 }
