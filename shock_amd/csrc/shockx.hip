@@ -15,7 +15,7 @@
 //                      the source (src/Functions.c:2287-2365) and writes the next stage state
 //                      into another buffer (the reference updates in place after all fluxes of
 //                      the stage are assembled, which the separate buffer reproduces exactly)
-//   k_rk_update        source + RK update for inviscid runs
+//   k_weno_last        the last direction's WENO sweep, which applies the update in inviscid runs
 //   k_plane            2D: all of the above after the ghost fill in one kernel per stage
 // Every hot kernel body is also reachable through a k_*_batch twin that runs many cases from
 // one launch over a tile work list (shx_batch_*).
@@ -873,9 +873,10 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
 }
 // Waves per SIMD asked of the compiler: the diagonal FP64 W5 sweeps run four (122-128 VGPRs, at most two
 // spilled), which the LDS of an 8 x 32 or 4 x 64 tile allows too; at three waves (132-134 VGPRs) the xi
-// sweep took 0.87 ms at 256^3 against 0.83.  The other variants are left to the compiler.
+// sweep took 0.87 ms at 256^3 against 0.83.  WENO9 and the general metric: three waves (138-168 VGPRs).
+// The mixed form is left to the compiler.
 template <int S, int AX, bool MIX>
-constexpr int weno_min_waves() { return (AX >= 0 && !MIX) ? (S == 5 ? 4 : 3) : 1; }
+constexpr int weno_min_waves() { return MIX ? 1 : (S == 5 && AX >= 0 ? 4 : 3); }
 
 template <int S, int TA, int TDI, int AX, bool MIX>
 __global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, AX, MIX>())) void k_weno(WenoArgs a)
@@ -894,8 +895,8 @@ __global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, AX, MIX>())) void k_we
 // coefficients K = (mu fac)_face averages; energy work term u_i (F(i+1/2) - F(i-1/2)) and the
 // nodal product term are evaluated per node as in the reference.
 // Stage update of one interior node (src/Functions.c:2300-2365) with the manufactured source
-// (Q += J src): shared by k_rk_update and the last viscous sweep of a stage, which applies it
-// directly instead of storing Q.
+// (Q += J src): shared by the last kernels of a stage, which apply it directly
+// instead of storing Q.
 struct RkArgs {
     CFields5 un, us, src;
     Fields5 out, qsum;
@@ -1668,39 +1669,48 @@ __global__ __launch_bounds__(256, (MIX ? 1 : ETA_WAVES)) void k_eta(EtaArgs z)
     eta_body<MIX>(z, bx, by, bz, lds);
 }
 
-// Stage update (src/Functions.c:2300-2365) + manufactured source: pointwise.
-struct UpdArgs {
-    Fields5 q;
-    gcdp J;
-    CFields10 met;        // metric rows, read for the CFL sum of the end-of-step check
-    Geom gm;
+// ---- WENO sweep along the contiguous axis (the last of the three) ------------------------------
+// The inviscid stage's last kernel: the sweep keeps its node's divergence in registers, adds it to Q and
+// applies the stage update (or stores Q, where viscous sweeps follow), instead of a separate pass that
+// read Q back: 128 x 128 x 144 inviscid, sweep and update 138 + 100 us -> 188.
+struct WenoLastArgs {
+    WenoArgs w;
+    CFields10 met;        // J, and the rows for the CFL sum of the end-of-step check
+    int update;
     RkArgs rk;
 };
-
-__device__ __forceinline__ void rk_body(const UpdArgs &A, const long t)
+template <int S, int TA, int TDI, int AX, bool MIX>
+__device__ __forceinline__ void weno_last_body(const WenoLastArgs &z, const int bx, const int by, const int bz, double *lds)
 {
-    const Geom &gm = A.gm;
-    const long nint = (long)gm.n[0] * gm.n[1] * gm.n[2];
-    double cfl = 0.0;
-    if (t < nint) {
-        const int kk = (int)(t % gm.n[2]);
-        const long r = t / gm.n[2];
-        const int jj = (int)(r % gm.n[1]);
-        const int ii = (int)(r / gm.n[1]);
-        const long n = (long)(ii + gm.lo[0]) * gm.st[0] + (long)(jj + gm.lo[1]) * gm.st[1] + kk + gm.lo[2];
-        double qv[5];
+    double keep[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, cfl = 0.0;
+    weno_body<S, TA, TDI, AX, MIX, true>(z.w, bx, by, bz, lds, keep);
+    const WenoArgs &a = z.w;
+    const int ta = threadIdx.x / TDI, di = threadIdx.x % TDI;
+    const int dn = bz * (TDI - 1) + di, pa = (a.alignA ? bx * TA : bx * TA + a.oA) + ta;
+    if (di < TDI - 1 && dn < a.nD && pa >= a.oA && pa < a.oA + a.nA) {
+        const long n = (long)(by + a.oB) * a.sB + (long)pa * a.sA + (long)(dn + a.oD) * a.sD;
+        double q[5];
 #pragma unroll
-        for (int m = 0; m < 5; m++) qv[m] = A.q.f[m][n];
-        double m9[9];
+        for (int m = 0; m < 5; m++) q[m] = (a.first ? 0.0 : a.q.f[m][n]) + keep[m];
+        if (z.update) {
+            double m9[9];
 #pragma unroll
-        for (int c = 0; c < 9; c++) m9[c] = A.rk.cfl_red ? A.met.f[c][n] : 0.0;
-        rk_point(A.rk, n, A.J[n], qv, m9, &cfl);
+            for (int c = 0; c < 9; c++) m9[c] = (z.rk.cfl_red && (AX < 0 || c % 4 == 0)) ? z.met.f[c][n] : 0.0;
+            rk_point<(AX >= 0)>(z.rk, n, z.met.f[9][n], q, m9, &cfl);
+        } else {
+#pragma unroll
+            for (int m = 0; m < 5; m++) a.q.f[m][n] = q[m];
+        }
     }
-    if (A.rk.cfl_red) wave_max_to(A.rk.cfl_red, cfl);
+    if (z.update && z.rk.cfl_red) wave_max_to(z.rk.cfl_red, cfl);
 }
-__global__ __launch_bounds__(256) void k_rk_update(UpdArgs A)
+template <int S, int TA, int TDI, int AX, bool MIX>
+__global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, AX, MIX>())) void k_weno_last(WenoLastArgs z)
 {
-    rk_body(A, (long)blockIdx.x * blockDim.x + threadIdx.x);
+    __shared__ double lds[weno_lds<S, TA, TDI, AX, MIX>()];
+    int bx, by, bz;
+    sweep_tile(blockIdx.x, z.w.tg, bx, by, bz);
+    weno_last_body<S, TA, TDI, AX, MIX>(z, bx, by, bz, lds);
 }
 
 // ---- viscous derivatives ------------------------------------------------------------------
@@ -2272,14 +2282,6 @@ __global__ __launch_bounds__(256) void k_ghost_values_batch(BATCH_PARAMS(GhostVa
     });
 }
 template <bool P>
-__global__ __launch_bounds__(256) void k_rk_batch(BATCH_PARAMS(UpdArgs))
-{
-    batch_walk<P>(total, [&](const int b) {
-        const int4 w = rec(work, b);
-        rk_body(rec(A, w.x), (long)w.y * 256 + threadIdx.x);
-    });
-}
-template <bool P>
 __global__ __launch_bounds__(256) void k_face_batch(BATCH_PARAMS(BcArgs))
 {
     batch_walk<P>(total, [&](const int b) {
@@ -2337,6 +2339,16 @@ __global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, AX, MIX>())) void k_we
     batch_walk<P>(total, [&](const int b) {
         const int4 w = rec(work, b);
         weno_body<S, TA, TDI, AX, MIX>(rec(A, w.x), w.y, w.z, w.w, lds);
+    });
+}
+
+template <int S, int TA, int TDI, int AX, bool MIX, bool P>
+__global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, AX, MIX>())) void k_weno_last_batch(BATCH_PARAMS(WenoLastArgs))
+{
+    __shared__ double lds[weno_lds<S, TA, TDI, AX, MIX>()];
+    batch_walk<P>(total, [&](const int b) {
+        const int4 w = rec(work, b);
+        weno_last_body<S, TA, TDI, AX, MIX>(rec(A, w.x), w.y, w.z, w.w, lds);
     });
 }
 
@@ -3476,6 +3488,12 @@ struct Pick {
 };
 
 template <int S, int TA, int TDI, int AX, bool MIX>
+static Pick weno_last_pick_t()
+{
+    return {(const void *)&k_weno_last<S, TA, TDI, AX, MIX>, (const void *)&k_weno_last_batch<S, TA, TDI, AX, MIX, false>,
+            (const void *)&k_weno_last_batch<S, TA, TDI, AX, MIX, true>, TA, TDI};
+}
+template <int S, int TA, int TDI, int AX, bool MIX>
 static Pick weno_pick_t()
 {
     return {(const void *)&k_weno<S, TA, TDI, AX, MIX>, (const void *)&k_weno_batch<S, TA, TDI, AX, MIX, false>,
@@ -3489,8 +3507,8 @@ template <int S, int TA, int TDI, bool MIX, bool COAL>
 static Pick weno_pick_m(int ax)
 {
     if constexpr (COAL) {
-        if (ax == 2) return weno_pick_t<S, TA, TDI, 2, MIX>();
-        return weno_pick_t<S, TA, TDI, -1, MIX>();
+        if (ax == 2) return weno_last_pick_t<S, TA, TDI, 2, MIX>();
+        return weno_last_pick_t<S, TA, TDI, -1, MIX>();
     } else {
         if (ax == 0) return weno_pick_t<S, TA, TDI, 0, MIX>();
         if (ax == 1) return weno_pick_t<S, TA, TDI, 1, MIX>();
@@ -3582,14 +3600,28 @@ static dim3 flat_grid(const dim3 g, int tg[4], int order)
 // tile order of a sweep (see sweep_tile): along the sweep, except the viscous sweep of the
 // slowest axis
 static int sweep_order(bool visc, int dir) { return (visc && dir == 0) ? 0 : 1; }
-static int weno_sweep(shx_case *c, double *const *pr, int dir, int first)
+// the last direction's record; rk: the stage update (null: Q is stored)
+static WenoLastArgs weno_last_args(const shx_case *c, double *const *pr, int first, const RkArgs *rk)
 {
-    WenoArgs a = weno_args(c, pr, dir, first);
+    WenoLastArgs z;
+    memset(&z, 0, sizeof z);
+    z.w = weno_args(c, pr, 2, first);
+    for (int m = 0; m < 10; m++) z.met.f[m] = c->met[m];
+    z.update = rk ? 1 : 0;
+    if (rk) z.rk = *rk;
+    return z;
+}
+static int weno_sweep(shx_case *c, double *const *pr, int dir, int first, const RkArgs *rk = nullptr)
+{
+    WenoLastArgs z;
+    if (dir == 2) z = weno_last_args(c, pr, first, rk);
+    else z.w = weno_args(c, pr, dir, first);
+    WenoArgs &a = z.w;
     const Pick p = weno_pick(c, dir);
     int rc = tbeg(c, KT_WENO0 + dir);
     if (rc) return rc;
     const dim3 grid = flat_grid(sweep_grid(a.nA, a.oA, a.alignA, a.nB, a.nD, p), a.tg, sweep_order(false, dir));
-    if ((rc = launch_pick(p.single, grid, p.TA * p.TDI, &a, c->stream))) return rc;
+    if ((rc = launch_pick(p.single, grid, p.TA * p.TDI, dir == 2 ? (void *)&z : (void *)&a, c->stream))) return rc;
     return tend(c);
 }
 
@@ -3755,7 +3787,7 @@ static int stage_fluxes(shx_case *c, double *const *pr, const RkArgs *rk, double
     const int nsep = fz ? gm.dims - 1 : gm.dims;
     for (int dir = 0; dir < nsep; dir++) {
         if (fe && dir == 1) continue;
-        if ((rc = weno_sweep(c, pr, dir, dir == 0))) return rc;
+        if ((rc = weno_sweep(c, pr, dir, dir == 0, c->d.inviscid ? rk : nullptr))) return rc;
     }
     if (fx && (rc = grad_march(c, pr, true))) return rc;
     if (!c->d.inviscid)
@@ -3925,24 +3957,6 @@ static RkArgs rk_args(shx_case *c, double *const *us, double *const *out, int s,
     return A;
 }
 
-static int rk_update(shx_case *c, const RkArgs &rk)
-{
-    const Geom &gm = c->gm;
-    const long nint = (long)gm.n[0] * gm.n[1] * gm.n[2];
-    UpdArgs A;
-    memset(&A, 0, sizeof A);
-    for (int m = 0; m < 5; m++) A.q.f[m] = c->q[m];
-    for (int m = 0; m < 10; m++) A.met.f[m] = c->met[m];
-    A.J = c->met[9];
-    A.gm = gm;
-    A.rk = rk;
-    int rc = tbeg(c, KT_RK);
-    if (rc) return rc;
-    k_rk_update<<<nblk(nint, 256), 256, 0, c->stream>>>(A);
-    LAUNCH_CHECK();
-    return tend(c);
-}
-
 static int check_ready(shx_case *c)
 {
     if (!c) return set_err(SHX_ERR_ARG, "null handle");
@@ -3980,11 +3994,8 @@ static int step_stage(shx_case *c, int s, double tau, int flags)
         if (flags & STEP_NAN) { rk.nan_cnt = c->d_nan; rk.nan_flag = &c->h_io->nan_flag; rk.nanP = c->P; }
         if (flags & STEP_CFL) rk.cfl_red = c->d_red;
     }
-    // viscous and 2D stages apply the update in their last kernel; 3D inviscid ones in k_rk_update
-    const bool sep = c->d.inviscid && c->gm.dims == 3;
-    if ((rc = stage_fluxes(c, c->prim[c->st_in], sep ? nullptr : &rk, tau))) return rc;
+    if ((rc = stage_fluxes(c, c->prim[c->st_in], &rk, tau))) return rc;    // its last kernel applies the update
     if ((rc = carry_ghosts(c, c->prim[c->st_in], c->prim[c->st_out]))) return rc;
-    if (sep && (rc = rk_update(c, rk))) return rc;
     c->st_in = c->st_out;
     c->st_out = (c->st_out == c->st_bx) ? c->st_by : c->st_bx;
     return SHX_OK;
@@ -4591,10 +4602,12 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
             std::vector<dim3> grids;
             for (int i = 0; i < nc; i++) {
                 const WenoArgs a = weno_args(g[i], in[i], dir, dir == 0);
-                put(recs, a);
+                if (dir == 2) put(recs, weno_last_args(g[i], in[i], 0, c0->d.inviscid ? &rk[i] : nullptr));
+                else put(recs, a);
                 grids.push_back(sweep_grid(a.nA, a.oA, a.alignA, a.nB, a.nD, p));
             }
-            batch_add(b, p.batch, p.batchp, p.TA * p.TDI, BK_WENO, recs, sizeof(WenoArgs), grids, ORDER_SWEEP);
+            batch_add(b, p.batch, p.batchp, p.TA * p.TDI, BK_WENO, recs, dir == 2 ? sizeof(WenoLastArgs) : sizeof(WenoArgs),
+                      grids, ORDER_SWEEP);
         }
         if (fx) {
             std::vector<char> recs;
@@ -4645,9 +4658,7 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                 grids.push_back(sweep_grid(z.w.nA, z.w.oA, z.w.alignA, z.w.nB, z.w.nD, p));
             }
             batch_add(b, p.batch, p.batchp, p.TA * p.TDI, BK_VISC, zrecs, sizeof(ZetaArgs), grids, ORDER_SWEEP);
-        } else if (dims == 2) {
-            // done
-        } else if (!c0->d.inviscid) {
+        } else if (dims == 3 && !c0->d.inviscid) {
             for (int dir = 0; dir < dims; dir++) {
                 const Pick p = visc_pick(c0, dir);
                 std::vector<char> recs;
@@ -4660,19 +4671,6 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                 batch_add(b, p.batch, p.batchp, p.TA * p.TDI, BK_VISC, recs, sizeof(ViscArgs), grids,
                           sweep_order(true, dir) ? ORDER_SWEEP : ORDER_NODES);
             }
-        } else {
-            std::vector<char> recs;
-            std::vector<dim3> grids;
-            for (int i = 0; i < nc; i++) {
-                shx_case *c = g[i];
-                UpdArgs A;
-                memset(&A, 0, sizeof A);
-                for (int m = 0; m < 5; m++) A.q.f[m] = c->q[m];
-                A.J = c->met[9]; A.gm = c->gm; A.rk = rk[i];
-                put(recs, A);
-                grids.push_back(dim3(nblk((long)c->gm.n[0] * c->gm.n[1] * c->gm.n[2], 256)));
-            }
-            batch_add(b, (const void *)&k_rk_batch<false>, (const void *)&k_rk_batch<true>, 256, BK_RK, recs, sizeof(UpdArgs), grids);
         }
         {   // ghost layers of non-periodic directions into the next stage buffer (ghost nodes only,
             // so the in-place last stage, whose update writes interior nodes of U_n, is unaffected)
