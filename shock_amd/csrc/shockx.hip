@@ -609,6 +609,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     constexpr int NW = WD * TA;
     constexpr int NVK = (AX < 0) ? NV : NV - 3;
     constexpr int VJ = (AX < 0) ? V_J : V_NX;
+    constexpr int NMET = (AX < 0) ? 3 : 1;
     // the FP64 form streams the stencil through registers pair by pair (weno_flux); the mixed form
     // projects one characteristic field at a time
     constexpr bool PAIRS = !MIX;
@@ -637,7 +638,15 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     // the plain node flux.
     auto node_pass = [&](auto wall_c) {
     constexpr bool WALL = decltype(wall_c)::value;
-    for (int idx = t; idx < NW; idx += NT) {
+    constexpr int PER = (NW + NT - 1) / NT;
+    // the loads of all rounds first
+    double in[PER][6 + NMET];
+    long nn[PER];
+    int dpr[PER], op[PER];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int idx = t + r * NT;
+        if (idx >= NW) continue;
         int aa, dd;
         if (a.coalesce_d) { aa = idx / WD; dd = idx - aa * WD; }
         else { dd = idx / TA; aa = idx - dd * TA; }
@@ -648,15 +657,24 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
         // wrap: a ghost node of the stage input is read at its periodic image
         long ns = n;
         if (NT != TA * TDI && a.wrap) ns += (long)(dp < a.oD ? a.nD : (dp >= a.oD + a.nD ? -a.nD : 0)) * a.sD;
-        const double rho = a.pr.f[0][ns], u = a.pr.f[1][ns], v = a.pr.f[2][ns], w = a.pr.f[3][ns],
-                     e = a.pr.f[4][ns];
-        const double J = a.J[n];
+#pragma unroll
+        for (int m = 0; m < 5; m++) in[r][m] = a.pr.f[m][ns];
+        in[r][5] = a.J[n];
+        in[r][6] = a.m0[n];
+        if constexpr (AX < 0) { in[r][7] = a.m1[n]; in[r][8] = a.m2[n]; }
+        nn[r] = n; dpr[r] = dp; op[r] = aa * WD + dd;
+    }
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        if (t + r * NT >= NW) continue;
+        const long n = nn[r];
+        const int dp = dpr[r], o = op[r];
+        const double rho = in[r][0], u = in[r][1], v = in[r][2], w = in[r][3], e = in[r][4], J = in[r][5];
         double p = pressure_fast(k, rho, u, v, w, e);
         const double ir = frcp(rho);
         double cs = sqrt(k.upsilon * k.gamma * p * ir);
         if ((a.pc_lo && dp < a.oD) || (a.pc_hi && dp >= a.oD + a.nD)) { p = a.P[n]; cs = a.C[n]; }
         const double pu = p * k.upsilon;
-        const int o = aa * WD + dd;
         // velocities of the convective momentum terms: times the wall corrector (+-1, exact) on
         // the ghost nodes of a wall face of this direction, the velocities themselves elsewhere
         double uc[3] = {u, v, w};
@@ -668,7 +686,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
             }
         }
         if constexpr (AX < 0) {
-            const double mx = a.m0[n], my = a.m1[n], mz = a.m2[n];
+            const double mx = in[r][6], my = in[r][7], mz = in[r][8];
             const double th = u * mx + v * my + w * mz;
             const double rt = rho * th;
             sm[V_F0 * NW + o] = J * rt;
@@ -683,7 +701,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
             sm[V_NY * NW + o] = my * imn;
             sm[V_NZ * NW + o] = mz * imn;
         } else {
-            const double md = a.m0[n];
+            const double md = in[r][6];
             const double uu[3] = {u, v, w};
             const double th = uu[AX] * md;
             const double rt = rho * th;
