@@ -1622,38 +1622,37 @@ __global__ __launch_bounds__(TA * TDI) void k_visc_sweep(ViscArgs a)
 }
 
 // ---- fused zeta direction: WENO and viscous sweeps and the stage update ----------------------
-// One block sweeps a 4 x 64 tile along zeta twice.  The WENO phase keeps each node's inviscid
+// One block sweeps a 4 x 64 tile (or 8 x 32, zeta_tile) along zeta twice.  The WENO phase keeps each node's inviscid
 // divergence in registers; after a barrier the viscous phase reloads its window into the same LDS,
 // adds that divergence and its own terms to Q and applies the stage update (or stores Q).  Q of
 // this direction is read once instead of read-written by two kernels, and blocks in their WENO
 // phase (VALU-bound) overlap blocks in their viscous phase (memory-bound).  Used for 3D cases with
-// the diagonal metric whose zeta WENO tile is 4 x 64 (the viscous zeta tile), viscous runs only.
+// the diagonal metric, viscous runs only.
 struct ZetaArgs { WenoArgs w; ViscArgs v; };
-template <int S, bool MIX>
+template <int S, int TA, int TDI, bool MIX>
 constexpr int zeta_lds()
 {
-    return weno_lds<S, 4, 64, 2, MIX>() > visc_lds<S, 2, 4, 64, true>() ? weno_lds<S, 4, 64, 2, MIX>()
-                                                                       : visc_lds<S, 2, 4, 64, true>();
+    return std::max(weno_lds<S, TA, TDI, 2, MIX>(), visc_lds<S, 2, TA, TDI, true>());
 }
-template <int S, bool MIX>
+template <int S, int TA, int TDI, bool MIX>
 __device__ __forceinline__ void zeta_body(const ZetaArgs &z, const int bx, const int by, const int bz, double *lds)
 {
     double inv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    weno_body<S, 4, 64, 2, MIX, true>(z.w, bx, by, bz, lds, inv);
+    weno_body<S, TA, TDI, 2, MIX, true>(z.w, bx, by, bz, lds, inv);
     __syncthreads();
     // Q, U_n and Q_sum loaded ahead (measured at 256^3: 1.95 -> 1.75 ms; the same in the fused eta
     // kernel, which stores Q instead of updating the stage, made it slower)
-    visc_diag_body<S, 2, 4, 64, true, true>(z.v, bx, by, bz, lds, inv);
+    visc_diag_body<S, 2, TA, TDI, true, true>(z.v, bx, by, bz, lds, inv);
 }
 // FP64 W5: held to 128 VGPRs (four waves per SIMD, as the LDS allows): 1.55 ms at 256^3 against
 // 1.67 at three waves
-template <int S, bool MIX>
-__global__ __launch_bounds__(256, (weno_min_waves<S, 2, MIX>())) void k_zeta(ZetaArgs z)
+template <int S, int TA, int TDI, bool MIX>
+__global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, 2, MIX>())) void k_zeta(ZetaArgs z)
 {
-    __shared__ double lds[zeta_lds<S, MIX>()];
+    __shared__ double lds[zeta_lds<S, TA, TDI, MIX>()];
     int bx, by, bz;
     sweep_tile(blockIdx.x, z.w.tg, bx, by, bz);
-    zeta_body<S, MIX>(z, bx, by, bz, lds);
+    zeta_body<S, TA, TDI, MIX>(z, bx, by, bz, lds);
 }
 
 // ---- fused eta direction: WENO and viscous eta sweeps in one kernel ----------------------------
@@ -2379,13 +2378,13 @@ __global__ __launch_bounds__(TA * TDI) void k_visc_batch(BATCH_PARAMS(ViscArgs))
         visc_body<S, DIR, TA, TDI, DIAG>(rec(A, w.x), w.y, w.z, w.w, lds);
     });
 }
-template <int S, bool MIX, bool P>
-__global__ __launch_bounds__(256, (weno_min_waves<S, 2, MIX>())) void k_zeta_batch(BATCH_PARAMS(ZetaArgs))
+template <int S, int TA, int TDI, bool MIX, bool P>
+__global__ __launch_bounds__(TA * TDI, (weno_min_waves<S, 2, MIX>())) void k_zeta_batch(BATCH_PARAMS(ZetaArgs))
 {
-    __shared__ double lds[zeta_lds<S, MIX>()];
+    __shared__ double lds[zeta_lds<S, TA, TDI, MIX>()];
     batch_walk<P>(total, [&](const int b) {
         const int4 w = rec(work, b);
-        zeta_body<S, MIX>(rec(A, w.x), w.y, w.z, w.w, lds);
+        zeta_body<S, TA, TDI, MIX>(rec(A, w.x), w.y, w.z, w.w, lds);
     });
 }
 
@@ -2869,7 +2868,7 @@ struct shx_case {
     int needs_bs;          // some face is SHX_BC_MANUFACTURED
     int diag;              // 3D metric is diagonal (only xi_x, eta_y, zeta_z and J non-zero)
     int flat;              // 2D: xi_z and eta_z are zero
-    int wtile[3];          // WENO tile variant per direction (set by shx_tune)
+    int wtile[3];          // WENO tile variant per direction (set by shx_tune; -1: by zeta_tile)
     unsigned long long *d_red;
     int *d_cnt;
     int *d_nan;            // running count of the fused checkNAN (shx_run, shx_run_cfl, shx_simulate)
@@ -3083,14 +3082,14 @@ extern "C" int shx_create(const shx_desc *desc, shx_case **out)
     if (e == hipSuccess) { memset(c->h_io, 0, sizeof(shx_case::HostIo)); e = hipStreamSynchronize(c->stream); }
     if (e != hipSuccess) { shx_destroy(c); return set_err(SHX_ERR_HIP, "setup: %s", hipGetErrorString(e)); }
     c->cur = 0;
-    // WENO tiles until shx_tune times them: 4 x 64 along the contiguous axis and 16 x 16 across it, but
+    // WENO tiles until shx_tune times them: by zeta_tile along the contiguous axis; 16 x 16 across it, but
     // 8 x 32 across it for the diagonal metric where the sweep is not the FP64 WENO9 one: that window
     // holds 1.19 nodes per interface node against 1.40, and its LDS lets a fourth block on a CU (256^3:
     // xi sweep 0.89 -> 0.82 ms FP64, 0.93 -> 0.81 mixed; 144 x 112 x 128 mixed WENO9: 224 -> 172 and
     // 247 -> 188 us).  FP64 WENO9 and the general metric run three blocks either way and lose on eta
     // (176 x 128 x 136 WENO9 326 -> 352 us, 119 x 96 x 104 general 79 -> 87).
     const bool wide = gm.dims == 3 && (d.quirks & SHX_QUIRK_METRIC_DIAG3D) && (S == 5 || d.precision == SHX_MIXED);
-    for (int dir = 0; dir < 3; dir++) c->wtile[dir] = (wide && gm.st[dir] != 1) ? 1 : 0;
+    for (int dir = 0; dir < 3; dir++) c->wtile[dir] = (gm.st[dir] == 1) ? -1 : (wide ? 1 : 0);
     *out = c;
     return SHX_OK;
 }
@@ -3518,7 +3517,7 @@ static Pick weno_pick_t()
             (const void *)&k_weno_batch<S, TA, TDI, AX, MIX, true>, TA, TDI};
 }
 // tile variants of the WENO sweeps (TA transverse x TDI along the sweep), chosen per case and
-// direction by shx_tune: sweeps along the contiguous axis 4 x 64 or 2 x 128, the others 16 x 16
+// direction by shx_tune: sweeps along the contiguous axis 4 x 64 or 8 x 32, the others 16 x 16
 // or 8 x 32.  Diagonal metrics only ever use AX = 2 on the contiguous axis and 0 or 1 otherwise.
 constexpr int NWTILE = 2;
 template <int S, int TA, int TDI, bool MIX, bool COAL>
@@ -3541,16 +3540,31 @@ static Pick weno_pick_s(int ax, bool mix)
 template <int S>
 static Pick weno_pick_v(bool coalesce, int variant, int ax, bool mix)
 {
-    if (coalesce) return variant ? weno_pick_s<S, 2, 128, true>(ax, mix) : weno_pick_s<S, 4, 64, true>(ax, mix);
+    if (coalesce) return variant ? weno_pick_s<S, 8, 32, true>(ax, mix) : weno_pick_s<S, 4, 64, true>(ax, mix);
     return variant ? weno_pick_s<S, 8, 32, false>(ax, mix) : weno_pick_s<S, 16, 16, false>(ax, mix);
 }
-static Pick weno_pick(const shx_case *c, int dir)
+// Tile along the contiguous axis for a launch over nc cases: 0 = 4 x 64, 1 = 8 x 32.  A row of 64 threads
+// covers 63 nodes and one of 32 covers 31, so the last tile of a row can be nearly empty: 8 x 32 where it
+// takes fewer than 7/8 of the threads.  128 x 128 x 144 inviscid (0.83 of them) 184 -> 161 us, WENO9
+// viscous 176 x 128 x 136 (0.83) 525 -> 456, mixed 144 x 112 x 128 (0.83) 315 -> 299; its shorter rows read
+// more halo, 256^3 WENO5 (0.90) 1.50 -> 1.53 ms, and at equal threads 97 x 85 x 106 WENO9 133 -> 136 us.
+static int zeta_tile(const shx_case *const *g, const int nc)
+{
+    if (g[0]->wtile[2] >= 0) return g[0]->wtile[2];
+    long wide = 0, narrow = 0;
+    for (int i = 0; i < nc; i++) {
+        const Geom &gm = g[i]->gm;
+        wide += gm.n[0] * (long)nblk(gm.n[1], 4) * nblk(gm.n[2], 63);
+        narrow += gm.n[0] * (long)nblk(gm.n[1], 8) * nblk(gm.n[2], 31);
+    }
+    return 8 * narrow < 7 * wide ? 1 : 0;
+}
+static Pick weno_pick(const shx_case *c, int dir, const int v)
 {
     const bool diag = (c->diag && c->gm.dims == 3);
     const bool mix = (c->d.precision == SHX_MIXED);
     const bool coalesce = (c->gm.st[dir] == 1);
     const int ax = diag ? dir : -1;
-    const int v = c->wtile[dir];
     return (c->d.space_order == 5) ? weno_pick_v<5>(coalesce, v, ax, mix) : weno_pick_v<9>(coalesce, v, ax, mix);
 }
 
@@ -3635,7 +3649,7 @@ static int weno_sweep(shx_case *c, double *const *pr, int dir, int first, const 
     if (dir == 2) z = weno_last_args(c, pr, first, rk);
     else z.w = weno_args(c, pr, dir, first);
     WenoArgs &a = z.w;
-    const Pick p = weno_pick(c, dir);
+    const Pick p = weno_pick(c, dir, dir == 2 ? zeta_tile(&c, 1) : c->wtile[dir]);
     int rc = tbeg(c, KT_WENO0 + dir);
     if (rc) return rc;
     const dim3 grid = flat_grid(sweep_grid(a.nA, a.oA, a.alignA, a.nB, a.nD, p), a.tg, sweep_order(false, dir));
@@ -3651,7 +3665,7 @@ static int zeta_sweep(shx_case *c, double *const *pr, const RkArgs *rk);
 // the zeta direction runs as one fused kernel (k_zeta)
 static bool fuse_zeta(const shx_case *c)
 {
-    return c->gm.dims == 3 && c->diag && !c->d.inviscid && c->wtile[2] == 0;
+    return c->gm.dims == 3 && c->diag && !c->d.inviscid;
 }
 // the viscous xi direction rides on the derivative march (k_visc_grad_march_xi; WENO5 order, whose
 // rings fit the march's registers)
@@ -3900,17 +3914,19 @@ static int visc_sweep(shx_case *c, double *const *pr, int dir, const RkArgs *rk)
     if ((rc = launch_pick(p.single, grid, p.TA * p.TDI, &a, c->stream))) return rc;
     return tend(c);
 }
-template <int S, bool MIX>
-static Pick zeta_pick_t()
+template <int S, int TA, int TDI>
+static Pick zeta_pick_t(const bool mix)
 {
-    return {(const void *)&k_zeta<S, MIX>, (const void *)&k_zeta_batch<S, MIX, false>,
-            (const void *)&k_zeta_batch<S, MIX, true>, 4, 64};
+    if (mix) return {(const void *)&k_zeta<S, TA, TDI, true>, (const void *)&k_zeta_batch<S, TA, TDI, true, false>,
+                     (const void *)&k_zeta_batch<S, TA, TDI, true, true>, TA, TDI};
+    return {(const void *)&k_zeta<S, TA, TDI, false>, (const void *)&k_zeta_batch<S, TA, TDI, false, false>,
+            (const void *)&k_zeta_batch<S, TA, TDI, false, true>, TA, TDI};
 }
-static Pick zeta_pick(const shx_case *c)
+static Pick zeta_pick(const shx_case *c, const int variant)
 {
     const bool mix = (c->d.precision == SHX_MIXED);
-    if (c->d.space_order == 5) return mix ? zeta_pick_t<5, true>() : zeta_pick_t<5, false>();
-    return mix ? zeta_pick_t<9, true>() : zeta_pick_t<9, false>();
+    if (c->d.space_order == 5) return variant ? zeta_pick_t<5, 8, 32>(mix) : zeta_pick_t<5, 4, 64>(mix);
+    return variant ? zeta_pick_t<9, 8, 32>(mix) : zeta_pick_t<9, 4, 64>(mix);
 }
 static ZetaArgs zeta_args(const shx_case *c, double *const *pr, const RkArgs *rk)
 {
@@ -3922,7 +3938,7 @@ static ZetaArgs zeta_args(const shx_case *c, double *const *pr, const RkArgs *rk
 static int zeta_sweep(shx_case *c, double *const *pr, const RkArgs *rk)
 {
     ZetaArgs z = zeta_args(c, pr, rk);
-    const Pick p = zeta_pick(c);
+    const Pick p = zeta_pick(c, zeta_tile(&c, 1));
     int rc = tbeg(c, KT_ZETA);
     if (rc) return rc;
     const dim3 grid = flat_grid(sweep_grid(z.w.nA, z.w.oA, z.w.alignA, z.w.nB, z.w.nD, p), z.w.tg, 1);
@@ -4615,7 +4631,7 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
         const int nsep = dims == 2 ? 0 : (fz ? dims - 1 : dims);
         for (int dir = 0; dir < nsep; dir++) {
             if (fe && dir == 1) continue;
-            const Pick p = weno_pick(c0, dir);
+            const Pick p = weno_pick(c0, dir, dir == 2 ? zeta_tile(g.data(), nc) : c0->wtile[dir]);
             std::vector<char> recs;
             std::vector<dim3> grids;
             for (int i = 0; i < nc; i++) {
@@ -4641,7 +4657,7 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                       BK_GRAD, recs, sizeof(GradArgs), grids, ORDER_NODES);
         }
         if (fz) {
-            const Pick p = zeta_pick(c0);
+            const Pick p = zeta_pick(c0, zeta_tile(g.data(), nc));
             std::vector<char> zrecs;
             std::vector<dim3> grids;
             // viscous xi (unless the march took it) and eta (or the fused eta kernel), then the
@@ -5044,7 +5060,7 @@ extern "C" int shx_tune(shx_case *c, int reps, int choice[3])
     double *const *pr = c->prim[c->cur];
     if (c->gm.dims == 2) {            // 2D stages run on k_plane's tile
         if (choice)
-            for (int d = 0; d < 3; d++) choice[d] = c->wtile[d];
+            for (int d = 0; d < 3; d++) choice[d] = std::max(c->wtile[d], 0);
         return SHX_OK;
     }
     if ((rc = ghost_fill(c, pr, 5))) return rc;
@@ -5052,8 +5068,7 @@ extern "C" int shx_tune(shx_case *c, int reps, int choice[3])
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     for (int dir = 0; dir < c->gm.dims && !rc; dir++) {
-        // the zeta sweep of a fusable case stays on the 4 x 64 tile of the fused kernel (k_zeta)
-        if (dir == 2 && c->gm.dims == 3 && c->diag && !c->d.inviscid) { c->wtile[2] = 0; continue; }
+        if (dir == 2 && fuse_zeta(c)) continue;      // the fused kernel's tile stays by zeta_tile
         if (dir == 1 && fuse_eta(c)) { c->wtile[1] = 1; continue; }   // the fused eta kernel's 8 x 32 tile
         float best = 1e30f;
         int bestv = 0;
@@ -5074,7 +5089,7 @@ extern "C" int shx_tune(shx_case *c, int reps, int choice[3])
     hipEventDestroy(e1);
     if (rc) return rc;
     if (choice)
-        for (int d = 0; d < 3; d++) choice[d] = c->wtile[d];
+        for (int d = 0; d < 3; d++) choice[d] = (d == 2) ? zeta_tile(&c, 1) : c->wtile[d];
     if (c->timing) drain_events(c);
     return SHX_OK;
 }
