@@ -433,7 +433,7 @@ struct WenoArgs {
     int first;            // 1: Q = -div (first direction of the stage), 0: Q -= div
     int coalesce_d;       // load mapping: 1 when the sweep axis is contiguous in memory
     int alignA;           // tiles start at padded A index 0 (A axis contiguous, pitch padded)
-    int wrap;             // the stage input's ghosts are read at their periodic image (2D tiles)
+    int wrap;             // the stage input's ghosts are read at their periodic image (state_wraps)
     Consts k;
 };
 
@@ -639,7 +639,8 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
     auto node_pass = [&](auto wall_c) {
     constexpr bool WALL = decltype(wall_c)::value;
     constexpr int PER = (NW + NT - 1) / NT;
-    // the loads of all rounds first
+    // the loads of all rounds first: the last round is one wavefront's, and the others wait for it at the
+    // barrier (256^3, k_zeta 1.57 -> 1.50 ms FP64, 1.64 -> 1.53 mixed)
     double in[PER][6 + NMET];
     long nn[PER];
     int dpr[PER], op[PER];
@@ -656,7 +657,7 @@ __device__ __forceinline__ void weno_body(const WenoArgs &a, const int bx, const
         const long n = bbase + (long)pa * a.sA + (long)dp * a.sD;
         // wrap: a ghost node of the stage input is read at its periodic image
         long ns = n;
-        if (NT != TA * TDI && a.wrap) ns += (long)(dp < a.oD ? a.nD : (dp >= a.oD + a.nD ? -a.nD : 0)) * a.sD;
+        if (a.wrap) ns += (long)(dp < a.oD ? a.nD : (dp >= a.oD + a.nD ? -a.nD : 0)) * a.sD;
 #pragma unroll
         for (int m = 0; m < 5; m++) in[r][m] = a.pr.f[m][ns];
         in[r][5] = a.J[n];
@@ -3578,7 +3579,14 @@ static void sweep_axes(const Geom &gm, int dir, int &A, int &B)
     }
 }
 
-static WenoArgs weno_args(const shx_case *c, double *const *pr, int dir, int first)
+// The stages of an all-periodic 2D or inviscid case read ghosts at their image instead of filling them
+// first (stored p and c need the fill's pass): 128 x 128 x 144 inviscid, a fill of 25 us beside sweeps of
+// 444.  The viscous sweeps of a 3D case read ghosts of nodal derivatives too, which the march forms there.
+static bool state_wraps(const shx_case *c)
+{
+    return (c->gm.dims == 2 || c->d.inviscid) && !c->faces && !c->pc;
+}
+static WenoArgs weno_args(const shx_case *c, double *const *pr, int dir, int first, const bool wrap = false)
 {
     const Geom &gm = c->gm;
     WenoArgs a;
@@ -3595,6 +3603,7 @@ static WenoArgs weno_args(const shx_case *c, double *const *pr, int dir, int fir
     a.oD = gm.lo[dir]; a.oA = gm.lo[A]; a.oB = gm.lo[B];
     a.ngD = gm.ng[dir];
     a.first = first;
+    a.wrap = wrap ? 1 : 0;
     a.coalesce_d = (a.sD == 1);
     a.alignA = (a.sA == 1);
     a.P = c->P; a.C = c->C;
@@ -3633,11 +3642,11 @@ static dim3 flat_grid(const dim3 g, int tg[4], int order)
 // slowest axis
 static int sweep_order(bool visc, int dir) { return (visc && dir == 0) ? 0 : 1; }
 // the last direction's record; rk: the stage update (null: Q is stored)
-static WenoLastArgs weno_last_args(const shx_case *c, double *const *pr, int first, const RkArgs *rk)
+static WenoLastArgs weno_last_args(const shx_case *c, double *const *pr, int first, const RkArgs *rk, const bool wrap)
 {
     WenoLastArgs z;
     memset(&z, 0, sizeof z);
-    z.w = weno_args(c, pr, 2, first);
+    z.w = weno_args(c, pr, 2, first, wrap);
     for (int m = 0; m < 10; m++) z.met.f[m] = c->met[m];
     z.update = rk ? 1 : 0;
     if (rk) z.rk = *rk;
@@ -3646,8 +3655,9 @@ static WenoLastArgs weno_last_args(const shx_case *c, double *const *pr, int fir
 static int weno_sweep(shx_case *c, double *const *pr, int dir, int first, const RkArgs *rk = nullptr)
 {
     WenoLastArgs z;
-    if (dir == 2) z = weno_last_args(c, pr, first, rk);
-    else z.w = weno_args(c, pr, dir, first);
+    const bool wrap = rk && state_wraps(c);      // (a residual alone: ghosts filled)
+    if (dir == 2) z = weno_last_args(c, pr, first, rk, wrap);
+    else z.w = weno_args(c, pr, dir, first, wrap);
     WenoArgs &a = z.w;
     const Pick p = weno_pick(c, dir, dir == 2 ? zeta_tile(&c, 1) : c->wtile[dir]);
     int rc = tbeg(c, KT_WENO0 + dir);
@@ -3741,8 +3751,6 @@ static int grad_march(shx_case *c, double *const *pr, const bool xi)
 static int eta_sweep(shx_case *c, double *const *pr);
 
 // ---- 2D stages: one k_plane launch (after the ghost fill and the face writers, where the case has them)
-// the stages of an all-periodic case read ghosts at their image; stored p and c need the fill's pass
-static bool plane_wraps(const shx_case *c) { return c->gm.dims == 2 && !c->faces && !c->pc; }
 static Pick plane_pick(const shx_case *c)
 {
     const bool mix = (c->d.precision == SHX_MIXED);
@@ -3759,9 +3767,8 @@ static PlaneArgs plane_args(const shx_case *c, double *const *pr, const RkArgs *
     PlaneArgs z;
     memset(&z, 0, sizeof z);
     for (int d = 0; d < 2; d++) {
-        z.w[d] = weno_args(c, pr, d, 1);
+        z.w[d] = weno_args(c, pr, d, 1, wrap);
         z.w[d].alignA = 0;
-        z.w[d].wrap = wrap ? 1 : 0;
         z.ng[d] = gm.ng[d]; z.lo[d] = gm.lo[d];
         z.nt[d] = (int)nblk(gm.n[d], PT);
         z.iso_hi[d] = (c->d.bc[2 * d + 1] == SHX_BC_WALL_ISOTHERMAL) ? 1 : 0;
@@ -3791,8 +3798,10 @@ static int stage_fluxes(shx_case *c, double *const *pr, const RkArgs *rk, double
     const Geom &gm = c->gm;
     int rc;
     // a caller of the residual alone finds the ghosts of its state filled, as always
-    if (rk && plane_wraps(c)) return plane_stage(c, pr, rk, true);
-    if (c->d.inviscid && !c->pc) {
+    const bool wrap = rk && state_wraps(c);
+    if (wrap && gm.dims == 2) return plane_stage(c, pr, rk, true);
+    if (wrap) {
+    } else if (c->d.inviscid && !c->pc) {
         if ((rc = ghost_fill(c, pr, 5))) return rc;
     } else {
         // periodic ghosts, then T and mu (viscous) and the stored p and c (subsonic outflow faces)
@@ -4532,9 +4541,9 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                 if (any) batch_add(b, (const void *)&k_face_save_batch<false>, (const void *)&k_face_save_batch<true>, 256, BK_GHOST, recs, sizeof(BcArgs), grids);
             }
         }
-        // 2D cases that read ghosts at their image need none filled, but the state keeps those of the
+        // cases that read ghosts at their image need none filled, but the state keeps those of the
         // step's start, as it always has in a batch
-        auto fills = [&](const shx_case *c) { return s == 0 || !plane_wraps(c); };
+        auto fills = [&](const shx_case *c) { return s == 0 || !state_wraps(c); };
         if (c0->d.inviscid) {   // periodic ghost fill of the stage input
             std::vector<char> recs;
             std::vector<dim3> grids;
@@ -4620,7 +4629,7 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
             std::vector<char> recs;
             std::vector<dim3> grids;
             for (int i = 0; i < nc; i++) {
-                const PlaneArgs z = plane_args(g[i], in[i], &rk[i], plane_wraps(g[i]));
+                const PlaneArgs z = plane_args(g[i], in[i], &rk[i], state_wraps(g[i]));
                 put(recs, z);
                 grids.push_back(dim3(z.nt[0] * z.nt[1]));
             }
@@ -4635,8 +4644,9 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
             std::vector<char> recs;
             std::vector<dim3> grids;
             for (int i = 0; i < nc; i++) {
-                const WenoArgs a = weno_args(g[i], in[i], dir, dir == 0);
-                if (dir == 2) put(recs, weno_last_args(g[i], in[i], 0, c0->d.inviscid ? &rk[i] : nullptr));
+                const bool wrap = state_wraps(g[i]);
+                const WenoArgs a = weno_args(g[i], in[i], dir, dir == 0, wrap);
+                if (dir == 2) put(recs, weno_last_args(g[i], in[i], 0, c0->d.inviscid ? &rk[i] : nullptr, wrap));
                 else put(recs, a);
                 grids.push_back(sweep_grid(a.nA, a.oA, a.alignA, a.nB, a.nD, p));
             }
@@ -5198,7 +5208,7 @@ static int sync_ghosts(shx_case *c)
     CFields5 a;
     Fields5 b;
     for (int m = 0; m < 5; m++) { a.f[m] = c->prim[c->last_in][m]; b.f[m] = c->prim[c->cur][m]; }
-    k_copy_ghosts<<<nblk(c->gm.ntot, 256), 256, 0, c->stream>>>(a, b, c->gm, (c->gm.dims == 2 && !c->faces) ? 1 : 0);
+    k_copy_ghosts<<<nblk(c->gm.ntot, 256), 256, 0, c->stream>>>(a, b, c->gm, ((c->gm.dims == 2 || c->d.inviscid) && !c->faces) ? 1 : 0);
     LAUNCH_CHECK();
     c->last_in = -1;
     return SHX_OK;
