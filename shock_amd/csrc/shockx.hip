@@ -2132,6 +2132,52 @@ __device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, d
     const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), t = threadIdx.x & 255;
     const int ti = tile / z.nt[1], tj = tile - ti * z.nt[1];
     const int ta = min(t / (PT + 1), PT - 1), di = t % (PT + 1);
+    const Consts &k = z.w[0].k;
+    const int i0 = z.lo[0] + ti * PT, j0 = z.lo[1] + tj * PT;    // padded index of the tile's first node
+    // The update's U_n and Q_sum and, for WENO5, the viscous window are loaded before the WENO sweeps: one
+    // block per CU has nothing else to overlap those loads with.  64^2 WENO5 18.8 -> 17.6 us a stage, 1000 x
+    // 768 207 -> 190, 211 x 157 WENO9 27.0 -> 25.6 (with its
+    // window as well 25.1, but 43 spilled registers in a batch).
+    constexpr int PER = (RN + 511) / 512;
+    double in[PER][12];
+    auto region = [&](const int idx, int &li, int &lj) {
+        li = idx / WD; lj = idx - li * WD;
+        return li >= G - 1 && li <= G + PT && lj >= G - 1 && lj <= G + PT;    // holds metric and mu
+    };
+    auto load_window = [&]() {
+        const WenoArgs &wx = z.w[0], &wy = z.w[1];
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            const int idx = threadIdx.x + r * 512;
+            if (idx >= RN) continue;
+            int li, lj;
+            const bool ring = region(idx, li, lj);
+            const int i = min(i0 - G + li, z.ng[0] - 1), j = min(j0 - G + lj, z.ng[1] - 1);
+            const long n = (long)i * z.st + j;
+            long ns = n;
+            if (z.wrap) {
+                ns += (long)(i < wx.oD ? wx.nD : (i >= wx.oD + wx.nD ? -wx.nD : 0)) * z.st;
+                ns += (j < wy.oD ? wy.nD : (j >= wy.oD + wy.nD ? -wy.nD : 0));
+            }
+            in[r][0] = wx.pr.f[1][ns]; in[r][1] = wx.pr.f[2][ns]; in[r][2] = wx.pr.f[3][ns];
+            if (z.wrap) {
+                in[r][3] = wx.pr.f[0][ns]; in[r][4] = wx.pr.f[4][ns];
+            } else {
+                in[r][3] = z.T[n];
+                if (ring) in[r][4] = z.mu[n];
+            }
+            if (ring) {
+                in[r][5] = z.met.f[0][n]; in[r][6] = z.met.f[1][n]; in[r][7] = z.met.f[3][n]; in[r][8] = z.met.f[4][n];
+                in[r][9] = z.met.f[9][n];
+                if (!z.flat) { in[r][10] = z.met.f[2][n]; in[r][11] = z.met.f[5][n]; }
+            }
+        }
+    };
+    if (S == 5 && z.visc) load_window();
+    const int ni = i0 + (int)threadIdx.x / PT, nj = j0 + (int)threadIdx.x % PT;
+    const bool own = threadIdx.x < NN && ni < z.w[0].oD + z.w[0].nD && nj < z.w[1].oD + z.w[1].nD;
+    RkPre pre;
+    if (z.update && own) rk_preload(z.rk, (long)ni * z.st + nj, pre);
     double keep[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     weno_body<S, PT, PT + 1, -1, MIX, true, 256>(z.w[half], half ? ti : tj, 0, half ? tj : ti, lds + half * WL, keep);
     __syncthreads();
@@ -2142,36 +2188,24 @@ __device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, d
 #pragma unroll
         for (int m = 0; m < 5; m++) QW[(half * 5 + m) * NN + node] = keep[m];
     }
-    const Consts &k = z.w[0].k;
-    const int i0 = z.lo[0] + ti * PT, j0 = z.lo[1] + tj * PT;    // padded index of the tile's first node
     if (z.visc) {
-        const WenoArgs &wx = z.w[0], &wy = z.w[1];
-        for (int idx = threadIdx.x; idx < RN; idx += 512) {
-            const int li = idx / WD, lj = idx - li * WD;
-            const int i = min(i0 - G + li, z.ng[0] - 1), j = min(j0 - G + lj, z.ng[1] - 1);
-            const long n = (long)i * z.st + j;
-            const bool ring = li >= G - 1 && li <= G + PT && lj >= G - 1 && lj <= G + PT;
-            long ns = n;
-            if (z.wrap) {
-                ns += (long)(i < wx.oD ? wx.nD : (i >= wx.oD + wx.nD ? -wx.nD : 0)) * z.st;
-                ns += (j < wy.oD ? wy.nD : (j >= wy.oD + wy.nD ? -wy.nD : 0));
-            }
-            const double u = wx.pr.f[1][ns], v = wx.pr.f[2][ns], w = wx.pr.f[3][ns];
-            double T, mu = 0.0;
-            if (z.wrap) {
-                const double rho = wx.pr.f[0][ns];
-                node_tmu(k, pressure(k, rho, u, v, w, wx.pr.f[4][ns]), rho, T, mu);
-            } else {
-                T = z.T[n];
-                if (ring) mu = z.mu[n];
-            }
+        if (S != 5) load_window();
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            const int idx = threadIdx.x + r * 512;
+            if (idx >= RN) continue;
+            int li, lj;
+            const bool ring = region(idx, li, lj);
+            const double u = in[r][0], v = in[r][1], w = in[r][2];
+            double T = in[r][3], mu = in[r][4];
+            if (z.wrap) node_tmu(k, pressure(k, in[r][3], u, v, w, in[r][4]), in[r][3], T, mu);
             UV[idx] = u; UV[RN + idx] = v; UV[2 * RN + idx] = w; UV[3 * RN + idx] = T;
             if (ring) {
                 double *const M = MM + (li - G + 1) * RING + lj - G + 1;
-                M[0] = z.met.f[0][n]; M[NR] = z.met.f[1][n]; M[2 * NR] = z.met.f[3][n]; M[3 * NR] = z.met.f[4][n];
-                M[4 * NR] = z.met.f[9][n];
+#pragma unroll
+                for (int c = 0; c < 5; c++) M[c * NR] = in[r][5 + c];
                 M[5 * NR] = mu;
-                if (!z.flat) { M[6 * NR] = z.met.f[2][n]; M[7 * NR] = z.met.f[5][n]; }
+                if (!z.flat) { M[6 * NR] = in[r][10]; M[7 * NR] = in[r][11]; }
             }
         }
         __syncthreads();
@@ -2201,10 +2235,10 @@ __device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, d
     }
     __syncthreads();
     double cflv = 0.0;
-    if (threadIdx.x < NN) {
-        const int node = threadIdx.x, i = i0 + node / PT, j = j0 + node % PT;
-        if (i < z.w[0].oD + z.w[0].nD && j < z.w[1].oD + z.w[1].nD) {
-            const long n = (long)i * z.st + j;
+    {
+        const int node = threadIdx.x;
+        if (own) {
+            const long n = (long)ni * z.st + nj;
             double q[5];
 #pragma unroll
             for (int m = 0; m < 5; m++) q[m] = QW[m * NN + node] + QW[(5 + m) * NN + node];
@@ -2220,7 +2254,7 @@ __device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, d
                 double m9[9];
 #pragma unroll
                 for (int c = 0; c < 9; c++) m9[c] = z.rk.cfl_red ? z.met.f[c][n] : 0.0;
-                rk_point(z.rk, n, z.met.f[9][n], q, m9, &cflv);
+                rk_point(z.rk, n, z.met.f[9][n], q, m9, &cflv, &pre);
             } else {
 #pragma unroll
                 for (int m = 0; m < 5; m++) z.w[0].q.f[m][n] = q[m];
