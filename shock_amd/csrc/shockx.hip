@@ -2,7 +2,8 @@
 //
 // Stage pipeline (one RK stage; src/Functions.c:2107-2365):
 //   k_ghost_periodic   on-device ghost fill of rho,u,v,w,e along periodic directions (replaces
-//                      the MPI self-interface halo, src/Functions.c:3580-3684)
+//                      the MPI self-interface halo, src/Functions.c:3580-3684); all-periodic inviscid
+//                      sweeps read ghosts at their image instead
 //   k_calc_values      T and mu on every padded node (CalcValues, src/Functions.c:2392-2481;
 //                      p, c and theta are recomputed inside the flux kernels instead of stored)
 //   k_face_bc          boundary writers of non-periodic faces, in face order (src/BC.c:13-74)
@@ -2007,9 +2008,9 @@ __global__ __launch_bounds__(GKX * GJX) void k_visc_grad_march_xi(GradArgs a)
 // interfaces fill 240 of 256 threads.  Periodic cases read ghosts at their image and form T and mu from
 // what they read, so their stages need no ghost fill.
 // A plane of 64^2 to 200^2 nodes leaves most of the chip idle and its time is the chain of its launches:
-// six dependent kernels of 7-12 us per stage, one of 19 us here (64^2 WENO5 58 -> 19 us, 211 x 157 WENO9
-// 74 -> 27).  Large planes are bound by the FP64 pipe and its latency (one block per CU by LDS) and gain
-// from the passes over memory between the kernels: 1000 x 768 283 -> 205 us.
+// six dependent kernels of 7-12 us per stage, one of 17 us here (64^2 WENO5 58 -> 17 us, 211 x 157 WENO9
+// 74 -> 26).  Large planes are bound by the FP64 pipe and its latency (one block per CU by LDS) and gain
+// from the passes over memory between the kernels: 1000 x 768 283 -> 188 us.
 constexpr int PT = 15;
 struct PlaneArgs {
     WenoArgs w[2];                // the sweep records of xi and eta (Q in w[0].q)
@@ -2135,8 +2136,8 @@ __device__ __forceinline__ void plane_body(const PlaneArgs &z, const int tile, d
     const Consts &k = z.w[0].k;
     const int i0 = z.lo[0] + ti * PT, j0 = z.lo[1] + tj * PT;    // padded index of the tile's first node
     // The update's U_n and Q_sum and, for WENO5, the viscous window are loaded before the WENO sweeps: one
-    // block per CU has nothing else to overlap those loads with.  64^2 WENO5 18.8 -> 17.6 us a stage, 1000 x
-    // 768 207 -> 190, 211 x 157 WENO9 27.0 -> 25.6 (with its
+    // block per CU has nothing else to overlap those loads with.  64^2 WENO5 18.8 -> 17.1 us a stage, 1000 x
+    // 768 207 -> 188, 211 x 157 WENO9 27.0 -> 25.6 (with its
     // window as well 25.1, but 43 spilled registers in a batch).
     constexpr int PER = (RN + 511) / 512;
     double in[PER][12];
@@ -2926,7 +2927,7 @@ struct shx_case {
     shx_batch *batch = nullptr;
     // pinned staging of host transfers (allocated on the first upload or download): STAGE_SLOTS slots
     // of stage_len doubles, each with the event of the launch that last used it
-    double *stage_h = nullptr;
+    double *stage_h[STAGE_SLOTS] = {};
     hipEvent_t stage_ev[STAGE_SLOTS] = {};
     long stage_len = 0;
 };
@@ -3142,9 +3143,10 @@ extern "C" int shx_destroy(shx_case *c)
     for (int m = 0; m < 6; m++) hipFree(c->bs[m]);
     hipFree(c->T); hipFree(c->mu); hipFree(c->d_red); hipFree(c->d_cnt); hipFree(c->d_nan);
     if (c->h_io) hipHostFree(c->h_io);
-    for (int b = 0; b < STAGE_SLOTS; b++)
+    for (int b = 0; b < STAGE_SLOTS; b++) {
         if (c->stage_ev[b]) hipEventDestroy(c->stage_ev[b]);
-    if (c->stage_h) hipHostFree(c->stage_h);
+        if (c->stage_h[b]) hipHostFree(c->stage_h[b]);
+    }
     hipFree(c->P); hipFree(c->C); hipFree(c->PL); hipFree(c->RL); hipFree(c->UL); hipFree(c->C0);
     for (int b = 0; b < 2; b++) {
         for (int m = 0; m < 5; m++) hipFree(c->bk[b][m]);
@@ -3190,7 +3192,7 @@ static hipError_t xfer_launch(const Xfer &x, const long i, const int slot)
     XferArgs k = x.k;
     k.t0 = i * x.chunk;
     k.n = std::min(x.chunk, x.total - k.t0);
-    k.host = x.c->stage_h + (long)slot * x.c->stage_len;
+    k.host = x.c->stage_h[slot];
     const unsigned grid = (unsigned)std::min<long>((k.n + 255) / 256, 1024);
     if (x.up) k_unpack<<<grid, 256, 0, x.c->stream>>>(k);
     else k_pack<<<grid, 256, 0, x.c->stream>>>(k);
@@ -3201,7 +3203,7 @@ static hipError_t xfer_launch(const Xfer &x, const long i, const int slot)
 // chunk i between its slot and the caller's arrays
 static void xfer_copy(const Xfer &x, const long i, const int slot)
 {
-    const double *s = x.c->stage_h + (long)slot * x.c->stage_len;
+    const double *s = x.c->stage_h[slot];
     for (long t = i * x.chunk, end = std::min(t + x.chunk, x.total); t < end;) {
         const long m = t / x.k.hw, r = t - m * x.k.hw, n = std::min(x.k.hw - r, end - t);
         if (x.up) memcpy((void *)s, x.host[m] + r, sizeof(double) * n);
@@ -3259,10 +3261,14 @@ static int transfer(shx_case *c, const bool up, const int nf, double *const *dev
         for (int q = 0; q < copies; q++) x.k.more[q][m] = more[q][m];
     }
     x.total = (long)nf * gm.ntot;
-    if (!c->stage_h) {
+    if (!c->stage_len) {
         // slots for the five fields of a state in two chunks per thread, within the limits
         const long len = std::max(STAGE_MIN, std::min(STAGE_MAX, (5 * gm.ntot + STAGE_SLOTS - 1) / STAGE_SLOTS));
-        HIPCHK(hipHostMalloc((void **)&c->stage_h, sizeof(double) * (size_t)len * STAGE_SLOTS, hipHostMallocDefault));
+        // one allocation per slot: a new case's are taken from what an earlier one gave back, where one of
+        // 16 MB was pinned anew (first upload of 176 x 128 x 136 5.2 -> 3.5 ms, 97 x 85 x 106 3.6 -> 2.5)
+        for (int b = 0; b < STAGE_SLOTS; b++)
+            if (!c->stage_h[b])
+                HIPCHK(hipHostMalloc((void **)&c->stage_h[b], sizeof(double) * (size_t)len, hipHostMallocDefault));
         c->stage_len = len;
     }
     for (int b = 0; b < STAGE_SLOTS; b++) {
