@@ -4858,26 +4858,31 @@ static hipError_t batch_enqueue(shx_batch *b)
     return e;
 }
 
+// (the graph before it stays until the new one is there)
 static int batch_capture(shx_batch *b)
 {
-    if (b->exec) { hipGraphExecDestroy(b->exec); b->exec = nullptr; }
-    if (b->graph) { hipGraphDestroy(b->graph); b->graph = nullptr; }
     int rc = batch_lanes(b);
     if (rc) return rc;
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
     HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     hipError_t e = batch_enqueue(b);
+    const hipError_t end = hipStreamEndCapture(b->stream, &graph);
+    if (e == hipSuccess) e = end;
+    if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     if (e != hipSuccess) {
-        hipGraph_t g = nullptr;
-        hipStreamEndCapture(b->stream, &g);
-        if (g) hipGraphDestroy(g);
+        if (graph) hipGraphDestroy(graph);
         return set_err(SHX_ERR_HIP, "batch capture: %s", hipGetErrorString(e));
     }
-    HIPCHK(hipStreamEndCapture(b->stream, &b->graph));
-    HIPCHK(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
+    if (b->exec) hipGraphExecDestroy(b->exec);
+    if (b->graph) hipGraphDestroy(b->graph);
+    b->graph = graph;
+    b->exec = exec;
     return SHX_OK;
 }
 
-// upload the tables (same layout on every rebuild, so captured pointers stay valid)
+// upload the tables: into the device's own where their layout is the same, which keeps captured pointers
+// valid, else into a new one (fresh)
 static int batch_upload(shx_batch *b, bool fresh)
 {
     if (fresh) {
@@ -4938,18 +4943,52 @@ extern "C" int shx_batch_create(shx_case *const *cases, int ncases, const double
     return SHX_OK;
 }
 
+// the launches of two builds read their tables at the same places with the same grids
+static bool same_layout(const std::vector<BatchLaunch> &a, const std::vector<BatchLaunch> &b)
+{
+    if (a.size() != b.size()) return false;
+    for (size_t i = 0; i < a.size(); i++)
+        if (a[i].fn != b[i].fn || a[i].fnp != b[i].fnp || a[i].threads != b[i].threads || a[i].total != b[i].total ||
+            a[i].klass != b[i].klass || a[i].group != b[i].group || a[i].args_off != b[i].args_off ||
+            a[i].work_off != b[i].work_off)
+            return false;
+    return true;
+}
+
+// The cases can change under a batch what its launches are: post-processing makes a case keep its
+// pressure (which adds passes, and ghost fills where it read ghosts at their image), a new metric or
+// shx_tune its kernels.  A build that no longer fits the tables and the captured graph replaces both; if
+// that fails, the batch stays as it was.
 extern "C" int shx_batch_set_tau(shx_batch *b, const double *tau)
 {
     if (!b || !tau) return set_err(SHX_ERR_ARG, "null argument");
     for (size_t i = 0; i < b->cases.size(); i++)
         if (!(tau[i] > 0.0)) return set_err(SHX_ERR_ARG, "case %zu: tau must be positive", i);
     HIPCHK(hipStreamSynchronize(b->stream));
+    std::vector<BatchLaunch> seq = b->seq;
+    std::vector<char> host = b->host;
+    std::vector<double> old_tau = b->tau;
+    char *const dev = b->dev;
+    const int ngroups = b->ngroups;
     b->tau.assign(tau, tau + b->cases.size());
-    std::vector<BatchLaunch> old = b->seq;
     int rc = batch_build(b);
-    if (rc) return rc;
-    for (size_t i = 0; i < b->seq.size(); i++) { b->seq[i].grid = old[i].grid; b->seq[i].run = old[i].run; }
-    return batch_upload(b, false);
+    if (!rc && same_layout(seq, b->seq) && host.size() == b->host.size()) {
+        for (size_t i = 0; i < b->seq.size(); i++) { b->seq[i].grid = seq[i].grid; b->seq[i].run = seq[i].run; }
+        return batch_upload(b, false);
+    }
+    b->dev = nullptr;
+    if (!rc) rc = batch_upload(b, true);
+    if (!rc) rc = batch_grids(b);
+    if (!rc) rc = batch_capture(b);
+    if (rc) {
+        if (b->dev) hipFree(b->dev);
+        b->dev = dev;
+        b->seq.swap(seq); b->host.swap(host); b->tau.swap(old_tau);
+        b->ngroups = ngroups;
+        return rc;
+    }
+    hipFree(dev);
+    return SHX_OK;
 }
 
 extern "C" int shx_batch_run(shx_batch *b, int nsteps)
