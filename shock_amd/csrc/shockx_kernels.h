@@ -488,9 +488,12 @@ __device__ __forceinline__ double w9_is(const double a, const double b, const do
 
 // Six times the WENO9 deviation of a field (Phi_Function_W9, src/WENO.c:11-116, of the minus side less
 // the plus side, as w5_pair) from the eight split differences of each side.  Each side's indicators are
-// scaled by the power of two that brings the largest to [1, 2) and epsilon is held at f = 2^-80 there:
-// with s_k = (IS_k + eps)^2 the sums D = sum_k 126 d_k prod_{j != k} s_j are at least f^6, so the product
-// of both sides' stays normal for the one reciprocal, and a capped weight is below 2^-160.
+// scaled by the power of two that brings the largest to [1, 2) and epsilon is held at f = 2^-160 there.
+// Beside a jump the smooth sub-stencils' indicators are the small ones, and they carry the weights: what
+// the floor hides is differences below 2^-80 of the largest, which are not seen beside its rounding.
+// With s_k = (IS_k + eps)^2 the sums D = sum_k 126 d_k prod_{j != k} s_j are at least f^6 = 2^-960, still
+// normal; a product that falls below belongs to a weight under 2^-55.  Each side's products are
+// scaled by the power of two that brings its D to [1, 2), so that one reciprocal serves both.
 __device__ __forceinline__ double w9_pair(const double eps, const double p[8], const double m[8])
 {
     double N[2], D[2], T[2];
@@ -502,15 +505,17 @@ __device__ __forceinline__ double w9_pair(const double eps, const double p[8], c
                        w9_is<0>(d[7], d[6], d[5], d[4])};
         const double mx = fmax(fmax(fmax(s[0], s[1]), fmax(s[2], s[3])), fmax(s[4], eps));
         const double sc = inv_pow2(mx);
-        const double fl = fmax(eps * sc, 0x1p-80);
+        const double fl = fmax(eps * sc, 0x1p-160);
 #pragma unroll
         for (int k = 0; k < 5; k++) {
             const double q = fma(s[k], sc, fl);
             s[k] = q * q;
         }
         const double p01 = s[0] * s[1], p012 = p01 * s[2], s34 = s[3] * s[4], s234 = s[2] * s34;
-        const double P0 = s[1] * s234, P1 = s[0] * s234, P2 = p01 * s34, P3 = p012 * s[4], P4 = p012 * s[3];
+        double P0 = s[1] * s234, P1 = s[0] * s234, P2 = p01 * s34, P3 = p012 * s[4], P4 = p012 * s[3];
         D[h] = fma(5., P4, fma(40., P3, fma(60., P2, fma(20., P1, P0))));
+        const double dn = inv_pow2(D[h]);
+        D[h] *= dn; P0 *= dn; P2 *= dn; P3 *= dn; P4 *= dn;
         double v[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) v[k] = fma(6., d[k + 2], fma(-4., d[k + 1] + d[k + 3], d[k] + d[k + 4]));
