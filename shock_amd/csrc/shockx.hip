@@ -2903,7 +2903,7 @@ struct shx_case {
     int faces;             // number of non-periodic faces
     int needs_bs;          // some face is SHX_BC_MANUFACTURED
     int diag;              // 3D metric is diagonal (only xi_x, eta_y, zeta_z and J non-zero)
-    int flat;              // 2D: xi_z and eta_z are zero
+    int flat;              // 2D: xi_z and eta_z are zero (joined blocks: diag and flat of all of them)
     int wtile[3];          // WENO tile variant per direction (set by shx_tune; -1: by zeta_tile)
     unsigned long long *d_red;
     int *d_cnt;
@@ -4388,6 +4388,10 @@ extern "C" int shx_blocks_transfer_metric(shx_blocks *g)
     int rc;
     if ((rc = join_blocks(g)) || (rc = gather(g, true)) || (rc = fork_blocks(g))) return rc;
     HIPCHK(hipStreamSynchronize(g->stream));
+    // a block's ghost rows are its neighbours' now: entries count as zero only where every block's are
+    int diag = 1, flat = 1;
+    for (const shx_case *c : g->b) { diag &= c->diag; flat &= c->flat; }
+    for (shx_case *c : g->b) { c->diag = diag; c->flat = flat; }
     return SHX_OK;
 }
 
