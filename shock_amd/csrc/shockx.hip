@@ -3217,7 +3217,7 @@ static hipError_t xfer_chunks(const Xfer &x, const int id)
 {
     const long nc = (x.total + x.chunk - 1) / x.chunk;
     const int s0 = 2 * id;
-    hipError_t e = id ? hipSetDevice(x.c->dev) : hipSuccess;   // a new thread starts on device 0
+    hipError_t e = hipSuccess;
     long turn = 0;
     if (x.up) {
         // a slot's previous launch (two turns back, or an earlier call's) has read it
@@ -3285,14 +3285,17 @@ static int transfer(shx_case *c, const bool up, const int nf, double *const *dev
     for (int t = 1; t < x.threads; t++) {
         err[t] = hipErrorUnknown;
         try {
-            th[t] = std::thread([&x, &err, t] { err[t] = xfer_chunks(x, t); });
+            th[t] = std::thread([&x, &err, t] {
+                err[t] = hipSetDevice(x.c->dev);           // a new thread starts on device 0
+                if (err[t] == hipSuccess) err[t] = xfer_chunks(x, t);
+            });
         } catch (...) {
         }
     }
     err[0] = xfer_chunks(x, 0);
     for (int t = 1; t < x.threads; t++) {
         if (th[t].joinable()) th[t].join();
-        else err[t] = xfer_chunks(x, t);       // no thread available: its chunks here
+        else err[t] = xfer_chunks(x, t);       // no thread available: its chunks here, on the caller's device
     }
     for (int t = 0; t < x.threads; t++) HIPCHK(err[t]);
     return SHX_OK;
