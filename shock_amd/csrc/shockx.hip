@@ -2925,11 +2925,12 @@ struct shx_case {
     // they were at shx_batch_create); stepping the case alone while it is set would leave the
     // batch advancing a stale buffer
     shx_batch *batch = nullptr;
-    // pinned staging of host transfers (allocated on the first upload or download): STAGE_SLOTS slots
-    // of stage_len doubles, each with the event of the launch that last used it
+    // pinned staging of host transfers: up to two slots per host thread of stage_len doubles (allocated by
+    // the first transfer that goes through them), each with the event of the launch that last used it
     double *stage_h[STAGE_SLOTS] = {};
     hipEvent_t stage_ev[STAGE_SLOTS] = {};
     long stage_len = 0;
+    int stage_threads = 0;   // host threads of a transfer, at most
 };
 
 extern "C" const char *shx_last_error(void) { return g_err; }
@@ -3177,8 +3178,14 @@ extern "C" int shx_padded_extent(const shx_case *c, int ng[3])
 // copy's threads started per slot, the pipeline drained between fields: state downloads of a 64^2 plane
 // 118 -> 21 us, 48^3 479 -> 250, 1000 x 768 1.25 -> 0.80 ms, 97 x 85 x 106 1.74 -> 1.12, 256^3 14.9 either
 // way (PCIe).  2 MB slots and four threads: 512 KB slots or eight threads measured slower.
+// A state of under 5 MB stays on the calling thread, where starting threads costs what they give (42^3
+// 177 us either way, 32^3 117 against 131), through two slots of a field or of a third of the state, and
+// one of up to 256 KB through one slot: a case pins what it needs (64^2 0.2 MB, 18^3 0.4, 32^3 0.9).  Eight
+// slots of 256 KB for each of them pinned 2 MB, and a new case's first upload took 255, 250 and 304 us
+// against 90, 137 and 160.
 // A pitched copy straight to or from pageable memory ran at 0.3 GB/s.
-constexpr long STAGE_MIN = 1L << 15, STAGE_MAX = 1L << 18;   // doubles per slot: 256 KB to 2 MB
+constexpr long STAGE_MIN = 1L << 15, STAGE_MAX = 1L << 18;   // doubles: 256 KB, and 2 MB per slot at most
+constexpr long STAGE_MANY = 5L << 17;                        // states from here on take four threads
 struct Xfer {
     shx_case *c;
     XferArgs k;
@@ -3262,24 +3269,27 @@ static int transfer(shx_case *c, const bool up, const int nf, double *const *dev
     }
     x.total = (long)nf * gm.ntot;
     if (!c->stage_len) {
-        // slots for the five fields of a state in two chunks per thread, within the limits
-        const long len = std::max(STAGE_MIN, std::min(STAGE_MAX, (5 * gm.ntot + STAGE_SLOTS - 1) / STAGE_SLOTS));
-        // one allocation per slot: a new case's are taken from what an earlier one gave back, where one of
-        // 16 MB was pinned anew (first upload of 176 x 128 x 136 5.2 -> 3.5 ms, 97 x 85 x 106 3.6 -> 2.5)
-        for (int b = 0; b < STAGE_SLOTS; b++)
-            if (!c->stage_h[b])
-                HIPCHK(hipHostMalloc((void **)&c->stage_h[b], sizeof(double) * (size_t)len, hipHostMallocDefault));
-        c->stage_len = len;
-    }
-    for (int b = 0; b < STAGE_SLOTS; b++) {
-        if (c->stage_ev[b]) continue;
-        HIPCHK(hipEventCreateWithFlags(&c->stage_ev[b], hipEventDisableTiming));
-        HIPCHK(hipEventRecord(c->stage_ev[b], c->stream));
+        const long state = 5 * gm.ntot;
+        c->stage_threads = (state < STAGE_MANY) ? 1 : STAGE_SLOTS / 2;
+        if (state <= STAGE_MIN) c->stage_len = state;
+        else if (state < STAGE_MANY) c->stage_len = std::max(gm.ntot, std::min(STAGE_MIN, (state + 2) / 3));
+        else c->stage_len = std::min(STAGE_MAX, (state + STAGE_SLOTS - 1) / STAGE_SLOTS);
     }
     x.chunk = c->stage_len;
     const long nc = (x.total + x.chunk - 1) / x.chunk;
-    // up to four threads; a call of few small chunks stays on the calling one
-    x.threads = (x.total < 2 * STAGE_SLOTS * STAGE_MIN / 4) ? 1 : (int)std::min<long>(STAGE_SLOTS / 2, nc);
+    x.threads = (int)std::min<long>(c->stage_threads, nc);
+    // the slots that xfer_chunks goes through, one allocation each: a new case's are taken from what an
+    // earlier one gave back, where one of 16 MB was pinned anew (first upload of 176 x 128 x 136 5.2 -> 3.5
+    // ms, 97 x 85 x 106 3.6 -> 2.5)
+    for (int id = 0; id < x.threads; id++)
+        for (int q = 0; q < 2 && id + (long)q * x.threads < nc; q++) {
+            const int b = 2 * id + q;
+            if (!c->stage_h[b])
+                HIPCHK(hipHostMalloc((void **)&c->stage_h[b], sizeof(double) * (size_t)c->stage_len, hipHostMallocDefault));
+            if (c->stage_ev[b]) continue;
+            HIPCHK(hipEventCreateWithFlags(&c->stage_ev[b], hipEventDisableTiming));
+            HIPCHK(hipEventRecord(c->stage_ev[b], c->stream));
+        }
     hipError_t err[STAGE_SLOTS / 2];
     std::thread th[STAGE_SLOTS / 2];
     for (int t = 1; t < x.threads; t++) {
