@@ -31,6 +31,7 @@
 #include <string.h>
 #include <type_traits>
 #include <algorithm>
+#include <functional>
 #include <thread>
 #include <vector>
 
@@ -3278,6 +3279,10 @@ static int transfer(shx_case *c, const bool up, const int nf, double *const *dev
     x.chunk = c->stage_len;
     const long nc = (x.total + x.chunk - 1) / x.chunk;
     x.threads = (int)std::min<long>(c->stage_threads, nc);
+    // fields that come down into one array are written in order, on one thread
+    for (int m = 1; !up && m < nf; m++)
+        for (int q = 0; q < m; q++)
+            if (std::less<double *>()(host[q], host[m] + gm.ntot) && std::less<double *>()(host[m], host[q] + gm.ntot)) x.threads = 1;
     // the slots that xfer_chunks goes through, one allocation each: a new case's are taken from what an
     // earlier one gave back, where one of 16 MB was pinned anew (first upload of 176 x 128 x 136 5.2 -> 3.5
     // ms, 97 x 85 x 106 3.6 -> 2.5)
