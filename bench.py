@@ -67,8 +67,6 @@ def algo_bytes(name, n, ng, time_order=4, diag=True):
     if name == "visc_grad_xi":                   # the march with viscous xi: u,v,w (padded); T, mu,
         # the diagonal metric and J, Q (momentum, energy) r/w per interior node; 7 derivatives out
         return (npad * 3 + nint * (2 + 4 + 8)) * FP64 + 7 * n * ng * ng * FP64
-    if name == "rk_update":          # U_n, Q, J in (Qsum r/w on RK4 stages), U_s+1 out
-        return nint * (5 + 5 + 1 + 5 + qsum) * FP64
     if name == "ghost_periodic":     # 5 fields read + written on ghost nodes
         return ghost * 5 * 2 * FP64
     return None

@@ -288,7 +288,9 @@ int shx_copy_probe(shx_case *c, int reps);
 
 /* Per-kernel timing with HIP events on the handle's stream.  When enabled, every launch is
  * bracketed by events; shx_kernel_times synchronizes and returns, per kernel class, the total
- * milliseconds and the launch count since the last reset.  names[k] points to static strings. */
+ * milliseconds and the launch count since the last reset.  names[k] points to static strings.  A
+ * 2D stage after its ghosts is one kernel (plane_stage); an inviscid stage's update is part of its
+ * last WENO sweep. */
 #define SHX_NUM_KERNELS 16
 int shx_set_timing(shx_case *c, int enable);
 int shx_kernel_times(shx_case *c, const char *names[SHX_NUM_KERNELS], double ms[SHX_NUM_KERNELS],
@@ -341,8 +343,9 @@ typedef struct shx_batch shx_batch;
 int shx_batch_create(shx_case *const *cases, int ncases, const double *tau, shx_batch **out);
 int shx_batch_set_tau(shx_batch *b, const double *tau);
 int shx_batch_run(shx_batch *b, int nsteps);
-/* Picks the resident blocks per CU of each kernel class (ghost, values, grad, weno, visc, rk) by
- * timing replayed steps; the case states are restored.  factors_out may be NULL. */
+/* Picks the resident blocks per CU of each kernel class (ghost, values, grad, weno, visc and
+ * plane, the whole 2D stage) by timing replayed steps; the case states are restored.  factors_out
+ * may be NULL. */
 int shx_batch_tune(shx_batch *b, int steps, int factors_out[6]);
 /* Waits for the batch's steps.  checkNAN (src/Functions.c:5419-5467) is fused into every case's
  * last stage as in shx_run, but read here rather than after every step, so that shx_batch_run

@@ -419,7 +419,7 @@ __device__ __forceinline__ void sweep_tile(const int p, const int tg[4], int &bx
 
 // ---- WENO sweep ---------------------------------------------------------------------------
 struct WenoArgs {
-    CFields5 pr;          // rho, u, v, w, e of the stage input (ghosts filled)
+    CFields5 pr;          // rho, u, v, w, e of the stage input (ghosts filled unless wrap)
     gcdp m0, m1, m2, J;               // metric row of the sweep direction and the Jacobian
                                       // (diagonal metrics: m0 is the row's diagonal entry)
     Fields5 q;            // stage residual, interior nodes
@@ -1678,7 +1678,7 @@ __device__ __forceinline__ void eta_body(const EtaArgs &z, const int bx, const i
     __syncthreads();
     visc_diag_body<5, 1, 8, 32, true>(z.v, bx, by, bz, lds, inv);
 }
-// FP64: four waves per SIMD (126 VGPRs; weno5_flux)
+// FP64: four waves per SIMD (126 VGPRs; weno_flux)
 constexpr int ETA_WAVES = 4;
 template <bool MIX>
 __global__ __launch_bounds__(256, (MIX ? 1 : ETA_WAVES)) void k_eta(EtaArgs z)
@@ -2845,11 +2845,10 @@ static int set_err(int code, const char *fmt, ...)
                            __FILE__, __LINE__);                                               \
     } while (0)
 
-// KT_ZETA also times k_plane, the whole 2D stage
-enum { KT_GHOST, KT_VALUES, KT_WENO0, KT_WENO1, KT_WENO2, KT_GRAD, KT_VISC0, KT_VISC1, KT_VISC2, KT_RK, KT_REDUCE, KT_METRIC, KT_FACES, KT_ZETA, KT_GRADXI, KT_ETA };
+enum { KT_GHOST, KT_VALUES, KT_WENO0, KT_WENO1, KT_WENO2, KT_GRAD, KT_VISC0, KT_VISC1, KT_VISC2, KT_PLANE, KT_REDUCE, KT_METRIC, KT_FACES, KT_ZETA, KT_GRADXI, KT_ETA };
 static const char *g_knames[SHX_NUM_KERNELS] = {
     "ghost_periodic", "ghost_values", "weno_xi", "weno_eta", "weno_zeta",
-    "visc_grad", "visc_xi", "visc_eta", "visc_zeta", "rk_update", "reduce", "metric", "ghost_faces",
+    "visc_grad", "visc_xi", "visc_eta", "visc_zeta", "plane_stage", "reduce", "metric", "ghost_faces",
     "weno_visc_zeta", "visc_grad_xi", "weno_visc_eta"};
 
 // face kinds whose writers store a p and c that the equation of state does not give from the
@@ -3689,7 +3688,6 @@ static int launch_pick(const void *fn, dim3 grid, int threads, void *arg, hipStr
     return SHX_OK;
 }
 
-// one WENO sweep along axis dir of the state `pr`
 // one-dimensional launch of a tile grid g; tg receives its extents and the tile order
 static dim3 flat_grid(const dim3 g, int tg[4], int order)
 {
@@ -3710,6 +3708,8 @@ static WenoLastArgs weno_last_args(const shx_case *c, double *const *pr, int fir
     if (rk) z.rk = *rk;
     return z;
 }
+// one WENO sweep along axis dir of the state `pr`; rk: the sweep is of an inviscid stage, whose last one
+// (k_weno_last) applies this update
 static int weno_sweep(shx_case *c, double *const *pr, int dir, int first, const RkArgs *rk = nullptr)
 {
     WenoLastArgs z;
@@ -3725,9 +3725,6 @@ static int weno_sweep(shx_case *c, double *const *pr, int dir, int first, const 
     return tend(c);
 }
 
-// residual of one stage into c->q: ghost fill, derived quantities, viscous derivatives, WENO
-// sweeps of every direction, then the viscous sweeps (the reference's accumulation order,
-// src/Functions.c:2161-2272)
 static int visc_sweep(shx_case *c, double *const *pr, int dir, const RkArgs *rk);
 static int zeta_sweep(shx_case *c, double *const *pr, const RkArgs *rk);
 // the zeta direction runs as one fused kernel (k_zeta)
@@ -3845,12 +3842,15 @@ static PlaneArgs plane_args(const shx_case *c, double *const *pr, const RkArgs *
 static int plane_stage(shx_case *c, double *const *pr, const RkArgs *rk, const bool wrap)
 {
     PlaneArgs z = plane_args(c, pr, rk, wrap);
-    int rc = tbeg(c, KT_ZETA);
+    int rc = tbeg(c, KT_PLANE);
     if (rc) return rc;
     if ((rc = launch_pick(plane_pick(c).single, dim3(z.nt[0] * z.nt[1]), 512, &z, c->stream))) return rc;
     return tend(c);
 }
-// rk: when given, the last viscous sweep applies this stage update instead of storing Q
+// residual of one stage into c->q: ghost fill, derived quantities, viscous derivatives, WENO
+// sweeps of every direction, then the viscous sweeps (the reference's accumulation order,
+// src/Functions.c:2161-2272).  rk: when given, the stage's last kernel (2D k_plane, inviscid k_weno_last,
+// else the last viscous sweep) applies this update instead of storing Q
 static int stage_fluxes(shx_case *c, double *const *pr, const RkArgs *rk, double tau)
 {
     const Geom &gm = c->gm;
@@ -4464,8 +4464,7 @@ struct BatchLaunch {
     const int4 *work;
 };
 
-enum { BK_GHOST, BK_VALUES, BK_GRAD, BK_WENO, BK_VISC, BK_RK, BK_NUM };
-static const char *g_bknames[BK_NUM] = {"ghost", "values", "grad", "weno", "visc", "rk"};
+enum { BK_GHOST, BK_VALUES, BK_GRAD, BK_WENO, BK_VISC, BK_PLANE, BK_NUM };
 
 struct shx_batch {
     std::vector<shx_case *> cases;
@@ -4695,7 +4694,7 @@ static int batch_group(shx_batch *b, const std::vector<shx_case *> &g, const std
                 put(recs, z);
                 grids.push_back(dim3(z.nt[0] * z.nt[1]));
             }
-            batch_add(b, p.batch, p.batchp, 512, BK_WENO, recs, sizeof(PlaneArgs), grids, ORDER_NODES);
+            batch_add(b, p.batch, p.batchp, 512, BK_PLANE, recs, sizeof(PlaneArgs), grids, ORDER_NODES);
         }
         // the same sweep sequence as stage_fluxes (fused eta and zeta directions where they apply)
         const bool fz = fuse_zeta(c0), fx = fuse_xi(c0), fe = fuse_eta(c0);

@@ -82,7 +82,7 @@ EXPORTS = [
     "shx_blocks_create", "shx_blocks_transfer_metric", "shx_blocks_run", "shx_blocks_destroy",
 ]
 ERR_NAN = -5
-BATCH_CLASSES = ("ghost", "values", "grad", "weno", "visc", "rk")
+BATCH_CLASSES = ("ghost", "values", "grad", "weno", "visc", "plane")
 
 _lib = None
 
