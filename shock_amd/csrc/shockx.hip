@@ -485,8 +485,8 @@ __device__ __forceinline__ double next_lane(const double v)
 // window is read 80 to 120 times per WENO5 interface instead of 190 (once per non-zero entry of the
 // left eigenvectors), which had the LDS as busy as the FP64 pipe, and FP64 instructions fall from 926
 // to about 750 (256^3, diagonal metric: xi sweep 1.04 -> 0.82 ms, k_eta 1.42 -> 1.26, k_zeta 1.70 -> 1.57).
-// WENO9, 176 x 128 x 136: xi and eta sweeps 425 and 457 -> 308 and 326 us, k_zeta 684 -> 489 (indicators as
-// sums of squares of the differences, w9_is, and three waves per SIMD instead of two).
+// WENO9, 176 x 128 x 136: xi and eta sweeps 425 and 457 -> 309 and 327 us, k_zeta 684 -> 523 (447 on its 8 x 32
+// tile; indicators as sums of squares of the differences, w9_is, and three waves per SIMD instead of two).
 // Bound by the FP64 pipe and its latency, so registers decide: the projections are pinned pair by pair
 // (else the compiler keeps several pairs in flight, 148-166 VGPRs for WENO5), which leaves WENO5 along
 // zeta 128 VGPRs, four waves per SIMD.  Along xi and eta one pass over all fields still spilled two
@@ -950,7 +950,7 @@ __device__ __forceinline__ int wave_sum(int v)
 }
 // Maxima of non-negative doubles reduce into RED_SLOTS slots (positive doubles order like their
 // bit patterns, so an unsigned 64-bit atomic max combines them); a block uses slot
-// blockIdx % RED_SLOTS, and the host takes the maximum of the slots.  One slot for a whole
+// blockIdx % RED_SLOTS, and k_red_report takes the maximum of the slots.  One slot for a whole
 // launch would serialise every wave's atomic on one cache line.
 constexpr int RED_SLOTS = 256;
 __device__ __forceinline__ void wave_max_to(unsigned long long *out, double v)
@@ -3124,7 +3124,8 @@ extern "C" int shx_create(const shx_desc *desc, shx_case **out)
     // holds 1.19 nodes per interface node against 1.40, and its LDS lets a fourth block on a CU (256^3:
     // xi sweep 0.89 -> 0.82 ms FP64, 0.93 -> 0.81 mixed; 144 x 112 x 128 mixed WENO9: 224 -> 172 and
     // 247 -> 188 us).  FP64 WENO9 and the general metric run three blocks either way and lose on eta
-    // (176 x 128 x 136 WENO9 326 -> 352 us, 119 x 96 x 104 general 79 -> 87).
+    // (176 x 128 x 136 WENO9 327 -> 352 us, 119 x 96 x 104 general 79 -> 91); along xi WENO9 goes either way
+    // with the size (97 x 85 x 106 96 -> 106 us, 176 x 128 x 136 309 -> 302, 384^3 5.70 -> 5.17 ms).
     const bool wide = gm.dims == 3 && (d.quirks & SHX_QUIRK_METRIC_DIAG3D) && (S == 5 || d.precision == SHX_MIXED);
     for (int dir = 0; dir < 3; dir++) c->wtile[dir] = (gm.st[dir] == 1) ? -1 : (wide ? 1 : 0);
     *out = c;
@@ -3603,8 +3604,8 @@ static Pick weno_pick_v(bool coalesce, int variant, int ax, bool mix)
 }
 // Tile along the contiguous axis for a launch over nc cases: 0 = 4 x 64, 1 = 8 x 32.  A row of 64 threads
 // covers 63 nodes and one of 32 covers 31, so the last tile of a row can be nearly empty: 8 x 32 where it
-// takes fewer than 7/8 of the threads.  128 x 128 x 144 inviscid (0.83 of them) 184 -> 161 us, WENO9
-// viscous 176 x 128 x 136 (0.83) 525 -> 456, mixed 144 x 112 x 128 (0.83) 315 -> 299; its shorter rows read
+// takes fewer than 7/8 of the threads.  128 x 128 x 144 inviscid (0.83 of them) 186 -> 162 us, WENO9
+// viscous 176 x 128 x 136 (0.83) 523 -> 447, mixed 144 x 112 x 128 (0.83) 315 -> 298; its shorter rows read
 // more halo, 256^3 WENO5 (0.90) 1.50 -> 1.53 ms, and at equal threads 97 x 85 x 106 WENO9 133 -> 136 us.
 static int zeta_tile(const shx_case *const *g, const int nc)
 {

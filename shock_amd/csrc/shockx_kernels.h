@@ -321,15 +321,18 @@ __device__ __forceinline__ double inv_pow2(const double x)
     const int hi = (int)(__double_as_longlong(x) >> 32);
     return __longlong_as_double((long long)(0x7FE00000 - (hi & 0x7FF00000)) << 32);
 }
-// N[1] / D[1] - N[0] / D[0] with one reciprocal: the hardware's (24 bits) and one third-order step
+// N / D from the hardware's reciprocal (24 bits) and one third-order step
+__device__ __forceinline__ double quotient(const double N, const double D)
+{
+    const double r = __builtin_amdgcn_rcp(D);
+    const double e = fma(-D, r, 1.0);
+    const double y = N * r;
+    return fma(y, fma(e, e, e), y);
+}
+// N[1] / D[1] - N[0] / D[0] with one reciprocal
 __device__ __forceinline__ double pair_quotient(const double N[2], const double D[2])
 {
-    const double num = fma(N[1], D[0], -(N[0] * D[1]));
-    const double dd = D[0] * D[1];
-    const double r = __builtin_amdgcn_rcp(dd);
-    const double e = fma(-dd, r, 1.0);
-    const double y = num * r;
-    return fma(y, fma(e, e, e), y);
+    return quotient(fma(N[1], D[0], -(N[0] * D[1])), D[0] * D[1]);
 }
 
 // Six times the Jiang-Shu WENO5 deviation of a field (Phi_Function_W5, src/WENO.c:118-204, of the minus
@@ -492,11 +495,11 @@ __device__ __forceinline__ double w9_is(const double a, const double b, const do
 // Beside a jump the smooth sub-stencils' indicators are the small ones, and they carry the weights: what
 // the floor hides is differences below 2^-80 of the largest, which are not seen beside its rounding.
 // With s_k = (IS_k + eps)^2 the sums D = sum_k 126 d_k prod_{j != k} s_j are at least f^6 = 2^-960, still
-// normal; a product that falls below belongs to a weight under 2^-55.  Each side's products are
-// scaled by the power of two that brings its D to [1, 2), so that one reciprocal serves both.
+// normal; a product that falls below belongs to a weight under 2^-55.  The product of both sides' would not
+// be, so each has its reciprocal (seven instructions; scaling both for one took eighteen).
 __device__ __forceinline__ double w9_pair(const double eps, const double p[8], const double m[8])
 {
-    double N[2], D[2], T[2];
+    double Q[2], T[2];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         const double *d = h ? m : p;
@@ -512,18 +515,16 @@ __device__ __forceinline__ double w9_pair(const double eps, const double p[8], c
             s[k] = q * q;
         }
         const double p01 = s[0] * s[1], p012 = p01 * s[2], s34 = s[3] * s[4], s234 = s[2] * s34;
-        double P0 = s[1] * s234, P1 = s[0] * s234, P2 = p01 * s34, P3 = p012 * s[4], P4 = p012 * s[3];
-        D[h] = fma(5., P4, fma(40., P3, fma(60., P2, fma(20., P1, P0))));
-        const double dn = inv_pow2(D[h]);
-        D[h] *= dn; P0 *= dn; P2 *= dn; P3 *= dn; P4 *= dn;
+        const double P0 = s[1] * s234, P1 = s[0] * s234, P2 = p01 * s34, P3 = p012 * s[4], P4 = p012 * s[3];
+        const double D = fma(5., P4, fma(40., P3, fma(60., P2, fma(20., P1, P0))));
         double v[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) v[k] = fma(6., d[k + 2], fma(-4., d[k + 1] + d[k + 3], d[k] + d[k + 4]));
         const double r = fma(3., v[1], -2. * v[2]);
-        N[h] = fma(0.25 * P4, fma(3., v[3], r), fma(2. * P3, r, fma(9. * P2, v[1], (0.6 * P0) * v[0])));
+        Q[h] = quotient(fma(0.25 * P4, fma(3., v[3], r), fma(2. * P3, r, fma(9. * P2, v[1], (0.6 * P0) * v[0]))), D);
         T[h] = fma(39., v[1], fma(-14., v[2], 3. * v[3]));
     }
-    return fma(1. / 280., T[0] - T[1], pair_quotient(N, D));
+    return fma(1. / 280., T[0] - T[1], Q[1] - Q[0]);
 }
 
 __device__ __forceinline__ double pressure(const Consts &k, double rho, double u, double v, double w, double e)
