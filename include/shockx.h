@@ -147,7 +147,7 @@ int shx_download_metric(shx_case *c, double *const met[10]);
  * (state, metric, source, boundary state, post-processing fields, residual) go through pinned
  * staging slots that the handle allocates as its transfers need them: a state of under 5 MB through
  * at most two on the calling thread (a field or a third of the state each, a state of up to 256 KB
- * through one), a larger one through eight of up to 2 MB, whose copies to and from the caller's
+ * through one), a larger one through four of up to 2 MB, whose copies to and from the caller's
  * arrays run on up to four short-lived host threads; an upload
  * returns once the caller's arrays have been read. */
 int shx_upload_state(shx_case *c, const double *const prim[5]);

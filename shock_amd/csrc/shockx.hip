@@ -2873,7 +2873,7 @@ static void wall_corrector(const int kind, const int dir, double cr[3])
     if (kind == SHX_BC_WALL_NOSLIP || kind == SHX_BC_WALL_ISOTHERMAL) cr[0] = cr[1] = cr[2] = -1.0;
 }
 
-constexpr int STAGE_SLOTS = 8;   // staging slots of host transfers, two per host thread
+constexpr int STAGE_SLOTS = 4;   // staging slots of host transfers: one per host thread, two where one thread is enough
 
 struct shx_case {
     shx_desc d;
@@ -2925,8 +2925,8 @@ struct shx_case {
     // they were at shx_batch_create); stepping the case alone while it is set would leave the
     // batch advancing a stale buffer
     shx_batch *batch = nullptr;
-    // pinned staging of host transfers: up to two slots per host thread of stage_len doubles (allocated by
-    // the first transfer that goes through them), each with the event of the launch that last used it
+    // pinned staging of host transfers: slots of stage_len doubles (allocated by the first transfer that
+    // goes through them), each with the event of the launch that last used it
     double *stage_h[STAGE_SLOTS] = {};
     hipEvent_t stage_ev[STAGE_SLOTS] = {};
     long stage_len = 0;
@@ -3125,7 +3125,7 @@ extern "C" int shx_create(const shx_desc *desc, shx_case **out)
     // xi sweep 0.89 -> 0.82 ms FP64, 0.93 -> 0.81 mixed; 144 x 112 x 128 mixed WENO9: 224 -> 172 and
     // 247 -> 188 us).  FP64 WENO9 and the general metric run three blocks either way and lose on eta
     // (176 x 128 x 136 WENO9 327 -> 352 us, 119 x 96 x 104 general 79 -> 91); along xi WENO9 goes either way
-    // with the size (97 x 85 x 106 96 -> 106 us, 176 x 128 x 136 309 -> 302, 384^3 5.70 -> 5.17 ms).
+    // with the size (97 x 85 x 106 96 -> 106 us, 176 x 128 x 136 309 -> 302, 384^3 5.89 -> 5.32 ms).
     const bool wide = gm.dims == 3 && (d.quirks & SHX_QUIRK_METRIC_DIAG3D) && (S == 5 || d.precision == SHX_MIXED);
     for (int dir = 0; dir < 3; dir++) c->wtile[dir] = (gm.st[dir] == 1) ? -1 : (wide ? 1 : 0);
     *out = c;
@@ -3173,17 +3173,18 @@ extern "C" int shx_padded_extent(const shx_case *c, int ng[3])
 
 // Host transfers.  Host arrays use the reference layout (dense rows); device rows are padded to the
 // pitch.  k_pack and k_unpack move chunks of all fields of a call between the device and slots of pinned
-// memory, and host threads copy between the slots and the caller's arrays.  A thread owns every fourth
-// chunk and two slots: the launch of its next chunk is in flight while it copies one (a thread copies
-// ~14 GB/s, PCIe moves 53), and no thread waits for another.  Field by field through two slots, with a
-// copy's threads started per slot, the pipeline drained between fields: state downloads of a 64^2 plane
-// 118 -> 21 us, 48^3 479 -> 250, 1000 x 768 1.25 -> 0.80 ms, 97 x 85 x 106 1.74 -> 1.12, 256^3 14.9 either
-// way (PCIe).  2 MB slots and four threads: 512 KB slots or eight threads measured slower.
-// A state of under 5 MB stays on the calling thread, where starting threads costs what they give (42^3
-// 177 us either way, 32^3 117 against 131), through two slots of a field or of a third of the state, and
-// one of up to 256 KB through one slot: a case pins what it needs (64^2 0.2 MB, 18^3 0.4, 32^3 0.9).  Eight
-// slots of 256 KB for each of them pinned 2 MB, and a new case's first upload took 255, 250 and 304 us
-// against 90, 137 and 160.
+// memory, and host threads copy between the slots and the caller's arrays.  A state from 5 MB on takes four
+// threads, each with every fourth chunk and a slot: while one copies (~14 GB/s), the launches of the others
+// are on the link (53 GB/s), and no thread waits for another.  Field by field through two slots, with a
+// copy's threads started per slot, the pipeline drained between fields: state downloads of 48^3 425 -> 240 us,
+// 1000 x 768 1.22 -> 0.78 ms, 97 x 85 x 106 1.60 -> 1.00, 256^3 14.9 either way (PCIe).  Slots of up to 2 MB: with
+// 1 MB 200^3 took 8.0 ms against 7.3, and eight threads were slower.
+// A smaller state stays on the calling thread, where starting threads costs what they give (42^3 177 us
+// either way, 32^3 117 against 131), through two slots, of a field or of a third of the state: the launch of
+// the next chunk is in flight while it copies one.  One of up to 256 KB goes through one slot (64^2 118 -> 21 us).
+// A case pins what it needs, and pinning is most of its first upload.  Eight slots of 256 KB to 2 MB for every
+// case, two a thread, moved 0-2 % more per second, and a new case's first upload took 0.50 ms at 64^2, 0.80 at
+// 32^3, 1.5 at 48^3, 4.0 at 97 x 85 x 106 and 2.9 at 1000 x 768 against 0.19, 0.56, 0.90, 2.6 and 2.0.
 // A pitched copy straight to or from pageable memory ran at 0.3 GB/s.
 constexpr long STAGE_MIN = 1L << 15, STAGE_MAX = 1L << 18;   // doubles: 256 KB, and 2 MB per slot at most
 constexpr long STAGE_MANY = 5L << 17;                        // states from here on take four threads
@@ -3193,7 +3194,7 @@ struct Xfer {
     bool up;
     double *host[XFER_FIELDS];    // the caller's arrays (read only by an upload)
     long total, chunk;
-    int threads;
+    int threads, per;             // slots of a thread
 };
 static hipError_t xfer_launch(const Xfer &x, const long i, const int slot)
 {
@@ -3220,30 +3221,29 @@ static void xfer_copy(const Xfer &x, const long i, const int slot)
         t += n;
     }
 }
-// the chunks of thread id: id, id + threads, ...
+// the chunks of thread id: id, id + threads, ..., through its slots in turn
 static hipError_t xfer_chunks(const Xfer &x, const int id)
 {
     const long nc = (x.total + x.chunk - 1) / x.chunk;
-    const int s0 = 2 * id;
     hipError_t e = hipSuccess;
-    long turn = 0;
+    int slot = id * x.per;
+    auto next = [&] { return (slot + 1 < (id + 1) * x.per) ? slot + 1 : id * x.per; };
     if (x.up) {
-        // a slot's previous launch (two turns back, or an earlier call's) has read it
-        for (long i = id; i < nc && e == hipSuccess; i += x.threads, turn++) {
-            const int slot = s0 + (int)(turn & 1);
+        // a slot's previous launch (of this call or an earlier one) has read it
+        for (long i = id; i < nc && e == hipSuccess; i += x.threads, slot = next()) {
             if ((e = hipEventSynchronize(x.c->stage_ev[slot])) != hipSuccess) break;
             xfer_copy(x, i, slot);
             e = xfer_launch(x, i, slot);
         }
         return e;
     }
-    for (int q = 0; q < 2 && e == hipSuccess; q++)
-        if (id + (long)q * x.threads < nc) e = xfer_launch(x, id + (long)q * x.threads, s0 + q);
-    for (long i = id; i < nc && e == hipSuccess; i += x.threads, turn++) {
-        const int slot = s0 + (int)(turn & 1);
+    const long ahead = (long)x.per * x.threads;
+    for (long i = id; i < nc && i < id + ahead && e == hipSuccess; i += x.threads, slot = next()) e = xfer_launch(x, i, slot);
+    slot = id * x.per;
+    for (long i = id; i < nc && e == hipSuccess; i += x.threads, slot = next()) {
         if ((e = hipEventSynchronize(x.c->stage_ev[slot])) != hipSuccess) break;
         xfer_copy(x, i, slot);
-        if (i + 2L * x.threads < nc) e = xfer_launch(x, i + 2L * x.threads, slot);
+        if (i + ahead < nc) e = xfer_launch(x, i + ahead, slot);
     }
     return e;
 }
@@ -3271,32 +3271,30 @@ static int transfer(shx_case *c, const bool up, const int nf, double *const *dev
     x.total = (long)nf * gm.ntot;
     if (!c->stage_len) {
         const long state = 5 * gm.ntot;
-        c->stage_threads = (state < STAGE_MANY) ? 1 : STAGE_SLOTS / 2;
+        c->stage_threads = (state < STAGE_MANY) ? 1 : STAGE_SLOTS;
         if (state <= STAGE_MIN) c->stage_len = state;
         else if (state < STAGE_MANY) c->stage_len = std::max(gm.ntot, std::min(STAGE_MIN, (state + 2) / 3));
-        else c->stage_len = std::min(STAGE_MAX, (state + STAGE_SLOTS - 1) / STAGE_SLOTS);
+        else c->stage_len = std::min(STAGE_MAX, (state + 2 * STAGE_SLOTS - 1) / (2 * STAGE_SLOTS));
     }
     x.chunk = c->stage_len;
     const long nc = (x.total + x.chunk - 1) / x.chunk;
     x.threads = (int)std::min<long>(c->stage_threads, nc);
+    x.per = (c->stage_threads == 1) ? 2 : 1;
     // fields that come down into one array are written in order, on one thread
     for (int m = 1; !up && m < nf; m++)
         for (int q = 0; q < m; q++)
             if (std::less<double *>()(host[q], host[m] + gm.ntot) && std::less<double *>()(host[m], host[q] + gm.ntot)) x.threads = 1;
     // the slots that xfer_chunks goes through, one allocation each: a new case's are taken from what an
-    // earlier one gave back, where one of 16 MB was pinned anew (first upload of 176 x 128 x 136 5.2 -> 3.5
-    // ms, 97 x 85 x 106 3.6 -> 2.5)
-    for (int id = 0; id < x.threads; id++)
-        for (int q = 0; q < 2 && id + (long)q * x.threads < nc; q++) {
-            const int b = 2 * id + q;
-            if (!c->stage_h[b])
-                HIPCHK(hipHostMalloc((void **)&c->stage_h[b], sizeof(double) * (size_t)c->stage_len, hipHostMallocDefault));
-            if (c->stage_ev[b]) continue;
-            HIPCHK(hipEventCreateWithFlags(&c->stage_ev[b], hipEventDisableTiming));
-            HIPCHK(hipEventRecord(c->stage_ev[b], c->stream));
-        }
-    hipError_t err[STAGE_SLOTS / 2];
-    std::thread th[STAGE_SLOTS / 2];
+    // earlier one gave back, where one of 16 MB was pinned anew
+    for (int b = 0; b < x.threads * x.per && b < nc; b++) {
+        if (!c->stage_h[b])
+            HIPCHK(hipHostMalloc((void **)&c->stage_h[b], sizeof(double) * (size_t)c->stage_len, hipHostMallocDefault));
+        if (c->stage_ev[b]) continue;
+        HIPCHK(hipEventCreateWithFlags(&c->stage_ev[b], hipEventDisableTiming));
+        HIPCHK(hipEventRecord(c->stage_ev[b], c->stream));
+    }
+    hipError_t err[STAGE_SLOTS];
+    std::thread th[STAGE_SLOTS];
     for (int t = 1; t < x.threads; t++) {
         err[t] = hipErrorUnknown;
         try {
