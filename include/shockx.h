@@ -338,7 +338,8 @@ int shx_blocks_destroy(shx_blocks *g);
  * shx_batch_run calls (work on a case's stream is ordered after the batch).  A case belongs to at
  * most one batch; while it does, shx_calc_runge_kutta, shx_run and shx_simulate on it (which
  * would move its state to another buffer than the batch's captured step uses) and shx_destroy
- * return SHX_ERR_STATE.  Destroy the batch before its cases. */
+ * return SHX_ERR_STATE.  Destroy the batch before its cases.  shx_batch_set_tau also takes up what
+ * has changed in the cases since (pressure kept for post-processing, source, tiles, metric). */
 typedef struct shx_batch shx_batch;
 int shx_batch_create(shx_case *const *cases, int ncases, const double *tau, shx_batch **out);
 int shx_batch_set_tau(shx_batch *b, const double *tau);
