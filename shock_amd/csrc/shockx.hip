@@ -4985,12 +4985,12 @@ extern "C" int shx_batch_set_tau(shx_batch *b, const double *tau)
     for (size_t i = 0; i < b->cases.size(); i++)
         if (!(tau[i] > 0.0)) return set_err(SHX_ERR_ARG, "case %zu: tau must be positive", i);
     HIPCHK(hipStreamSynchronize(b->stream));
-    std::vector<BatchLaunch> seq = b->seq;
-    std::vector<char> host = b->host;
-    std::vector<double> old_tau = b->tau;
+    std::vector<BatchLaunch> seq;
+    std::vector<char> host;
+    std::vector<double> old_tau(tau, tau + b->cases.size());
+    seq.swap(b->seq); host.swap(b->host); old_tau.swap(b->tau);
     char *const dev = b->dev;
     const int ngroups = b->ngroups;
-    b->tau.assign(tau, tau + b->cases.size());
     int rc = batch_build(b);
     if (!rc && same_layout(seq, b->seq) && host.size() == b->host.size()) {
         for (size_t i = 0; i < b->seq.size(); i++) { b->seq[i].grid = seq[i].grid; b->seq[i].run = seq[i].run; }
